@@ -15,9 +15,9 @@ namespace lfrv {
 // launchers (k_cnn.hip)
 hipError_t cnn_conv_fwd(const uint16_t *X, const uint16_t *Wt, const float *bias, const uint16_t *skip, void *Y,
                         int B, int H, int W, int Cin, int Cout, int epi, hipStream_t s);
-hipError_t cnn_conv_wgrad(const uint16_t *dU, const uint16_t *X, float *dW, int B, int H, int W, int Cin, int Cout,
-                          hipStream_t s);
-hipError_t cnn_bias_grad(const uint16_t *dU, float *db, int P, int C, hipStream_t s);
+size_t cnn_wgrad_ws_floats(int B, int H, int W, int Cin, int Cout);
+hipError_t cnn_conv_wgrad(const uint16_t *dU, const uint16_t *X, float *dW, float *db, float *ws, int B, int H, int W,
+                          int Cin, int Cout, hipStream_t s);
 hipError_t cnn_relu_bwd(const float *dY, const uint16_t *y, uint16_t *dU, float *dskip, size_t n, int relu,
                         hipStream_t s);
 hipError_t cnn_pool2(const uint16_t *x, uint16_t *y, int B, int H, int W, int C, hipStream_t s);
@@ -75,6 +75,8 @@ struct lfrv_cnn {
     float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;  // FP32 master, Adam moments, gradient
     uint16_t *wb = nullptr, *wf = nullptr;  // bf16 weights and the flipped copies of the input-gradient convs
     uint16_t *dU = nullptr;                 // bf16 masked output gradient of the conv being differentiated
+    float *gws = nullptr;                   // partial sums of a layer's weight gradient (grown on demand)
+    size_t gws_floats = 0;
     float *base = nullptr, *target = nullptr, *pred = nullptr;
     double *partials = nullptr, *partials_host = nullptr;
     int B = 0, H = 0, W = 0;
@@ -305,7 +307,18 @@ lfrv_status backward(lfrv_cnn *c)
         const Tensor &t = c->T[i];
         CNN_HIP(c, cnn_fill(t.grad, level_pixels(c, t.level, B, H, W) * t.c, 0.0f, s));
     }
-    CNN_HIP(c, cnn_fill(c->g, c->nparams, 0.0f, s));
+    size_t ws = 0;
+    for (const Op &o : c->ops)
+        if (o.kind == OP_CONV)
+            ws = std::max(ws, cnn_wgrad_ws_floats(B, H >> c->T[o.in].level, W >> c->T[o.in].level, o.cin, o.cout));
+    if (ws > c->gws_floats) {
+        CNN_HIP(c, hipStreamSynchronize(s));
+        (void)hipFree(c->gws);
+        c->gws = nullptr;
+        c->gws_floats = 0;
+        CNN_HIP(c, hipMalloc((void **)&c->gws, ws * 4));
+        c->gws_floats = ws;
+    }
     for (const Op &o : c->ops)
         if (o.kind == OP_CONV && o.in != 0) CNN_HIP(c, cnn_flip_weights(c->wb + o.woff, c->wf + o.woff, o.cin, o.cout, s));
     for (auto it = c->ops.rbegin(); it != c->ops.rend(); ++it) {
@@ -325,9 +338,9 @@ lfrv_status backward(lfrv_cnn *c)
                                 o.skip >= 0 ? c->T[o.skip].grad : nullptr, n, o.relu ? 1 : 0, s));
         hipEvent_t a;
         ev_begin(c, &a);
-        CNN_HIP(c, cnn_conv_wgrad(c->dU, (const uint16_t *)ti.data, c->g + o.woff, B, h, w, o.cin, o.cout, s));
+        CNN_HIP(c, cnn_conv_wgrad(c->dU, (const uint16_t *)ti.data, c->g + o.woff, c->g + o.boff, c->gws, B, h, w, o.cin,
+                                  o.cout, s));
         ev_end(c, a, conv_flops(c, o));
-        CNN_HIP(c, cnn_bias_grad(c->dU, c->g + o.boff, B * h * w, o.cout, s));
         if (o.in != 0) {
             ev_begin(c, &a);
             CNN_HIP(c, cnn_conv_fwd(c->dU, c->wf + o.woff, nullptr, nullptr, ti.grad, B, h, w, o.cout, o.cin,
@@ -405,7 +418,7 @@ extern "C" void lfrv_cnn_destroy(lfrv_cnn *c)
         if (t.grad) (void)hipFree(t.grad);
     }
     for (void *q : {(void *)c->w, (void *)c->m, (void *)c->v, (void *)c->g, (void *)c->wb, (void *)c->wf,
-                    (void *)c->dU, (void *)c->base, (void *)c->target, (void *)c->pred, (void *)c->partials})
+                    (void *)c->dU, (void *)c->gws, (void *)c->base, (void *)c->target, (void *)c->pred, (void *)c->partials})
         if (q) (void)hipFree(q);
     if (c->partials_host) (void)hipHostFree(c->partials_host);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -580,8 +593,8 @@ extern "C" lfrv_status lfrv_op_conv3x3_wgrad(int B, int H, int W, int Cin, int C
                                              float *dW, void *stream)
 {
     if (B < 1 || H < 1 || W < 1 || Cin < 32 || Cin % 32 || Cout < 8 || Cout % 8 || !dU || !X || !dW) return LFRV_E_ARG;
-    const hipError_t e = cnn_conv_wgrad((const uint16_t *)dU, (const uint16_t *)X, dW, B, H, W, Cin, Cout,
-                                        (hipStream_t)stream);
+    const hipError_t e = cnn_conv_wgrad((const uint16_t *)dU, (const uint16_t *)X, dW, nullptr, nullptr, B, H, W, Cin,
+                                        Cout, (hipStream_t)stream);
     return e == hipSuccess ? LFRV_OK : LFRV_E_HIP;
 }
 

@@ -19,7 +19,7 @@
 // v_mfma_f32_16x16x32_bf16 on 16-pixel x 16-channel tiles.  The backward
 // pass with respect to the input is the
 // same kernel on the output gradient with the weights flipped in space and
-// transposed in channels; the weight gradient is a second MFMA kernel whose
+// transposed in channels; the weight gradient is another MFMA kernel whose
 // K runs over pixels.
 #include "lfrv_internal.hpp"
 #include "tile_common.hpp"
@@ -296,92 +296,191 @@ k_conv3x3_halo(const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wt, 
     }
 }
 
-// Weight gradient, split over pixel chunks:
-//   dW[co][t][ci] += sum_{p in chunk} dU[p][co] X[p + off(t)][ci].
-// GEMM with M = co (64 per block), N = ci of one tap (32 per block), K =
-// pixels (32 per LDS stage, kWgChunk per block).  Both tiles are stored
-// transposed in LDS ([co][p], [ci][p]) so an MFMA fragment's 4 consecutive K
-// values are contiguous.  Each wave owns 16 rows of co and both 16-column
-// tiles of ci; the block adds its 64 x 32 partial to dW with FP32 atomics.
-constexpr int kWgChunk = 512;
-constexpr int kWgPitch = 36;  // bf16 per LDS row of 32 pixels (+4: rows spread over the banks)
+// Weight and bias gradient, split over pixels:
+//   dW[co][t][ci] += sum_p dU[p][co] X[p + off(t)][ci],  db[co] += sum_p dU[p][co].
+// GEMM with M = co, N = (tap, ci), K = pixels.  A block owns BCO x BCI output
+// and input channels and all 9 taps, so one staging of dU and of X with its
+// halo serves 9 BCO BCI products per pixel.  The pixels go in 8 x 8 cells; a
+// stage is four cells, one for each 16-lane group of an MFMA operand (its 8 K
+// values are 8 pixels of a row), so images of any width fill the K of 32.
+// Both operands lie in LDS as they lie in memory, channels contiguous, and are
+// transposed by ds_read_b64_tr_b16 on the way to the registers.  A row of X
+// is read once per column offset and multiplied with the three rows of dU it
+// meets (3 NCO MFMAs per operand), which keeps the MFMAs ahead of the LDS
+// reads.  The bias gradient is one more product, with ones.
+// LDS: the pixel pitch is an odd multiple of 32 bytes and the cells are half
+// the banks apart, so the 4 x 16 channel blocks of two lane groups never meet
+// in a bank.  The next stage's loads are in flight while this one is
+// multiplied.
+// Splitting K over at most kWgBlocks blocks in all (two per CU; 512 against
+// the 36 k blocks of one tap, 64 x 32 channels and 512 pixels each that this
+// replaced) keeps the partial sums few.  With ws they go there, [split][co][9]
+// [ci] and then [split][co], for k_wgrad_reduce; without, they are added to
+// dW by atomics.
+// 8 scenes of 256 x 256: the 15 layers together 536 us and 114 us for the sums
+// of the splits, against 2400 us and 960 us for the bias sums in a kernel of
+// their own (36,864 atomic partial sums of 64 x 32 per layer at most).
+constexpr int kWgBlocks = 512;
+constexpr int kWgCell = 8, kWgHalo = kWgCell + 2, kWgMaxBCI = 64;
 
-__global__ void __launch_bounds__(256)
-k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X, float *__restrict__ dW, int B,
-                int H, int W, int Cin, int Cout)
+template <int NCO, int WCO, int WCI>
+struct WgDims {
+    static constexpr int BCO = 16 * NCO * WCO, BCI = 16 * WCI;
+    static constexpr int pitch(int c) { return (2 * c / 32) % 2 ? 2 * c : 2 * c + 32; }  // bytes per pixel
+    // bytes per cell, half the banks (128 of 256 bytes) past a multiple of all of them
+    static constexpr int cell(int px, int c) { return px * pitch(c) + (384 - px * pitch(c) % 256) % 256; }
+    static constexpr int PD = pitch(BCO), PX = pitch(BCI);
+    static constexpr int SD = cell(kWgCell * kWgCell, BCO), SX = cell(kWgHalo * kWgHalo, BCI);
+    static constexpr int GD = BCO / 8, GX = BCI / 8;  // 16-byte groups per pixel
+    static constexpr int ND = (4 * kWgCell * kWgCell * GD + 255) / 256, NX = (4 * kWgHalo * kWgHalo * GX + 255) / 256;
+};
+
+__device__ __forceinline__ bf8v lds_transpose8(const char *p, int pitch)
 {
-    __shared__ __align__(16) uint16_t Ds[64 * kWgPitch];
-    __shared__ __align__(16) uint16_t Xs[32 * kWgPitch];
-    const int HW = H * W, P = B * HW;
-    const int pc0 = blockIdx.x * kWgChunk;
-    const int co0 = blockIdx.y * 64;
-    const int t = blockIdx.z / (Cin / 32), ci0 = (blockIdx.z % (Cin / 32)) * 32;
-    const int dy = t / 3 - 1, dx = t % 3 - 1;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    f4v acc[2] = {f4v{0.f, 0.f, 0.f, 0.f}, f4v{0.f, 0.f, 0.f, 0.f}};
-    // staging: dU tile 32 pixels x 64 co = 256 x 8 bf16 (one 16-byte load per
-    // thread); X tile 32 pixels x 32 ci = 128 x 8 bf16 (threads 0..127)
-    const int dp = tid >> 3, dc = (tid & 7) * 8;
-    const int xp = (tid & 127) >> 2, xc = (tid & 3) * 8;
-    const uint4 zero = make_uint4(0, 0, 0, 0);
-    const int pend = min(pc0 + kWgChunk, P);
-    for (int pb = pc0; pb < pend; pb += 32) {
-        uint4 dv = zero, xv = zero;
-        {
-            const int p = pb + dp;
-            if (p < pend && co0 + dc < Cout) dv = *(const uint4 *)(dU + (size_t)p * Cout + co0 + dc);
-        }
-        if (tid < 128) {
-            const int p = pb + xp;
-            if (p < pend) {
-                const int b = p / HW, r = p - b * HW, y = r / W + dy, x = r % W + dx;
-                if (y >= 0 && y < H && x >= 0 && x < W)
-                    xv = *(const uint4 *)(X + ((size_t)(b * H + y) * W + x) * Cin + ci0 + xc);
-            }
-        }
-        __syncthreads();
-        {
-            const uint16_t *d = (const uint16_t *)&dv;
-#pragma unroll
-            for (int k = 0; k < 8; k++) Ds[(dc + k) * kWgPitch + dp] = d[k];
-        }
-        if (tid < 128) {
-            const uint16_t *d = (const uint16_t *)&xv;
-#pragma unroll
-            for (int k = 0; k < 8; k++) Xs[(xc + k) * kWgPitch + xp] = d[k];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 32; kk += 16) {
-            const s4v a = *(const s4v *)(Ds + (wv * 16 + (lane & 15)) * kWgPitch + kk + 4 * (lane >> 4));
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const s4v b = *(const s4v *)(Xs + (j * 16 + (lane & 15)) * kWgPitch + kk + 4 * (lane >> 4));
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int ci = ci0 + j * 16 + (lane & 15);
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int co = co0 + wv * 16 + 4 * (lane >> 4) + r;
-            if (co < Cout) atomicAdd(dW + ((size_t)co * 9 + t) * Cin + ci, acc[j][r]);
-        }
-    }
+    typedef __attribute__((address_space(3))) s4v *lds_ptr;
+    const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p);
+    const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 4 * pitch));
+    typedef short s8v __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(bf8v, (s8v)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// db[c] += sum_p dU[p][c] over a chunk of pixels per block (C <= 256).
-__global__ void __launch_bounds__(256)
-k_bias_grad(const uint16_t *__restrict__ dU, float *__restrict__ db, int P, int C)
+// grid (splits, co blocks, ci blocks); split k takes stages k, k + splits, ...
+template <int NCO, int WCO, int WCI>
+__global__ void __launch_bounds__(256, 2)
+k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X, float *__restrict__ dW,
+                float *__restrict__ db, float *__restrict__ ws, int B, int H, int W, int Cin, int Cout)
 {
-    const int c = threadIdx.x;
-    if (c >= C) return;
-    const int p0 = blockIdx.x * 256, p1 = min(p0 + 256, P);
+    using D = WgDims<NCO, WCO, WCI>;
+    static_assert(WCO * WCI == 4, "four waves");
+    constexpr int R = kWgCell, HX = kWgHalo;
+    __shared__ __align__(16) char ds[4 * D::SD];
+    __shared__ __align__(16) char xs[4 * D::SX];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wco = wv / WCI, wci = wv % WCI;
+    const int co0 = blockIdx.y * D::BCO, ci0 = blockIdx.z * D::BCI;
+    const int ncx = (W + R - 1) / R, ncy = (H + R - 1) / R, ncells = B * ncx * ncy;
+    const int nstages = (ncells + 3) / 4;
+    u32x4 dr[D::ND], xr[D::NX];
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    // (every load reads a valid address and is zeroed afterwards)
+    auto load = [&](int st) {
+#pragma unroll
+        for (int j = 0; j < D::ND; j++) {
+            const int idx = tid + 256 * j, q = idx % D::GD, px = idx / D::GD, c = px / (R * R);
+            const int cell = 4 * st + c, b = cell / (ncx * ncy), rem = cell - b * ncx * ncy;
+            const int cy = rem / ncx, cx = rem - cy * ncx;
+            const int y = cy * R + px / R % R, x = cx * R + px % R;
+            const bool in = c < 4 && cell < ncells && y < H && x < W && co0 + 8 * q < Cout;
+            const u32x4 v = *(const u32x4 *)(dU + (in ? ((size_t)(b * H + y) * W + x) * Cout + co0 + 8 * q : 0));
+            dr[j] = in ? v : z;
+        }
+#pragma unroll
+        for (int j = 0; j < D::NX; j++) {
+            const int idx = tid + 256 * j, q = idx % D::GX, px = idx / D::GX, c = px / (HX * HX);
+            const int cell = 4 * st + c, b = cell / (ncx * ncy), rem = cell - b * ncx * ncy;
+            const int cy = rem / ncx, cx = rem - cy * ncx, hp = px - c * HX * HX;
+            const int y = cy * R - 1 + hp / HX, x = cx * R - 1 + hp % HX;
+            const bool in = c < 4 && cell < ncells && y >= 0 && y < H && x >= 0 && x < W && ci0 + 8 * q < Cin;
+            const u32x4 v = *(const u32x4 *)(X + (in ? ((size_t)(b * H + y) * W + x) * Cin + ci0 + 8 * q : 0));
+            xr[j] = in ? v : z;
+        }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int j = 0; j < D::ND; j++) {
+            const int idx = tid + 256 * j, q = idx % D::GD, px = idx / D::GD, c = px / (R * R);
+            if (c < 4) *(u32x4 *)(ds + c * D::SD + (px - c * R * R) * D::PD + 16 * q) = dr[j];
+        }
+#pragma unroll
+        for (int j = 0; j < D::NX; j++) {
+            const int idx = tid + 256 * j, q = idx % D::GX, px = idx / D::GX, c = px / (HX * HX);
+            if (c < 4) *(u32x4 *)(xs + c * D::SX + (px - c * HX * HX) * D::PX + 16 * q) = xr[j];
+        }
+    };
+    f4v acc[9][NCO], accb[NCO];
+#pragma unroll
+    for (int i = 0; i < NCO; i++) {
+        accb[i] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 9; t++) acc[t][i] = f4v{0.f, 0.f, 0.f, 0.f};
+    }
+    bf8v ones;
+#pragma unroll
+    for (int k = 0; k < 8; k++) ones[k] = (__bf16)1.0f;
+    const bool bias = db && blockIdx.z == 0 && wci == 0;
+    // this lane's share of an operand block: 4 channels of pixel (lane % 16) / 4 of its group's cell
+    const int grp = lane >> 4, lp = (lane & 15) >> 2, lc = 4 * (lane & 3);
+    const char *dsl = ds + grp * D::SD + lp * D::PD + 2 * (wco * 16 * NCO + lc);
+    const char *xsl = xs + grp * D::SX + lp * D::PX + 2 * (wci * 16 + lc);
+    load(blockIdx.x);
+    for (int st = blockIdx.x; st < nstages; st += gridDim.x) {
+        __syncthreads();  // the former stage is multiplied out
+        store();
+        __syncthreads();
+        if (st + (int)gridDim.x < nstages) load(st + gridDim.x);
+        bf8v a[3][NCO];
+#pragma unroll
+        for (int hr = 0; hr < HX; hr++) {
+            if (hr < R)
+#pragma unroll
+                for (int i = 0; i < NCO; i++) {
+                    a[hr % 3][i] = lds_transpose8(dsl + hr * R * D::PD + 32 * i, D::PD);
+                    if (bias) accb[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[hr % 3][i], ones, accb[i], 0, 0, 0);
+                }
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++) {
+                const bf8v b = lds_transpose8(xsl + (hr * HX + dx) * D::PX, D::PX);
+#pragma unroll
+                for (int dy = 0; dy < 3; dy++) {
+                    const int r = hr - dy;  // the row of dU that tap (dy, dx) pairs with this row of X
+                    if (r < 0 || r >= R) continue;
+#pragma unroll
+                    for (int i = 0; i < NCO; i++)
+                        acc[3 * dy + dx][i] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r % 3][i], b, acc[3 * dy + dx][i], 0, 0, 0);
+                }
+            }
+        }
+    }
+    const size_t nw = (size_t)Cout * 9 * Cin;
+    float *wsp = ws ? ws + (size_t)blockIdx.x * (nw + Cout) : nullptr;
+    const int ci = ci0 + wci * 16 + (lane & 15);
+#pragma unroll
+    for (int i = 0; i < NCO; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int co = co0 + (wco * NCO + i) * 16 + 4 * (lane >> 4) + r;
+            if (co >= Cout) continue;
+            if (ci < Cin)
+#pragma unroll
+                for (int t = 0; t < 9; t++) {
+                    const size_t o = ((size_t)co * 9 + t) * Cin + ci;
+                    if (wsp) wsp[o] = acc[t][i][r];
+                    else atomicAdd(dW + o, acc[t][i][r]);
+                }
+            if (bias && (lane & 15) == 0) {
+                if (wsp) wsp[nw + co] = accb[i][r];
+                else atomicAdd(db + co, accb[i][r]);
+            }
+        }
+}
+
+// g[i] = sum over the splits of ws[split][i], in split order by four
+// interleaved chains; the weights and biases of a layer are contiguous in g.
+__global__ void __launch_bounds__(256)
+k_wgrad_reduce(const float *__restrict__ ws, float *__restrict__ g, size_t n, int splits)
+{
+    __shared__ float part[4][64];
+    const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+    const size_t i = (size_t)blockIdx.x * 64 + x;
     float s = 0.0f;
-    for (int p = p0; p < p1; p++) s += bf2f(dU[(size_t)p * C + c]);
-    atomicAdd(db + c, s);
+    if (i < n) {
+        const float *p = ws + i;
+#pragma unroll 8
+        for (int k = y; k < splits; k += 4) s += p[(size_t)k * n];
+    }
+    part[y][x] = s;
+    __syncthreads();
+    if (y == 0 && i < n) g[i] = (part[0][x] + part[1][x]) + (part[2][x] + part[3][x]);
 }
 
 // dU = bf16(dY * [y > 0]) (y: the layer's ReLU output; relu = 0: no mask);
@@ -688,21 +787,40 @@ hipError_t cnn_conv_fwd(const uint16_t *X, const uint16_t *Wt, const float *bias
     return hipGetLastError();
 }
 
-hipError_t cnn_conv_wgrad(const uint16_t *dU, const uint16_t *X, float *dW, int B, int H, int W, int Cin, int Cout,
-                          hipStream_t s)
+// The splits of a layer's weight gradient: as many as fill kWgBlocks blocks with
+// its channel blocks (see k_conv3x3_wgrad), at most one per stage.
+static void wgrad_plan(int B, int H, int W, int Cin, int Cout, bool &tall, bool &wide, dim3 &grid)
 {
-    if (Cin % 32 != 0 || Cout % 8 != 0) return hipErrorInvalidValue;
-    const size_t P = (size_t)B * H * W;
-    const dim3 grid((unsigned int)((P + kWgChunk - 1) / kWgChunk), (unsigned int)((Cout + 63) / 64),
-                    (unsigned int)(9 * (Cin / 32)));
-    k_conv3x3_wgrad<<<grid, 256, 0, s>>>(dU, X, dW, B, H, W, Cin, Cout);
-    return hipGetLastError();
+    tall = Cout > 32;                      // 64 x 32 channels per block
+    wide = !tall && Cin % kWgMaxBCI == 0;  // 32 x 64; else 32 x 32
+    const int nco = (Cout + (tall ? 63 : 31)) / (tall ? 64 : 32), nci = Cin / (wide ? 64 : 32);
+    const int stages = (B * ((H + kWgCell - 1) / kWgCell) * ((W + kWgCell - 1) / kWgCell) + 3) / 4;
+    grid = dim3((unsigned int)std::max(1, std::min(stages, kWgBlocks / (nco * nci))), (unsigned int)nco,
+                (unsigned int)nci);
 }
 
-hipError_t cnn_bias_grad(const uint16_t *dU, float *db, int P, int C, hipStream_t s)
+size_t cnn_wgrad_ws_floats(int B, int H, int W, int Cin, int Cout)
 {
-    if (C > 256) return hipErrorInvalidValue;
-    k_bias_grad<<<(P + 255) / 256, 256, 0, s>>>(dU, db, P, C);
+    bool tall, wide;
+    dim3 grid;
+    wgrad_plan(B, H, W, Cin, Cout, tall, wide, grid);
+    return grid.x * ((size_t)Cout * 9 * Cin + Cout);
+}
+
+// dW (Cout x 9 x Cin) and, when it is not null, db; with ws (of cnn_wgrad_ws_floats)
+// they are set (db must follow dW), without ws they are added to.
+hipError_t cnn_conv_wgrad(const uint16_t *dU, const uint16_t *X, float *dW, float *db, float *ws, int B, int H, int W,
+                          int Cin, int Cout, hipStream_t s)
+{
+    const size_t nw = (size_t)Cout * 9 * Cin;
+    if (Cin % 32 != 0 || Cout % 8 != 0 || (ws && db != dW + nw)) return hipErrorInvalidValue;
+    bool tall, wide;
+    dim3 grid;
+    wgrad_plan(B, H, W, Cin, Cout, tall, wide, grid);
+    if (tall) k_conv3x3_wgrad<2, 2, 2><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout);
+    else if (wide) k_conv3x3_wgrad<2, 1, 4><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout);
+    else k_conv3x3_wgrad<1, 2, 2><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout);
+    if (ws) k_wgrad_reduce<<<(unsigned int)((nw + Cout + 63) / 64), 256, 0, s>>>(ws, dW, nw + Cout, (int)grid.x);
     return hipGetLastError();
 }
 

@@ -276,3 +276,28 @@ def test_trained_warm_start_saves_iterations_on_held_out_scenes():
         if r["used_net"]:
             assert r["energy_net_start"] < r["energy_plain_start"]
     assert warm.mean() < plain.mean()
+
+
+@pytest.mark.parametrize("B,H,W,Cin,Cout", [(1, 1, 1, 32, 32),    # one pixel
+                                            (3, 9, 7, 128, 32),   # cells cut on both sides, 64-input-channel blocks
+                                            (1, 8, 24, 96, 72),   # a stage's fourth cell missing, 8 last channels
+                                            (2, 33, 40, 64, 104)])
+def test_conv3x3_wgrad_tile_edges(B, H, W, Cin, Cout):
+    """The weight gradient at the edges of its cells, stages and channel blocks, added to what dW holds."""
+    print(f"conv3x3 wgrad B={B} {H}x{W} {Cin}->{Cout}", flush=True)
+    L, rng = cnn_lib(), np.random.default_rng([B, H, W, Cin, Cout])
+    X = to_bf16(rng.standard_normal((B, H, W, Cin)).astype(np.float32))
+    G = to_bf16(rng.standard_normal((B, H, W, Cout)).astype(np.float32))
+    dW0 = rng.standard_normal((Cout, 9, Cin)).astype(np.float32)
+    dX, dG, dWb = Raw(X), Raw(G), Raw(dW0)
+    assert L.lfrv_op_conv3x3_wgrad(B, H, W, Cin, Cout, dG.ptr, dX.ptr, dWb.ptr, None) == 0
+    lfrv.device_sync()
+    got = dWb.get(np.float32, (Cout, 9, Cin))
+    Xf, Gf = from_bf16(X).astype(np.float64), from_bf16(G).astype(np.float64)
+    Xp = np.pad(Xf, ((0, 0), (1, 1), (1, 1), (0, 0)))
+    want = dW0.astype(np.float64)
+    for t in range(9):
+        Xs = Xp[:, t // 3:t // 3 + H, t % 3:t % 3 + W, :]
+        want[:, t, :] += Gf.reshape(-1, Cout).T @ Xs.reshape(-1, Cin)
+    # FP32 sums of up to B H W products: eps sqrt(n) of their scale sqrt(n), well under 2e-5 of the largest entry
+    assert np.max(np.abs(got - want)) <= 2e-5 * max(1.0, np.abs(want).max())
