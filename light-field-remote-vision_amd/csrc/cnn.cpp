@@ -13,23 +13,15 @@
 namespace lfrv {
 
 // launchers (k_cnn.hip)
-hipError_t cnn_conv_fwd(const uint16_t *X, const uint16_t *Wt, const float *bias, const uint16_t *skip, void *Y,
-                        int B, int H, int W, int Cin, int Cout, int epi, hipStream_t s);
+hipError_t cnn_conv(int epi, CnnConv a, hipStream_t s);
 size_t cnn_wgrad_ws_floats(int B, int H, int W, int Cin, int Cout);
 hipError_t cnn_conv_wgrad(const uint16_t *dU, const uint16_t *X, float *dW, float *db, float *ws, int B, int H, int W,
-                          int Cin, int Cout, hipStream_t s);
-hipError_t cnn_relu_bwd(const float *dY, const uint16_t *y, uint16_t *dU, float *dskip, size_t n, int relu,
-                        hipStream_t s);
-hipError_t cnn_pool2(const uint16_t *x, uint16_t *y, int B, int H, int W, int C, hipStream_t s);
-hipError_t cnn_pool2_bwd(const float *dy, float *dx, int B, int H, int W, int C, hipStream_t s);
-hipError_t cnn_up2(const uint16_t *x, uint16_t *y, int B, int H, int W, int C, hipStream_t s);
-hipError_t cnn_up2_bwd(const float *dy, float *dx, int B, int H, int W, int C, hipStream_t s);
+                          int Cin, int Cout, int up, hipStream_t s);
 hipError_t cnn_fill(float *a, size_t n, float v, hipStream_t s);
 hipError_t cnn_to_bf16(const float *a, uint16_t *b, size_t n, hipStream_t s);
-hipError_t cnn_flip_weights(const uint16_t *Wt, uint16_t *Wf, int Cin, int Cout, hipStream_t s);
-hipError_t cnn_sq_loss(const float *out, const float *base, const float *target, float *dout, double *partials,
-                       int nblocks, int B, int HW, int co, float scale, hipStream_t s);
-hipError_t cnn_add_prediction(const float *out, const float *base, float *pred, int B, int HW, int co, hipStream_t s);
+hipError_t cnn_flip_weights(const uint16_t *wb, uint16_t *wf, const CnnLayers &l, hipStream_t s);
+hipError_t cnn_sq_loss(const float *pred, const float *target, uint16_t *dU, double *partials, int nblocks, int B,
+                       int HW, int co, float scale, hipStream_t s);
 hipError_t cnn_adam(float *w, float *m, float *v, const float *g, uint16_t *wb, size_t n, float lr, float b1,
                     float b2, float eps, int step, hipStream_t s);
 int cnn_stack_group();
@@ -38,16 +30,19 @@ hipError_t cnn_stack_group_pass(int dsf, int w, int h, int W, int H, const float
                                 const float *views, int v0, int nv, float *anchors, uint16_t *out, int cpad,
                                 int zero_from, hipStream_t s);
 
-constexpr int kEpiRelu = 1, kEpiSkip = 2, kEpiF32 = 4, kEpiAccum = 8, kEpiBias = 16;
 constexpr int kHeadCout = 32;     // the head's 3 channels, computed as 32
 constexpr int kLossBlocks = 256;  // partial sums of the loss
 
-// One tensor of the network: NHWC, [B][h][w][c] at its level.
+// One tensor of the network: bf16 NHWC, [B][h][w][c] at its level.  The
+// upsampled ones and the head's output are never stored (the convolutions read
+// the former from their source, the head writes the prediction).
 struct Tensor {
     int level = 0, c = 0;
-    bool f32 = false;       // the head's output
-    void *data = nullptr;   // bf16 (uint16_t) or float
-    float *grad = nullptr;  // FP32 gradient (nullptr for the input)
+    int op = -1;               // the op that makes it
+    bool stored = true;
+    bool skipped = false;      // read by a later skip
+    uint16_t *data = nullptr;
+    float *grad = nullptr;     // the skip's FP32 share of its gradient (skipped tensors)
 };
 
 enum OpKind { OP_CONV, OP_POOL, OP_UP };
@@ -74,7 +69,8 @@ struct lfrv_cnn {
     size_t nparams = 0;
     float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;  // FP32 master, Adam moments, gradient
     uint16_t *wb = nullptr, *wf = nullptr;  // bf16 weights and the flipped copies of the input-gradient convs
-    uint16_t *dU = nullptr;                 // bf16 masked output gradient of the conv being differentiated
+    uint16_t *dU[2] = {nullptr, nullptr};   // bf16 masked output gradients of the conv being differentiated and the next
+    CnnLayers flipped{};                    // the convolutions whose input gradient is formed
     float *gws = nullptr;                   // partial sums of a layer's weight gradient (grown on demand)
     size_t gws_floats = 0;
     float *base = nullptr, *target = nullptr, *pred = nullptr;
@@ -128,16 +124,17 @@ void build_graph(lfrv_cnn *c)
 {
     const int L = c->p.levels;
     auto ch = [&](int l) { return std::min(c->p.base_channels << l, 256); };
-    auto tensor = [&](int level, int chn, bool f32 = false) {
+    auto tensor = [&](int level, int chn, bool stored = true) {
         Tensor t;
         t.level = level;
         t.c = chn;
-        t.f32 = f32;
+        t.op = (int)c->ops.size();
+        t.stored = stored;
         c->T.push_back(t);
         return (int)c->T.size() - 1;
     };
     size_t off = 0;
-    auto conv = [&](int in, int cout, bool relu, int skip, bool f32 = false) {
+    auto conv = [&](int in, int cout, bool relu, int skip, bool stored = true) {
         Op o;
         o.kind = OP_CONV;
         o.in = in;
@@ -145,11 +142,19 @@ void build_graph(lfrv_cnn *c)
         o.cout = cout;
         o.relu = relu;
         o.skip = skip;
-        o.out = tensor(c->T[in].level, cout, f32);
+        if (skip >= 0) c->T[skip].skipped = true;
+        o.out = tensor(c->T[in].level, cout, stored);
         o.woff = off;
         off += (size_t)cout * 9 * o.cin;
         o.boff = off;
         off += (size_t)cout;
+        if (in != 0) {
+            CnnLayers &f = c->flipped;
+            f.woff[f.n] = o.woff;
+            f.cin[f.n] = o.cin;
+            f.cout[f.n] = o.cout;
+            f.n++;
+        }
         c->ops.push_back(o);
         return o.out;
     };
@@ -157,11 +162,12 @@ void build_graph(lfrv_cnn *c)
         Op o;
         o.kind = k;
         o.in = in;
-        o.out = tensor(c->T[in].level + (k == OP_POOL ? 1 : -1), c->T[in].c);
+        o.out = tensor(c->T[in].level + (k == OP_POOL ? 1 : -1), c->T[in].c, k == OP_POOL);
         c->ops.push_back(o);
         return o.out;
     };
     int x = tensor(0, c->cpad);
+    c->T[x].op = -1;
     std::vector<int> enc(L);
     for (int l = 0; l < L; l++) {
         if (l > 0) x = simple(OP_POOL, x);
@@ -174,7 +180,7 @@ void build_graph(lfrv_cnn *c)
         x = conv(x, ch(l), true, enc[l]);
         x = conv(x, ch(l), true, -1);
     }
-    conv(x, kHeadCout, false, -1, true);
+    conv(x, kHeadCout, false, -1, false);
     c->nparams = off;
 }
 
@@ -184,15 +190,12 @@ lfrv_status alloc_buffers(lfrv_cnn *c)
     for (size_t i = 0; i < c->T.size(); i++) {
         Tensor &t = c->T[i];
         const size_t n = level_pixels(c, t.level, B, H, W) * t.c;
-        CNN_HIP(c, hipMalloc(&t.data, n * (t.f32 ? 4 : 2)));
-        if (i > 0) CNN_HIP(c, hipMalloc((void **)&t.grad, n * 4));
+        if (t.stored) CNN_HIP(c, hipMalloc((void **)&t.data, n * 2));
+        if (t.skipped) CNN_HIP(c, hipMalloc((void **)&t.grad, n * 4));
     }
-    size_t max_out = 0, max_w = 0;
+    size_t max_out = 0;
     for (const Op &o : c->ops)
-        if (o.kind == OP_CONV) {
-            max_out = std::max(max_out, level_pixels(c, c->T[o.out].level, B, H, W) * o.cout);
-            max_w = std::max(max_w, (size_t)o.cout * 9 * o.cin);
-        }
+        if (o.kind == OP_CONV) max_out = std::max(max_out, level_pixels(c, c->T[o.out].level, B, H, W) * o.cout);
     const size_t np = c->nparams;
     CNN_HIP(c, hipMalloc((void **)&c->w, np * 4));
     CNN_HIP(c, hipMalloc((void **)&c->m, np * 4));
@@ -200,14 +203,13 @@ lfrv_status alloc_buffers(lfrv_cnn *c)
     CNN_HIP(c, hipMalloc((void **)&c->g, np * 4));
     CNN_HIP(c, hipMalloc((void **)&c->wb, np * 2));
     CNN_HIP(c, hipMalloc((void **)&c->wf, np * 2));
-    CNN_HIP(c, hipMalloc((void **)&c->dU, max_out * 2));
+    for (uint16_t *&d : c->dU) CNN_HIP(c, hipMalloc((void **)&d, max_out * 2));
     const size_t nimg = (size_t)B * 3 * H * W;
     CNN_HIP(c, hipMalloc((void **)&c->base, nimg * 4));
     CNN_HIP(c, hipMalloc((void **)&c->target, nimg * 4));
     CNN_HIP(c, hipMalloc((void **)&c->pred, nimg * 4));
     CNN_HIP(c, hipMalloc((void **)&c->partials, kLossBlocks * sizeof(double)));
     CNN_HIP(c, hipHostMalloc((void **)&c->partials_host, kLossBlocks * sizeof(double), hipHostMallocDefault));
-    (void)max_w;
     return LFRV_OK;
 }
 
@@ -272,41 +274,59 @@ double conv_flops(const lfrv_cnn *c, const Op &o)
     return 2.0 * 9.0 * o.cin * o.cout * (double)level_pixels(c, c->T[o.out].level, c->B, c->H, c->W);
 }
 
+// The stored tensor a convolution reads, and whether it reads it upsampled.
+const Tensor &conv_input(const lfrv_cnn *c, const Op &o, int &up)
+{
+    const Tensor &t = c->T[o.in];
+    up = t.op >= 0 && c->ops[t.op].kind == OP_UP;
+    return up ? c->T[c->ops[t.op].in] : t;
+}
+
+// pred <- base + the network's output; pooling rides on the convolution that
+// makes its input, upsampling on the one that reads its output.
 lfrv_status forward(lfrv_cnn *c)
 {
     const hipStream_t s = c->stream;
-    const int B = c->B, H = c->H, W = c->W;
-    for (const Op &o : c->ops) {
-        const Tensor &ti = c->T[o.in], &to = c->T[o.out];
-        const int h = H >> ti.level, w = W >> ti.level;
-        if (o.kind == OP_POOL) {
-            CNN_HIP(c, cnn_pool2((const uint16_t *)ti.data, (uint16_t *)to.data, B, h, w, ti.c, s));
-        } else if (o.kind == OP_UP) {
-            CNN_HIP(c, cnn_up2((const uint16_t *)ti.data, (uint16_t *)to.data, B, h, w, ti.c, s));
+    for (size_t k = 0; k < c->ops.size(); k++) {
+        const Op &o = c->ops[k];
+        if (o.kind != OP_CONV) continue;
+        const Tensor &to = c->T[o.out];
+        CnnConv a{};
+        a.X = conv_input(c, o, a.up).data;
+        a.Wt = c->wb + o.woff;
+        a.bias = c->w + o.boff;
+        a.B = c->B;
+        a.H = c->H >> to.level;
+        a.W = c->W >> to.level;
+        a.Cin = o.cin;
+        a.Cout = o.cout;
+        const bool head = !to.stored;
+        if (head) {
+            a.base = c->base;
+            a.Y = c->pred;
         } else {
-            int epi = kEpiBias;
-            if (o.relu) epi |= kEpiRelu;
-            if (o.skip >= 0) epi |= kEpiSkip;
-            if (to.f32) epi |= kEpiF32;
-            hipEvent_t a;
-            ev_begin(c, &a);
-            CNN_HIP(c, cnn_conv_fwd((const uint16_t *)ti.data, c->wb + o.woff, c->w + o.boff,
-                                    o.skip >= 0 ? (const uint16_t *)c->T[o.skip].data : nullptr, to.data, B, h, w,
-                                    o.cin, o.cout, epi, s));
-            ev_end(c, a, conv_flops(c, o));
+            a.relu = o.relu;
+            a.aux = o.skip >= 0 ? c->T[o.skip].data : nullptr;
+            a.Y = to.data;
+            if (k + 1 < c->ops.size() && c->ops[k + 1].kind == OP_POOL) a.pool = c->T[c->ops[k + 1].out].data;
         }
+        hipEvent_t e;
+        ev_begin(c, &e);
+        CNN_HIP(c, cnn_conv(head ? CNN_HEAD : CNN_FWD, a, s));
+        ev_end(c, e, conv_flops(c, o));
     }
     return LFRV_OK;
 }
 
+// The gradient of the parameters from the head's (c->dU[0], left by the
+// loss).  A convolution's input gradient goes at once to the masked bf16
+// gradient of the convolution before it: through a pooling (with the share
+// that the skip left in the pooled tensor's grad) or an upsampling where one
+// lies between; a skip's share is left in its tensor's grad, in FP32.
 lfrv_status backward(lfrv_cnn *c)
 {
     const hipStream_t s = c->stream;
     const int B = c->B, H = c->H, W = c->W;
-    for (size_t i = 1; i + 1 < c->T.size(); i++) {
-        const Tensor &t = c->T[i];
-        CNN_HIP(c, cnn_fill(t.grad, level_pixels(c, t.level, B, H, W) * t.c, 0.0f, s));
-    }
     size_t ws = 0;
     for (const Op &o : c->ops)
         if (o.kind == OP_CONV)
@@ -319,45 +339,53 @@ lfrv_status backward(lfrv_cnn *c)
         CNN_HIP(c, hipMalloc((void **)&c->gws, ws * 4));
         c->gws_floats = ws;
     }
-    for (const Op &o : c->ops)
-        if (o.kind == OP_CONV && o.in != 0) CNN_HIP(c, cnn_flip_weights(c->wb + o.woff, c->wf + o.woff, o.cin, o.cout, s));
+    CNN_HIP(c, cnn_flip_weights(c->wb, c->wf, c->flipped, s));
+    int cur = 0;
     for (auto it = c->ops.rbegin(); it != c->ops.rend(); ++it) {
         const Op &o = *it;
-        const Tensor &ti = c->T[o.in], &to = c->T[o.out];
+        if (o.kind != OP_CONV) continue;
+        const Tensor &ti = c->T[o.in];
         const int h = H >> ti.level, w = W >> ti.level;
-        if (o.kind == OP_POOL) {
-            CNN_HIP(c, cnn_pool2_bwd(to.grad, ti.grad, B, h, w, ti.c, s));
-            continue;
+        int up;
+        const Tensor &src = conv_input(c, o, up);
+        hipEvent_t e;
+        ev_begin(c, &e);
+        CNN_HIP(c, cnn_conv_wgrad(c->dU[cur], src.data, c->g + o.woff, c->g + o.boff, c->gws, B, h, w, o.cin, o.cout, up, s));
+        ev_end(c, e, conv_flops(c, o));
+        if (o.in == 0) continue;
+        CnnConv a{};
+        a.X = c->dU[cur];
+        a.Wt = c->wf + o.woff;
+        a.B = B;
+        a.H = h;
+        a.W = w;
+        a.Cin = o.cout;
+        a.Cout = o.cin;
+        cur ^= 1;
+        a.Y = c->dU[cur];
+        const Op &before = c->ops[ti.op];
+        int epi = CNN_MASK;
+        if (before.kind == OP_CONV) {
+            a.aux = ti.data;
+            if (before.skip >= 0) a.dskip = c->T[before.skip].grad;
+        } else {
+            epi = before.kind == OP_UP ? CNN_MASK_UP : CNN_MASK_POOL;
+            a.aux = c->T[before.in].data;
+            if (epi == CNN_MASK_POOL) a.dskip = c->T[before.in].grad;
         }
-        if (o.kind == OP_UP) {
-            CNN_HIP(c, cnn_up2_bwd(to.grad, ti.grad, B, h, w, ti.c, s));
-            continue;
-        }
-        const size_t n = (size_t)B * h * w * o.cout;
-        CNN_HIP(c, cnn_relu_bwd(to.grad, to.f32 ? nullptr : (const uint16_t *)to.data, c->dU,
-                                o.skip >= 0 ? c->T[o.skip].grad : nullptr, n, o.relu ? 1 : 0, s));
-        hipEvent_t a;
-        ev_begin(c, &a);
-        CNN_HIP(c, cnn_conv_wgrad(c->dU, (const uint16_t *)ti.data, c->g + o.woff, c->g + o.boff, c->gws, B, h, w, o.cin,
-                                  o.cout, s));
-        ev_end(c, a, conv_flops(c, o));
-        if (o.in != 0) {
-            ev_begin(c, &a);
-            CNN_HIP(c, cnn_conv_fwd(c->dU, c->wf + o.woff, nullptr, nullptr, ti.grad, B, h, w, o.cout, o.cin,
-                                    kEpiF32 | kEpiAccum, s));
-            ev_end(c, a, conv_flops(c, o));
-        }
+        ev_begin(c, &e);
+        CNN_HIP(c, cnn_conv(epi, a, s));
+        ev_end(c, e, conv_flops(c, o));
     }
     return LFRV_OK;
 }
 
-lfrv_status loss(lfrv_cnn *c, bool with_grad, double *out)
+// The squared error of pred and its gradient with respect to the head's output.
+lfrv_status loss(lfrv_cnn *c, double *out)
 {
     const int HW = c->H * c->W;
-    const Tensor &head = c->T.back();
     const float scale = 2.0f / (float)((double)c->B * 3 * HW);
-    CNN_HIP(c, cnn_sq_loss((const float *)head.data, c->base, c->target, with_grad ? head.grad : nullptr, c->partials,
-                           kLossBlocks, c->B, HW, kHeadCout, scale, c->stream));
+    CNN_HIP(c, cnn_sq_loss(c->pred, c->target, c->dU[0], c->partials, kLossBlocks, c->B, HW, kHeadCout, scale, c->stream));
     CNN_HIP(c, hipMemcpyAsync(c->partials_host, c->partials, kLossBlocks * sizeof(double), hipMemcpyDeviceToHost,
                               c->stream));
     CNN_HIP(c, hipStreamSynchronize(c->stream));
@@ -418,7 +446,7 @@ extern "C" void lfrv_cnn_destroy(lfrv_cnn *c)
         if (t.grad) (void)hipFree(t.grad);
     }
     for (void *q : {(void *)c->w, (void *)c->m, (void *)c->v, (void *)c->g, (void *)c->wb, (void *)c->wf,
-                    (void *)c->dU, (void *)c->gws, (void *)c->base, (void *)c->target, (void *)c->pred, (void *)c->partials})
+                    (void *)c->dU[0], (void *)c->dU[1], (void *)c->gws, (void *)c->base, (void *)c->target, (void *)c->pred, (void *)c->partials})
         if (q) (void)hipFree(q);
     if (c->partials_host) (void)hipHostFree(c->partials_host);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -518,7 +546,6 @@ extern "C" lfrv_status lfrv_cnn_forward(lfrv_cnn *c, float *pred)
     lfrv_status st = forward(c);
     if (st != LFRV_OK) return st;
     const int HW = c->H * c->W;
-    CNN_HIP(c, cnn_add_prediction((const float *)c->T.back().data, c->base, c->pred, c->B, HW, kHeadCout, c->stream));
     if (pred) {
         CNN_HIP(c, hipMemcpyAsync(pred, c->pred, (size_t)c->B * 3 * HW * 4, hipMemcpyDefault, c->stream));
         CNN_HIP(c, hipStreamSynchronize(c->stream));
@@ -532,7 +559,7 @@ extern "C" lfrv_status lfrv_cnn_loss_grad(lfrv_cnn *c, double *lossv)
     if (!c) return LFRV_E_ARG;
     if (c->B == 0 || !c->have_target) return cfail(c, LFRV_E_STATE, "no batch with targets set");
     lfrv_status st = forward(c);
-    if (st == LFRV_OK) st = loss(c, true, lossv);
+    if (st == LFRV_OK) st = loss(c, lossv);
     if (st == LFRV_OK) st = backward(c);
     ev_flush(c);
     return st;
@@ -584,8 +611,17 @@ extern "C" lfrv_status lfrv_op_conv3x3(int B, int H, int W, int Cin, int Cout, c
                                        const float *bias, float *Y, void *stream)
 {
     if (B < 1 || H < 1 || W < 1 || Cin < 32 || Cin % 32 || Cout < 1 || !X || !Wt || !Y) return LFRV_E_ARG;
-    const hipError_t e = cnn_conv_fwd((const uint16_t *)X, (const uint16_t *)Wt, bias, nullptr, Y, B, H, W, Cin, Cout,
-                                      bias ? (kEpiF32 | kEpiBias) : kEpiF32, (hipStream_t)stream);
+    CnnConv a{};
+    a.X = (const uint16_t *)X;
+    a.Wt = (const uint16_t *)Wt;
+    a.bias = bias;
+    a.Y = Y;
+    a.B = B;
+    a.H = H;
+    a.W = W;
+    a.Cin = Cin;
+    a.Cout = Cout;
+    const hipError_t e = cnn_conv(CNN_F32, a, (hipStream_t)stream);
     return e == hipSuccess ? LFRV_OK : LFRV_E_HIP;
 }
 
@@ -594,7 +630,7 @@ extern "C" lfrv_status lfrv_op_conv3x3_wgrad(int B, int H, int W, int Cin, int C
 {
     if (B < 1 || H < 1 || W < 1 || Cin < 32 || Cin % 32 || Cout < 8 || Cout % 8 || !dU || !X || !dW) return LFRV_E_ARG;
     const hipError_t e = cnn_conv_wgrad((const uint16_t *)dU, (const uint16_t *)X, dW, nullptr, nullptr, B, H, W, Cin,
-                                        Cout, (hipStream_t)stream);
+                                        Cout, 0, (hipStream_t)stream);
     return e == hipSuccess ? LFRV_OK : LFRV_E_HIP;
 }
 

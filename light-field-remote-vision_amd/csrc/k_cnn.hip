@@ -11,18 +11,19 @@
 // 32 (the first layer's are zero-padded), so a K chunk of 32 never straddles
 // a tap.
 //
-// The convolution is an implicit GEMM: C[pixel][cout] = sum_k A[pixel][k]
-// W[cout][k] with A[p][(t, ci)] = X[p + offset(t)][ci] (0 outside the
-// image).  k_conv3x3 walks K by (tap, 32-channel chunk) over 128 pixels in
-// row order; k_conv3x3_halo (64 input channels and more) by 32-channel chunk
-// over a 2-D pixel tile whose halo serves all 9 taps.  Both run
-// v_mfma_f32_16x16x32_bf16 on 16-pixel x 16-channel tiles.  The backward
-// pass with respect to the input is the
-// same kernel on the output gradient with the weights flipped in space and
-// transposed in channels; the weight gradient is another MFMA kernel whose
-// K runs over pixels.
+// The convolution is an implicit GEMM: C[cout][pixel] = sum_k W[cout][k]
+// A[k][pixel] with A[(t, ci)][p] = X[p + offset(t)][ci] (0 outside the image),
+// by chunk of 32 input channels over a 2-D pixel tile whose halo serves all 9
+// taps (v_mfma_f32_16x16x32_bf16).  Skips, ReLU, pooling, upsampling and the
+// prediction ride on its loads and its epilogue.  The backward pass with
+// respect to the input is the same kernel on the output gradient with the
+// weights flipped in space and transposed in channels; the weight gradient is
+// another MFMA kernel whose K runs over pixels.
 #include "lfrv_internal.hpp"
 #include "tile_common.hpp"
+
+#include <algorithm>
+#include <climits>
 
 namespace lfrv {
 
@@ -39,260 +40,247 @@ __device__ __forceinline__ uint16_t f2bf(float f)
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-constexpr int kCvBM = 128, kCvBK = 32, kCvPitch = 40;  // LDS rows of 40 bf16 (80 B, 16-byte aligned)
+constexpr int kCvBK = 32, kCvPitch = 40;  // LDS rows of 40 bf16 (80 B, 16-byte aligned)
 
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-enum : int { kEpiRelu = 1, kEpiSkip = 2, kEpiF32 = 4, kEpiAccum = 8, kEpiBias = 16 };
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
-// Y[p][co] = act(sum_{t,ci} W[co][t][ci] X[p + off(t)][ci] + bias[co] + skip[p][co]).
-// EPI: kEpiRelu, kEpiSkip (bf16 skip), kEpiBias, and the output kind: bf16,
-// or FP32 (kEpiF32), optionally added to what Y holds (kEpiAccum).
-// A block owns 128 pixels x 32 WN output channels; its 4 waves are arranged
-// (4 / WN) x WN, each on (128 WN / 4) pixels x 32 channels, i.e. 2 WN x 2
-// tiles of v_mfma_f32_16x16x32_bf16 (gfx950).  Per K chunk of 32 (one tap,
-// 32 input channels) the next chunk's tiles are loaded into registers while
-// the current one is multiplied out of LDS, then stored into the other LDS
-// buffer: one barrier per chunk.  An MFMA operand's 8 K values per lane are
-// 8 consecutive input channels in both the pixel and the weight tile, so
-// any K order the instruction uses inside pairs them alike.
-template <int EPI, int WN>
-__global__ void __launch_bounds__(256)
-k_conv3x3(const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wt, const float *__restrict__ bias,
-          const uint16_t *__restrict__ skip, void *__restrict__ Y, int B, int H, int W, int Cin, int Cout)
+// What a convolution does with its sums (CnnConv, lfrv_internal.hpp).  The
+// fused forms leave no elementwise pass of the network outside the
+// convolutions: what each replaced read and wrote the activations (or their
+// FP32 gradients) once more.
+template <int EPI>
+__device__ __forceinline__ void conv_epilogue(const CnnConv &a, f4v (&v)[4], int img, int y, int x, int co)
 {
-    constexpr int BN = 32 * WN, WM = 4 / WN, FM = kCvBM / WM / 16;
-    __shared__ __align__(16) uint16_t As[2][kCvBM * kCvPitch];
-    __shared__ __align__(16) uint16_t Bs[2][BN * kCvPitch];
-    const int HW = H * W, P = B * HW;
-    const int p0 = blockIdx.x * kCvBM, co0 = blockIdx.y * BN;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wm = wv / WN, wn = wv % WN;
-    // staging: A rows sr and sr + 64 (8 channels each), B row sr (threads < 4 BN)
-    const int sr = tid >> 2, sc = (tid & 3) * 8;
-    int sb[2], sy[2], sx[2];
-    bool prow[2];
+    // v[i]: channels co .. co + 3 of pixel (y + i, x); y is a multiple of 4, x of this lane: lane & 1
+    const bool xin = x < a.W && co < a.Cout;
+    if constexpr (EPI == CNN_F32) {
+        float *Y = (float *)a.Y;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int sp = p0 + sr + 64 * h;
-        prow[h] = sp < P;
-        sb[h] = prow[h] ? sp / HW : 0;
-        const int rem = prow[h] ? sp - sb[h] * HW : 0;
-        sy[h] = rem / W;
-        sx[h] = rem - sy[h] * W;
-    }
-    const int sco = co0 + sr;
-    const bool bload = tid < 4 * BN && sco < Cout;
-    const int ncc = Cin / kCvBK, nk = 9 * ncc;
-    // loads always read a valid address (pixel 0 / row 0 when the tap falls
-    // outside) and zero the value afterwards: a select between the load and a
-    // zero constant would put the constant in scratch memory and make every
-    // load a flat load through it
-    u32x4 a0, a1, b0;
-    bool m0, m1;
-#define CV_LOAD(kc)                                                                                         \
-    do {                                                                                                    \
-        const int t_ = (kc) / ncc, ci0_ = ((kc) - t_ * ncc) * kCvBK;                                       \
-        const int dy_ = t_ / 3 - 1, dx_ = t_ % 3 - 1;                                                       \
-        const int y0_ = sy[0] + dy_, x0_ = sx[0] + dx_, y1_ = sy[1] + dy_, x1_ = sx[1] + dx_;               \
-        const bool v0_ = prow[0] && y0_ >= 0 && y0_ < H && x0_ >= 0 && x0_ < W;                             \
-        const bool v1_ = prow[1] && y1_ >= 0 && y1_ < H && x1_ >= 0 && x1_ < W;                             \
-        const size_t o0_ = v0_ ? ((size_t)(sb[0] * H + y0_) * W + x0_) * Cin : 0;                          \
-        const size_t o1_ = v1_ ? ((size_t)(sb[1] * H + y1_) * W + x1_) * Cin : 0;                          \
-        a0 = *(const u32x4 *)(X + o0_ + ci0_ + sc);                                                         \
-        a1 = *(const u32x4 *)(X + o1_ + ci0_ + sc);                                                         \
-        b0 = *(const u32x4 *)(Wt + (bload ? ((size_t)sco * 9 + t_) * Cin : 0) + ci0_ + sc);                 \
-        m0 = v0_;                                                                                           \
-        m1 = v1_;                                                                                           \
-    } while (0)
-#define CV_STORE(buf)                                                                                       \
-    do {                                                                                                    \
-        const u32x4 z_ = {0u, 0u, 0u, 0u};                                                                  \
-        *(u32x4 *)(&As[buf][sr * kCvPitch + sc]) = m0 ? a0 : z_;                                            \
-        *(u32x4 *)(&As[buf][(sr + 64) * kCvPitch + sc]) = m1 ? a1 : z_;                                     \
-        if (tid < 4 * BN) *(u32x4 *)(&Bs[buf][sr * kCvPitch + sc]) = bload ? b0 : z_;                       \
-    } while (0)
-    f4v acc[FM][2];
+        for (int i = 0; i < 4; i++) {
+            if (!xin || y + i >= a.H) continue;
+            const size_t o = ((size_t)(img * a.H + y + i) * a.W + x) * a.Cout + co;
+            if (a.vec) *(f4v *)(Y + o) = v[i];
+            else
+                for (int r = 0; r < 4; r++)
+                    if (co + r < a.Cout) Y[o + r] = v[i][r];
+        }
+    } else if constexpr (EPI == CNN_HEAD) {
+        const size_t HW = (size_t)a.H * a.W;
 #pragma unroll
-    for (int i = 0; i < FM; i++)
+        for (int i = 0; i < 4; i++) {
+            if (!xin || y + i >= a.H || co != 0) continue;
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f4v{0.f, 0.f, 0.f, 0.f};
-    CV_LOAD(0);
-    CV_STORE(0);
-    __syncthreads();
-    for (int kc = 0; kc < nk; kc++) {
-        const int buf = kc & 1;
-        if (kc + 1 < nk) CV_LOAD(kc + 1);
-        bf8v a[FM], b[2];
+            for (int r = 0; r < 3; r++) {
+                const size_t o = ((size_t)img * 3 + r) * HW + (size_t)(y + i) * a.W + x;
+                ((float *)a.Y)[o] = a.base[o] + v[i][r];
+            }
+        }
+    } else if constexpr (EPI == CNN_FWD) {
+        u16x4 h[4];
 #pragma unroll
-        for (int i = 0; i < FM; i++)
-            a[i] = *(const bf8v *)(&As[buf][(wm * (kCvBM / WM) + i * 16 + (lane & 15)) * kCvPitch + 8 * (lane >> 4)]);
+        for (int i = 0; i < 4; i++) {
+            const bool in = xin && y + i < a.H;
+            const size_t o = in ? ((size_t)(img * a.H + y + i) * a.W + x) * a.Cout + co : 0;
+            if (a.aux) {
+                const u16x4 sk = *(const u16x4 *)(a.aux + o);
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-            b[j] = *(const bf8v *)(&Bs[buf][(wn * 32 + j * 16 + (lane & 15)) * kCvPitch + 8 * (lane >> 4)]);
+                for (int r = 0; r < 4; r++) v[i][r] += bf2f(sk[r]);
+            }
 #pragma unroll
-        for (int i = 0; i < FM; i++)
+            for (int r = 0; r < 4; r++) h[i][r] = f2bf(a.relu ? fmaxf(v[i][r], 0.0f) : v[i][r]);
+            if (in) *(u16x4 *)((uint16_t *)a.Y + o) = h[i];
+        }
+        if (a.pool) {  // (H and W even: a pair of rows and of lanes is whole)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        if (kc + 1 < nk) CV_STORE(buf ^ 1);
-        __syncthreads();
-    }
-#undef CV_LOAD
-#undef CV_STORE
-    // lane holds rows 4 (lane / 16) + r, column lane % 16 of each 16 x 16 tile
+            for (int i = 0; i < 4; i += 2) {
+                u16x4 q;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int co = co0 + wn * 32 + j * 16 + (lane & 15);
-        if (co >= Cout) continue;
-        const float bco = (EPI & kEpiBias) ? bias[co] : 0.0f;
+                for (int r = 0; r < 4; r++) {
+                    const float t0 = bf2f(h[i][r]), t1 = bf2f(h[i + 1][r]);
+                    q[r] = f2bf(0.25f * ((t0 + __shfl_xor(t0, 1)) + (t1 + __shfl_xor(t1, 1))));
+                }
+                if (xin && y + i < a.H && !(x & 1))
+                    *(u16x4 *)(a.pool + ((size_t)(img * (a.H / 2) + (y + i) / 2) * (a.W / 2) + x / 2) * a.Cout + co) = q;
+            }
+        }
+    } else if constexpr (EPI == CNN_MASK) {
 #pragma unroll
-        for (int i = 0; i < FM; i++)
+        for (int i = 0; i < 4; i++) {
+            if (!xin || y + i >= a.H) continue;
+            const size_t o = ((size_t)(img * a.H + y + i) * a.W + x) * a.Cout + co;
+            const u16x4 act = *(const u16x4 *)(a.aux + o);
+            u16x4 h;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int p = p0 + wm * (kCvBM / WM) + i * 16 + 4 * (lane >> 4) + r;
-                if (p >= P) continue;
-                const size_t o = (size_t)p * Cout + co;
-                float v = acc[i][j][r] + bco;
-                if (EPI & kEpiSkip) v += bf2f(skip[o]);
-                if (EPI & kEpiRelu) v = fmaxf(v, 0.0f);
-                if (EPI & kEpiF32) {
-                    float *yf = (float *)Y;
-                    yf[o] = (EPI & kEpiAccum) ? yf[o] + v : v;
-                } else {
-                    ((uint16_t *)Y)[o] = f2bf(v);
-                }
+                if (!(bf2f(act[r]) > 0.0f)) v[i][r] = 0.0f;
+                h[r] = f2bf(v[i][r]);
             }
+            if (a.dskip) *(f4v *)(a.dskip + o) = v[i];
+            *(u16x4 *)((uint16_t *)a.Y + o) = h;
+        }
+    } else if constexpr (EPI == CNN_MASK_UP) {
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+            float t[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                t[r] = (v[i][r] + __shfl_xor(v[i][r], 1)) + (v[i + 1][r] + __shfl_xor(v[i + 1][r], 1));
+            if (!xin || y + i >= a.H || (x & 1)) continue;
+            const size_t o = ((size_t)(img * (a.H / 2) + (y + i) / 2) * (a.W / 2) + x / 2) * a.Cout + co;
+            const u16x4 act = *(const u16x4 *)(a.aux + o);
+            u16x4 h;
+#pragma unroll
+            for (int r = 0; r < 4; r++) h[r] = f2bf(bf2f(act[r]) > 0.0f ? t[r] : 0.0f);
+            *(u16x4 *)((uint16_t *)a.Y + o) = h;
+        }
+    } else {  // CNN_MASK_POOL
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (!xin || y + i >= a.H) continue;
+            const size_t o0 = ((size_t)(img * 2 * a.H + 2 * (y + i)) * 2 * a.W + 2 * x) * a.Cout + co;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const size_t o = o0 + ((size_t)(k >> 1) * 2 * a.W + (k & 1)) * a.Cout;
+                const u16x4 act = *(const u16x4 *)(a.aux + o);
+                const f4v ds = *(const f4v *)(a.dskip + o);
+                u16x4 h;
+#pragma unroll
+                for (int r = 0; r < 4; r++) h[r] = f2bf(bf2f(act[r]) > 0.0f ? ds[r] + 0.25f * v[i][r] : 0.0f);
+                *(u16x4 *)((uint16_t *)a.Y + o) = h;
+            }
+        }
     }
 }
 
-// The same convolution for layers with 64 or more input channels, staged by
-// chunk of 32 input channels instead of by (tap, chunk): a block owns a
-// TH x 16 pixel tile of one image and 32 WN output channels.  Per chunk the
-// (TH + 2) x 18 halo of the tile (32 channels per pixel) and the weights of
-// all 9 taps go to LDS once; the 9 taps then read the halo at their offsets,
-// so a pixel's input is fetched (TH + 2) 18 / (16 TH) times per chunk instead
-// of 9, and a wave runs 9 FM 2 MFMAs between barriers instead of FM 2.  The
-// next chunk's halo and weights are loaded into registers before the 9 taps
-// are multiplied out and stored after them (two barriers: the weights have
-// one LDS buffer, the halo two).  With a single chunk (32 input channels)
-// nothing is left to overlap, and k_conv3x3 is the faster form.
-template <int EPI, int WN, int TH>
-__global__ void __launch_bounds__(256)
-k_conv3x3_halo(const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wt, const float *__restrict__ bias,
-             const uint16_t *__restrict__ skip, void *__restrict__ Y, int B, int H, int W, int Cin, int Cout)
+// v[p][co] = sum_{t,ci} W[co][t][ci] X[p + off(t)][ci] + bias[co], then the epilogue EPI.
+// A block owns 16 x 16 pixels (a wave 4 rows of 16) and BN = 16 NJ output
+// channels.  Per chunk of 32 input channels the tile's 18 x 18 halo and the
+// weights of all 9 taps go to LDS once.  A wave reads each halo row once per
+// column offset and multiplies it with the (up to) three taps of that column,
+// whose weights it holds in registers: 18 + 9 NJ LDS reads for 36 NJ MFMAs
+// (reading per tap would be 36 + 9 NJ), so that NJ = 4 is bound by the matrix
+// units and not by LDS.  The weights are the MFMA's first operand, so a lane
+// ends with 4 consecutive channels of one pixel and stores them at once.  The
+// next chunk's (or tile's) loads are in flight while this one is multiplied; a
+// block runs through its tiles, and with 32 input channels keeps the weights.
+// With up, X is half the image's size and read as its 2x nearest upsampling.
+// One image of 1024 x 1024: the 15 layers 757 us (500 TFLOP/s) with what rides
+// on them, against 988 us and 382 us of pooling, upsampling and prediction
+// passes before; 8 of 256 x 256 forwards and backwards: the step 1.76 ms
+// against 2.92 (the masks, skips, fills and resamplings of the backward pass
+// took 0.75 ms).
+template <int EPI, int NJ>
+__global__ void __launch_bounds__(256, NJ == 4 ? 2 : 3) k_conv3x3(CnnConv a)
 {
-    constexpr int TW = 16, HX = TW + 2, HP = HX * (TH + 2);
-    constexpr int BN = 32 * WN, WM = 4 / WN, FM = TH / WM;
-    static_assert(TH % WM == 0, "tile rows split evenly over the waves");
+    constexpr int FM = 4, TH = 16, TW = 16, HX = TW + 2, HP = HX * (TH + 2), BN = 16 * NJ;
     constexpr int NA = (HP * 4 + 255) / 256, NB = (36 * BN + 255) / 256;
-    __shared__ __align__(16) uint16_t As[2][HP * kCvPitch];
+    __shared__ __align__(16) uint16_t As[HP * kCvPitch];
     __shared__ __align__(16) uint16_t Bs[9 * BN * kCvPitch];
-    const int ntx = (W + TW - 1) / TW, nty = (H + TH - 1) / TH;
-    const int img = blockIdx.x / (ntx * nty), trem = blockIdx.x - img * ntx * nty;
-    const int ty = trem / ntx, tx = trem - ty * ntx;
-    const int y0 = ty * TH, x0 = tx * TW, co0 = blockIdx.y * BN;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wm = wv / WN, wn = wv % WN;
+    const int H = a.H, W = a.W, Cin = a.Cin, Cout = a.Cout;
+    const int ntx = (W + TW - 1) / TW, nty = (H + TH - 1) / TH, ntiles = a.B * ntx * nty;
+    const int co0 = blockIdx.y * BN;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int ncc = Cin / kCvBK;
-    size_t aoff[NA];
-    int alds[NA];
-    bool am[NA];
-#pragma unroll
-    for (int j = 0; j < NA; j++) {
-        const int idx = tid + 256 * j, hp = idx >> 2, q = idx & 3;
-        const bool slot = idx < HP * 4;
-        const int hy = hp / HX, hx = hp - hy * HX, y = y0 - 1 + hy, x = x0 - 1 + hx;
-        am[j] = slot && y >= 0 && y < H && x >= 0 && x < W;
-        aoff[j] = am[j] ? ((size_t)(img * H + y) * W + x) * Cin + 8 * q : 0;
-        alds[j] = slot ? hp * kCvPitch + 8 * q : -1;
-    }
-    // weight slots: idx -> tap idx / (4 BN), channel row (idx / 4) % BN, 8-channel group idx % 4
-    size_t boff[NB];
-    int blds[NB];
-    bool bm[NB];
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-        const int idx = tid + 256 * j, t = idx / (4 * BN), r = (idx >> 2) - t * BN, q = idx & 3;
-        const bool slot = idx < 36 * BN;
-        bm[j] = slot && co0 + r < Cout;
-        boff[j] = bm[j] ? ((size_t)(co0 + r) * 9 + t) * Cin + 8 * q : 0;
-        blds[j] = slot ? (t * BN + r) * kCvPitch + 8 * q : -1;
-    }
-    const u32x4 z = {0u, 0u, 0u, 0u};
+    const int Hs = H >> a.up, Ws = W >> a.up;  // X's own size
+    // loads always read a valid address; what lies outside is zeroed on its way to LDS
     u32x4 ar[NA], br[NB];
-    auto load = [&](int cc) {
+    unsigned amask = 0;
+    auto load = [&](int tile, int cc) {
+        const int img = tile / (ntx * nty), trem = tile - img * ntx * nty, ty = trem / ntx, tx = trem - ty * ntx;
+        amask = 0;
 #pragma unroll
-        for (int j = 0; j < NA; j++) ar[j] = *(const u32x4 *)(X + aoff[j] + cc * kCvBK);
-#pragma unroll
-        for (int j = 0; j < NB; j++) br[j] = *(const u32x4 *)(Wt + boff[j] + cc * kCvBK);
+        for (int j = 0; j < NA; j++) {
+            const int idx = tid + 256 * j, hp = idx >> 2, hy = hp / HX, hx = hp - hy * HX;
+            const int y = ty * TH - 1 + hy, x = tx * TW - 1 + hx;
+            const bool in = hp < HP && y >= 0 && y < H && x >= 0 && x < W;
+            ar[j] = *(const u32x4 *)(a.X + (in ? ((size_t)(img * Hs + (y >> a.up)) * Ws + (x >> a.up)) * Cin : 0) +
+                                     cc * kCvBK + 8 * (idx & 3));
+            amask |= (in ? 1u : 0u) << j;
+        }
     };
-    auto store = [&](int abuf) {
+    auto load_weights = [&](int cc) {
 #pragma unroll
-        for (int j = 0; j < NA; j++)
-            if (alds[j] >= 0) *(u32x4 *)(&As[abuf][alds[j]]) = am[j] ? ar[j] : z;
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-            if (blds[j] >= 0) *(u32x4 *)(&Bs[blds[j]]) = bm[j] ? br[j] : z;
+        for (int j = 0; j < NB; j++) {
+            const int idx = tid + 256 * j, t = idx / (4 * BN), r = (idx >> 2) - t * BN;
+            const bool in = idx < 36 * BN && co0 + r < Cout;
+            const unsigned o = (in ? (unsigned)((co0 + r) * 9 + t) * Cin : 0u) + 8 * (idx & 3);  // (a layer's weights: far under 2^31)
+            br[j] = *(const u32x4 *)(a.Wt + cc * kCvBK + o);
+        }
     };
-    f4v acc[FM][2];
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    auto store = [&](bool weights) {
 #pragma unroll
-    for (int i = 0; i < FM; i++)
+        for (int j = 0; j < NA; j++) {
+            const int idx = tid + 256 * j;
+            if ((idx >> 2) < HP) *(u32x4 *)(&As[(idx >> 2) * kCvPitch + 8 * (idx & 3)]) = (amask >> j & 1) ? ar[j] : z;
+        }
+        if (weights)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f4v{0.f, 0.f, 0.f, 0.f};
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int cc = 0; cc < ncc; cc++) {
-        const int abuf = cc & 1;
-        if (cc + 1 < ncc) load(cc + 1);
-#pragma unroll 3
-        for (int t = 0; t < 9; t++) {
-            const int dy = t / 3, dx = t - 3 * dy;
-            bf8v a[FM], b[2];
+            for (int j = 0; j < NB; j++) {
+                const int idx = tid + 256 * j, row = idx >> 2;  // t BN + r
+                if (idx < 36 * BN)
+                    *(u32x4 *)(&Bs[row * kCvPitch + 8 * (idx & 3)]) = co0 + row % BN < Cout ? br[j] : z;
+            }
+    };
+    const uint16_t *al = As + (wv * FM * HX + (lane & 15)) * kCvPitch + 8 * (lane >> 4);
+    const uint16_t *bl = Bs + (lane & 15) * kCvPitch + 8 * (lane >> 4);
+    f4v bias[NJ];
 #pragma unroll
-            for (int i = 0; i < FM; i++) {
-                const int hp = (wm * FM + i + dy) * HX + (lane & 15) + dx;
-                a[i] = *(const bf8v *)(&As[abuf][hp * kCvPitch + 8 * (lane >> 4)]);
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int co = co0 + 16 * j + 4 * (lane >> 4) + r;
+            bias[j][r] = a.bias && co < Cout ? a.bias[co] : 0.0f;
+        }
+    bool weights = true;
+    load(blockIdx.x, 0);
+    load_weights(0);
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        f4v acc[NJ][FM];
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int i = 0; i < FM; i++) acc[j][i] = bias[j];
+        for (int cc = 0; cc < ncc; cc++) {
+            __syncthreads();  // the former chunk is multiplied out
+            store(weights);
+            __syncthreads();
+            const int nc = cc + 1 < ncc ? cc + 1 : 0, nt = nc ? tile : tile + (int)gridDim.x;
+            weights = ncc > 1;
+            if (nt < ntiles) {
+                load(nt, nc);
+                if (weights) load_weights(nc);
             }
 #pragma unroll
-            for (int j = 0; j < 2; j++)
-                b[j] = *(const bf8v *)(&Bs[(t * BN + wn * 32 + j * 16 + (lane & 15)) * kCvPitch + 8 * (lane >> 4)]);
+            for (int dx = 0; dx < 3; dx++) {
+                if (NJ > 1) __builtin_amdgcn_sched_barrier(0);  // one column's weights in registers at a time: no spills
+                bf8v w[3][NJ];
 #pragma unroll
-            for (int i = 0; i < FM; i++)
+                for (int dy = 0; dy < 3; dy++)
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (cc + 1 < ncc) {
-            __syncthreads();  // every wave is done with the weights of this chunk
-            store(abuf ^ 1);
-            __syncthreads();
-        }
-    }
+                    for (int j = 0; j < NJ; j++)
+                        w[dy][j] = *(const bf8v *)(bl + ((3 * dy + dx) * BN + 16 * j) * kCvPitch);
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int co = co0 + wn * 32 + j * 16 + (lane & 15);
-        if (co >= Cout) continue;
-        const float bco = (EPI & kEpiBias) ? bias[co] : 0.0f;
+                for (int hr = 0; hr < FM + 2; hr++) {
+                    const bf8v px = *(const bf8v *)(al + (hr * HX + dx) * kCvPitch);
 #pragma unroll
-        for (int i = 0; i < FM; i++) {
-            const int y = y0 + wm * FM + i;
+                    for (int dy = 0; dy < 3; dy++) {
+                        if (hr - dy < 0 || hr - dy >= FM) continue;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int x = x0 + 4 * (lane >> 4) + r;
-                if (y >= H || x >= W) continue;
-                const size_t o = ((size_t)(img * H + y) * W + x) * Cout + co;
-                float v = acc[i][j][r] + bco;
-                if (EPI & kEpiSkip) v += bf2f(skip[o]);
-                if (EPI & kEpiRelu) v = fmaxf(v, 0.0f);
-                if (EPI & kEpiF32) {
-                    float *yf = (float *)Y;
-                    yf[o] = (EPI & kEpiAccum) ? yf[o] + v : v;
-                } else {
-                    ((uint16_t *)Y)[o] = f2bf(v);
+                        for (int j = 0; j < NJ; j++)
+                            acc[j][hr - dy] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dy][j], px, acc[j][hr - dy], 0, 0, 0);
+                    }
                 }
             }
         }
+        const int img = tile / (ntx * nty), trem = tile - img * ntx * nty, ty = trem / ntx, tx = trem - ty * ntx;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            conv_epilogue<EPI>(a, acc[j], img, ty * TH + wv * FM, tx * TW + (lane & 15), co0 + 16 * j + 4 * (lane >> 4));
     }
 }
 
@@ -348,7 +336,7 @@ __device__ __forceinline__ bf8v lds_transpose8(const char *p, int pitch)
 template <int NCO, int WCO, int WCI>
 __global__ void __launch_bounds__(256, 2)
 k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X, float *__restrict__ dW,
-                float *__restrict__ db, float *__restrict__ ws, int B, int H, int W, int Cin, int Cout)
+                float *__restrict__ db, float *__restrict__ ws, int B, int H, int W, int Cin, int Cout, int up)
 {
     using D = WgDims<NCO, WCO, WCI>;
     static_assert(WCO * WCI == 4, "four waves");
@@ -359,10 +347,13 @@ k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X,
     const int co0 = blockIdx.y * D::BCO, ci0 = blockIdx.z * D::BCI;
     const int ncx = (W + R - 1) / R, ncy = (H + R - 1) / R, ncells = B * ncx * ncy;
     const int nstages = (ncells + 3) / 4;
+    const int Hs = H >> up, Ws = W >> up;  // X's own size (with up: half, read as its 2x nearest upsampling)
     u32x4 dr[D::ND], xr[D::NX];
+    unsigned dmask = 0, xmask = 0;
     const u32x4 z = {0u, 0u, 0u, 0u};
-    // (every load reads a valid address and is zeroed afterwards)
+    // (every load reads a valid address; what lies outside is zeroed on its way to LDS)
     auto load = [&](int st) {
+        dmask = xmask = 0;
 #pragma unroll
         for (int j = 0; j < D::ND; j++) {
             const int idx = tid + 256 * j, q = idx % D::GD, px = idx / D::GD, c = px / (R * R);
@@ -370,8 +361,8 @@ k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X,
             const int cy = rem / ncx, cx = rem - cy * ncx;
             const int y = cy * R + px / R % R, x = cx * R + px % R;
             const bool in = c < 4 && cell < ncells && y < H && x < W && co0 + 8 * q < Cout;
-            const u32x4 v = *(const u32x4 *)(dU + (in ? ((size_t)(b * H + y) * W + x) * Cout + co0 + 8 * q : 0));
-            dr[j] = in ? v : z;
+            dr[j] = *(const u32x4 *)(dU + (in ? ((size_t)(b * H + y) * W + x) * Cout + co0 + 8 * q : 0));
+            dmask |= (in ? 1u : 0u) << j;
         }
 #pragma unroll
         for (int j = 0; j < D::NX; j++) {
@@ -380,20 +371,20 @@ k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X,
             const int cy = rem / ncx, cx = rem - cy * ncx, hp = px - c * HX * HX;
             const int y = cy * R - 1 + hp / HX, x = cx * R - 1 + hp % HX;
             const bool in = c < 4 && cell < ncells && y >= 0 && y < H && x >= 0 && x < W && ci0 + 8 * q < Cin;
-            const u32x4 v = *(const u32x4 *)(X + (in ? ((size_t)(b * H + y) * W + x) * Cin + ci0 + 8 * q : 0));
-            xr[j] = in ? v : z;
+            xr[j] = *(const u32x4 *)(X + (in ? ((size_t)(b * Hs + (y >> up)) * Ws + (x >> up)) * Cin + ci0 + 8 * q : 0));
+            xmask |= (in ? 1u : 0u) << j;
         }
     };
     auto store = [&]() {
 #pragma unroll
         for (int j = 0; j < D::ND; j++) {
             const int idx = tid + 256 * j, q = idx % D::GD, px = idx / D::GD, c = px / (R * R);
-            if (c < 4) *(u32x4 *)(ds + c * D::SD + (px - c * R * R) * D::PD + 16 * q) = dr[j];
+            if (c < 4) *(u32x4 *)(ds + c * D::SD + (px - c * R * R) * D::PD + 16 * q) = (dmask >> j & 1) ? dr[j] : z;
         }
 #pragma unroll
         for (int j = 0; j < D::NX; j++) {
             const int idx = tid + 256 * j, q = idx % D::GX, px = idx / D::GX, c = px / (HX * HX);
-            if (c < 4) *(u32x4 *)(xs + c * D::SX + (px - c * HX * HX) * D::PX + 16 * q) = xr[j];
+            if (c < 4) *(u32x4 *)(xs + c * D::SX + (px - c * HX * HX) * D::PX + 16 * q) = (xmask >> j & 1) ? xr[j] : z;
         }
     };
     f4v acc[9][NCO], accb[NCO];
@@ -483,90 +474,6 @@ k_wgrad_reduce(const float *__restrict__ ws, float *__restrict__ g, size_t n, in
     if (y == 0 && i < n) g[i] = (part[0][x] + part[1][x]) + (part[2][x] + part[3][x]);
 }
 
-// dU = bf16(dY * [y > 0]) (y: the layer's ReLU output; relu = 0: no mask);
-// with dskip: dskip += the masked gradient (the skip input's share).
-__global__ void k_relu_bwd(const float *__restrict__ dY, const uint16_t *__restrict__ y, uint16_t *__restrict__ dU,
-                           float *__restrict__ dskip, size_t n, int relu)
-{
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float g = dY[i];
-        if (relu && !(bf2f(y[i]) > 0.0f)) g = 0.0f;
-        dU[i] = f2bf(g);
-        if (dskip) dskip[i] += g;
-    }
-}
-
-// 2x2 average pooling of NHWC bf16 (H, W even): out [B][H/2][W/2][C].
-__global__ void k_pool2(const uint16_t *__restrict__ x, uint16_t *__restrict__ y, int B, int H, int W, int C)
-{
-    const int Ho = H / 2, Wo = W / 2;
-    const size_t n = (size_t)B * Ho * Wo * C;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        size_t q = i / C;
-        const int xo = (int)(q % Wo);
-        q /= Wo;
-        const int yo = (int)(q % Ho);
-        const int b = (int)(q / Ho);
-        const size_t r0 = ((size_t)(b * H + 2 * yo) * W + 2 * xo) * C + c, r1 = r0 + (size_t)W * C;
-        y[i] = f2bf(0.25f * ((bf2f(x[r0]) + bf2f(x[r0 + C])) + (bf2f(x[r1]) + bf2f(x[r1 + C]))));
-    }
-}
-
-// Gradient of the pooling: dx[4 children] += dy / 4 (FP32).
-__global__ void k_pool2_bwd(const float *__restrict__ dy, float *__restrict__ dx, int B, int H, int W, int C)
-{
-    const int Ho = H / 2, Wo = W / 2;
-    const size_t n = (size_t)B * Ho * Wo * C;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        size_t q = i / C;
-        const int xo = (int)(q % Wo);
-        q /= Wo;
-        const int yo = (int)(q % Ho);
-        const int b = (int)(q / Ho);
-        const float g = 0.25f * dy[i];
-        const size_t r0 = ((size_t)(b * H + 2 * yo) * W + 2 * xo) * C + c, r1 = r0 + (size_t)W * C;
-        dx[r0] += g;
-        dx[r0 + C] += g;
-        dx[r1] += g;
-        dx[r1 + C] += g;
-    }
-}
-
-// Nearest 2x upsampling of NHWC bf16: out [B][2H][2W][C].
-__global__ void k_up2(const uint16_t *__restrict__ x, uint16_t *__restrict__ y, int B, int H, int W, int C)
-{
-    const int Ho = 2 * H, Wo = 2 * W;
-    const size_t n = (size_t)B * Ho * Wo * C;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        size_t q = i / C;
-        const int xo = (int)(q % Wo);
-        q /= Wo;
-        const int yo = (int)(q % Ho);
-        const int b = (int)(q / Ho);
-        y[i] = x[((size_t)(b * H + yo / 2) * W + xo / 2) * C + c];
-    }
-}
-
-// Gradient of the upsampling: dx += the sum of the 4 children of dy (FP32).
-__global__ void k_up2_bwd(const float *__restrict__ dy, float *__restrict__ dx, int B, int H, int W, int C)
-{
-    const size_t n = (size_t)B * H * W * C;
-    const int Wo = 2 * W;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        size_t q = i / C;
-        const int x = (int)(q % W);
-        q /= W;
-        const int y = (int)(q % H);
-        const int b = (int)(q / H);
-        const size_t r0 = ((size_t)(b * 2 * H + 2 * y) * Wo + 2 * x) * C + c, r1 = r0 + (size_t)Wo * C;
-        dx[i] += (dy[r0] + dy[r0 + C]) + (dy[r1] + dy[r1 + C]);
-    }
-}
-
 __global__ void k_fill_f32(float *__restrict__ a, size_t n, float v)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = v;
@@ -578,56 +485,53 @@ __global__ void k_f32_to_bf16(const float *__restrict__ a, uint16_t *__restrict_
         b[i] = f2bf(a[i]);
 }
 
-// Wf[ci][t][co] = W[co][8 - t][ci]: the weights of the input-gradient convolution.
-__global__ void k_flip_weights(const uint16_t *__restrict__ Wt, uint16_t *__restrict__ Wf, int Cin, int Cout)
+// Wf[ci][t][co] = W[co][8 - t][ci]: the weights of the input-gradient
+// convolutions, every layer of the list in one launch (grid.y).
+__global__ void k_flip_weights(const uint16_t *__restrict__ wb, uint16_t *__restrict__ wf, CnnLayers l)
 {
+    const int Cin = l.cin[blockIdx.y], Cout = l.cout[blockIdx.y];
+    const uint16_t *Wt = wb + l.woff[blockIdx.y];
+    uint16_t *Wf = wf + l.woff[blockIdx.y];
     const size_t n = (size_t)Cout * 9 * Cin;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int ci = (int)(i % Cin);
-        const size_t q = i / Cin;
+        const int co = (int)(i % Cout);
+        const size_t q = i / Cout;
         const int t = (int)(q % 9);
-        const int co = (int)(q / 9);
-        Wf[((size_t)ci * 9 + (8 - t)) * Cout + co] = Wt[i];
+        const int ci = (int)(q / 9);
+        Wf[i] = Wt[((size_t)co * 9 + (8 - t)) * Cin + ci];
     }
 }
 
-// Loss of the prediction base + out[., 0..2] against the target (planar FP32
-// [B][3][H][W] for base and target; out NHWC FP32 with `co` channels):
+// Loss of the prediction against the target (planar FP32 [B][3][H][W]):
 // per-block partial sums of the squared error (FP64) and the gradient
-// d loss / d out = 2 (pred - target) / count (0 on the padding channels).
+// d loss / d out = 2 (pred - target) / count as the bf16 the head's backward
+// pass reads, NHWC with co channels (0 on the padding channels; co a multiple
+// of 8).
 __global__ void __launch_bounds__(256)
-k_sq_loss(const float *__restrict__ out, const float *__restrict__ base, const float *__restrict__ target,
-          float *__restrict__ dout, double *__restrict__ partials, int B, int HW, int co, float scale)
+k_sq_loss(const float *__restrict__ pred, const float *__restrict__ target, uint16_t *__restrict__ dU,
+          double *__restrict__ partials, int B, int HW, int co, float scale)
 {
     double s = 0.0;
     const size_t n = (size_t)B * HW;
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (size_t)gridDim.x * blockDim.x) {
         const size_t b = p / HW, o = p - b * HW;
-        for (int c = 0; c < co; c++) {
-            float g = 0.0f;
-            if (c < 3) {
-                const size_t q = (b * 3 + c) * HW + o;
-                const float d = base[q] + out[p * co + c] - target[q];
-                s += (double)d * d;
-                g = scale * d;
-            }
-            if (dout) dout[p * co + c] = g;
+        uint32_t h[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const size_t q = (b * 3 + c) * HW + o;
+            const float d = pred[q] - target[q];
+            s += (double)d * d;
+            h[c] = f2bf(scale * d);
+        }
+        u32x4 v = {h[0] | h[1] << 16, h[2], 0u, 0u};
+        for (int c = 0; c < co; c += 8) {
+            *(u32x4 *)(dU + p * co + c) = v;
+            v = u32x4{0u, 0u, 0u, 0u};
         }
     }
     __shared__ double red[16];
     double v[1] = {s};
     block_partials<1>(v, partials, red);
-}
-
-// pred (planar FP32 [B][3][H][W]) = base + out[., 0..2].
-__global__ void k_add_prediction(const float *__restrict__ out, const float *__restrict__ base, float *__restrict__ pred,
-                                 int B, int HW, int co)
-{
-    const size_t n = (size_t)B * 3 * HW;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const size_t o = i % HW, bc = i / HW, b = bc / 3, c = bc % 3;
-        pred[i] = base[i] + out[(b * HW + o) * co + c];
-    }
 }
 
 // Adam on FP32 master weights (Kingma & Ba, bias-corrected), then the bf16
@@ -754,33 +658,35 @@ k_stack_box_pack(int W, int H, int WA, int HA, const float *__restrict__ anchors
 
 inline unsigned int ew_blocks(size_t n) { return (unsigned int)std::min<size_t>((n + 255) / 256, 16384); }
 
-hipError_t cnn_conv_fwd(const uint16_t *X, const uint16_t *Wt, const float *bias, const uint16_t *skip, void *Y,
-                        int B, int H, int W, int Cin, int Cout, int epi, hipStream_t s)
+// The output channels per block (64, 32 or 16): the widest that the layer's
+// channels fill and that leaves a block for each of the 256 CUs; narrower
+// blocks stage the halo more often.
+hipError_t cnn_conv(int epi, CnnConv a, hipStream_t s)
 {
-    if (Cin % kCvBK != 0) return hipErrorInvalidValue;
-    const unsigned int gm = (unsigned int)(((size_t)B * H * W + kCvBM - 1) / kCvBM);
-    // 64-channel blocks when there are more than 32 output channels, else 32
-    const bool wide = Cout > 32;
-    const unsigned int gn = (unsigned int)((Cout + (wide ? 63 : 31)) / (wide ? 64 : 32));
-    const dim3 grid(gm, gn);
-    // halo tiles of 8 x 16 pixels from 64 input channels up
-    const bool halo = Cin >= 2 * kCvBK;
-    const dim3 hgrid((unsigned int)((size_t)B * ((W + 15) / 16) * ((H + 7) / 8)), gn);
-#define CV(E)                                                                                                 \
-    do {                                                                                                      \
-        if (halo && wide) k_conv3x3_halo<E, 2, 8><<<hgrid, 256, 0, s>>>(X, Wt, bias, skip, Y, B, H, W, Cin, Cout); \
-        else if (halo) k_conv3x3_halo<E, 1, 8><<<hgrid, 256, 0, s>>>(X, Wt, bias, skip, Y, B, H, W, Cin, Cout); \
-        else if (wide) k_conv3x3<E, 2><<<grid, 256, 0, s>>>(X, Wt, bias, skip, Y, B, H, W, Cin, Cout);        \
-        else k_conv3x3<E, 1><<<grid, 256, 0, s>>>(X, Wt, bias, skip, Y, B, H, W, Cin, Cout);                  \
-    } while (0)
+    if (a.Cin % kCvBK != 0 || (epi != CNN_F32 && a.Cout % 4 != 0)) return hipErrorInvalidValue;
+    const long tiles = (long)a.B * ((a.W + 15) / 16) * ((a.H + 15) / 16);
+    if (tiles > INT_MAX) return hipErrorInvalidValue;
+    const int couts = epi == CNN_HEAD ? 3 : a.Cout;
+    a.vec = a.Cout % 4 == 0 && (uintptr_t)a.Y % 16 == 0;
+    auto groups = [&](int nj) { return (couts + 16 * nj - 1) / (16 * nj); };
+    const int nj = couts > 32 && tiles * groups(4) >= 256 ? 4 : couts > 16 && (tiles * groups(2) >= 256 || couts <= 32) ? 2 : 1;
+    // resident blocks per CU: 2 of 64 channels, 3 of 32, 4 of 16; every block the same number of tiles
+    const long cap = std::max(1L, (nj == 4 ? 512L : nj == 2 ? 768L : 1024L) / groups(nj));
+    const long rounds = (tiles + cap - 1) / cap;
+    const dim3 grid((unsigned int)((tiles + rounds - 1) / rounds), (unsigned int)groups(nj));
+#define CV(E)                                                          \
+    case E:                                                            \
+        if (nj == 4) k_conv3x3<E, 4><<<grid, 256, 0, s>>>(a);          \
+        else if (nj == 2) k_conv3x3<E, 2><<<grid, 256, 0, s>>>(a);     \
+        else k_conv3x3<E, 1><<<grid, 256, 0, s>>>(a);                  \
+        break
     switch (epi) {
-    case kEpiBias | kEpiRelu: CV(kEpiBias | kEpiRelu); break;
-    case kEpiBias | kEpiRelu | kEpiSkip: CV(kEpiBias | kEpiRelu | kEpiSkip); break;
-    case kEpiBias: CV(kEpiBias); break;
-    case kEpiBias | kEpiF32: CV(kEpiBias | kEpiF32); break;
-    case kEpiF32: CV(kEpiF32); break;
-    case kEpiF32 | kEpiAccum: CV(kEpiF32 | kEpiAccum); break;
-    case 0: CV(0); break;
+        CV(CNN_F32);
+        CV(CNN_FWD);
+        CV(CNN_MASK);
+        CV(CNN_MASK_UP);
+        CV(CNN_MASK_POOL);
+    case CNN_HEAD: k_conv3x3<CNN_HEAD, 1><<<grid, 256, 0, s>>>(a); break;
     default: return hipErrorInvalidValue;
     }
 #undef CV
@@ -810,48 +716,17 @@ size_t cnn_wgrad_ws_floats(int B, int H, int W, int Cin, int Cout)
 // dW (Cout x 9 x Cin) and, when it is not null, db; with ws (of cnn_wgrad_ws_floats)
 // they are set (db must follow dW), without ws they are added to.
 hipError_t cnn_conv_wgrad(const uint16_t *dU, const uint16_t *X, float *dW, float *db, float *ws, int B, int H, int W,
-                          int Cin, int Cout, hipStream_t s)
+                          int Cin, int Cout, int up, hipStream_t s)
 {
     const size_t nw = (size_t)Cout * 9 * Cin;
     if (Cin % 32 != 0 || Cout % 8 != 0 || (ws && db != dW + nw)) return hipErrorInvalidValue;
     bool tall, wide;
     dim3 grid;
     wgrad_plan(B, H, W, Cin, Cout, tall, wide, grid);
-    if (tall) k_conv3x3_wgrad<2, 2, 2><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout);
-    else if (wide) k_conv3x3_wgrad<2, 1, 4><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout);
-    else k_conv3x3_wgrad<1, 2, 2><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout);
+    if (tall) k_conv3x3_wgrad<2, 2, 2><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout, up);
+    else if (wide) k_conv3x3_wgrad<2, 1, 4><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout, up);
+    else k_conv3x3_wgrad<1, 2, 2><<<grid, 256, 0, s>>>(dU, X, dW, db, ws, B, H, W, Cin, Cout, up);
     if (ws) k_wgrad_reduce<<<(unsigned int)((nw + Cout + 63) / 64), 256, 0, s>>>(ws, dW, nw + Cout, (int)grid.x);
-    return hipGetLastError();
-}
-
-hipError_t cnn_relu_bwd(const float *dY, const uint16_t *y, uint16_t *dU, float *dskip, size_t n, int relu,
-                        hipStream_t s)
-{
-    k_relu_bwd<<<ew_blocks(n), 256, 0, s>>>(dY, y, dU, dskip, n, relu);
-    return hipGetLastError();
-}
-
-hipError_t cnn_pool2(const uint16_t *x, uint16_t *y, int B, int H, int W, int C, hipStream_t s)
-{
-    k_pool2<<<ew_blocks((size_t)B * H * W * C / 4), 256, 0, s>>>(x, y, B, H, W, C);
-    return hipGetLastError();
-}
-
-hipError_t cnn_pool2_bwd(const float *dy, float *dx, int B, int H, int W, int C, hipStream_t s)
-{
-    k_pool2_bwd<<<ew_blocks((size_t)B * H * W * C / 4), 256, 0, s>>>(dy, dx, B, H, W, C);
-    return hipGetLastError();
-}
-
-hipError_t cnn_up2(const uint16_t *x, uint16_t *y, int B, int H, int W, int C, hipStream_t s)
-{
-    k_up2<<<ew_blocks((size_t)B * H * W * C * 4), 256, 0, s>>>(x, y, B, H, W, C);
-    return hipGetLastError();
-}
-
-hipError_t cnn_up2_bwd(const float *dy, float *dx, int B, int H, int W, int C, hipStream_t s)
-{
-    k_up2_bwd<<<ew_blocks((size_t)B * H * W * C), 256, 0, s>>>(dy, dx, B, H, W, C);
     return hipGetLastError();
 }
 
@@ -867,22 +742,18 @@ hipError_t cnn_to_bf16(const float *a, uint16_t *b, size_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t cnn_flip_weights(const uint16_t *Wt, uint16_t *Wf, int Cin, int Cout, hipStream_t s)
+hipError_t cnn_flip_weights(const uint16_t *wb, uint16_t *wf, const CnnLayers &l, hipStream_t s)
 {
-    k_flip_weights<<<ew_blocks((size_t)Cout * 9 * Cin), 256, 0, s>>>(Wt, Wf, Cin, Cout);
+    size_t n = 0;
+    for (int i = 0; i < l.n; i++) n = std::max(n, (size_t)l.cout[i] * 9 * l.cin[i]);
+    if (l.n > 0) k_flip_weights<<<dim3(std::min(ew_blocks(n), 512u), l.n), 256, 0, s>>>(wb, wf, l);
     return hipGetLastError();
 }
 
-hipError_t cnn_sq_loss(const float *out, const float *base, const float *target, float *dout, double *partials,
-                       int nblocks, int B, int HW, int co, float scale, hipStream_t s)
+hipError_t cnn_sq_loss(const float *pred, const float *target, uint16_t *dU, double *partials, int nblocks, int B,
+                       int HW, int co, float scale, hipStream_t s)
 {
-    k_sq_loss<<<nblocks, 256, 0, s>>>(out, base, target, dout, partials, B, HW, co, scale);
-    return hipGetLastError();
-}
-
-hipError_t cnn_add_prediction(const float *out, const float *base, float *pred, int B, int HW, int co, hipStream_t s)
-{
-    k_add_prediction<<<ew_blocks((size_t)B * 3 * HW), 256, 0, s>>>(out, base, pred, B, HW, co);
+    k_sq_loss<<<nblocks, 256, 0, s>>>(pred, target, dU, partials, B, HW, co, scale);
     return hipGetLastError();
 }
 

@@ -593,4 +593,36 @@ hipError_t launch_radial_to_ortho(int W, int H, const double *K, float *z, float
 hipError_t launch_sobel(int W, int H, const float *r, const float *g, const float *b, float *gx,
                         float *gy, const float *visf, const uint8_t *visb, hipStream_t s);
 
+// ---- the warm-start network (k_cnn.hip, cnn.cpp) ---------------------------
+
+// What a 3x3 convolution does with its sums v (FP32, bias added):
+enum CnnEpilogue : int {
+    CNN_F32,       // Y (float) = v
+    CNN_FWD,       // Y (bf16) = act(v + aux), and with pool its 2x2 means
+    CNN_HEAD,      // Y (float, planar [B][3][H][W]) = base + the first three channels
+    CNN_MASK,      // Y (bf16) = v where aux > 0, else 0; with dskip the same in FP32 there
+    CNN_MASK_UP,   // Y, aux at half the size: Y (bf16) = the sum of v over 2x2 where aux > 0
+    CNN_MASK_POOL  // Y, aux, dskip at twice the size: Y (bf16) = dskip + v / 4 where aux > 0
+};
+
+// A 3x3 convolution: NHWC bf16 X [B][H][W][Cin] (with up [B][H/2][W/2][Cin],
+// read as its 2x nearest upsampling), weights [Cout][9][Cin].
+struct CnnConv {
+    const uint16_t *X, *Wt;
+    const float *bias;    // nullable
+    const uint16_t *aux;  // CNN_FWD: the skip (nullable); CNN_MASK*: the activations of the ReLU
+    void *Y;
+    float *dskip;         // CNN_MASK: nullable
+    uint16_t *pool;       // CNN_FWD: nullable
+    const float *base;
+    int B, H, W, Cin, Cout, up, relu;
+    int vec;              // set by the launcher: four channels of Y are 16-byte aligned
+};
+
+// Layers by the offsets of their weights (at most 2 levels + 2 (levels - 1) + 1 of 6 levels).
+struct CnnLayers {
+    size_t woff[24];
+    int cin[24], cout[24], n;
+};
+
 }  // namespace lfrv

@@ -301,3 +301,45 @@ def test_conv3x3_wgrad_tile_edges(B, H, W, Cin, Cout):
         want[:, t, :] += Gf.reshape(-1, Cout).T @ Xs.reshape(-1, Cin)
     # FP32 sums of up to B H W products: eps sqrt(n) of their scale sqrt(n), well under 2e-5 of the largest entry
     assert np.max(np.abs(got - want)) <= 2e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("B,H,W,Cin,Cout", [(1, 1, 1, 32, 1), (1, 17, 33, 32, 70),      # 16 channels per block, cut
+                                            (1, 250, 270, 32, 40), (2, 200, 190, 64, 66)])  # 32 and 64 per block
+def test_conv3x3_tile_edges(B, H, W, Cin, Cout):
+    """The convolution at the edges of its pixel tiles and channel blocks, in each block width."""
+    print(f"conv3x3 B={B} {H}x{W} {Cin}->{Cout}", flush=True)
+    L, rng = cnn_lib(), np.random.default_rng([B, H, W, Cin, Cout])
+    X = to_bf16(rng.standard_normal((B, H, W, Cin)).astype(np.float32))
+    Wt = to_bf16(rng.standard_normal((Cout, 9, Cin)).astype(np.float32) / np.sqrt(9 * Cin))
+    b = rng.standard_normal(Cout).astype(np.float32)
+    dX, dW, db, dY = Raw(X), Raw(Wt), Raw(b), Raw(B * H * W * Cout * 4)
+    assert L.lfrv_op_conv3x3(B, H, W, Cin, Cout, dX.ptr, dW.ptr, db.ptr, dY.ptr, None) == 0
+    lfrv.device_sync()
+    Y = dY.get(np.float32, (B, H, W, Cout))
+    Xp = np.pad(from_bf16(X).astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    want = np.zeros((B, H, W, Cout)) + b
+    for t in range(9):
+        want += Xp[:, t // 3:t // 3 + H, t % 3:t % 3 + W, :] @ from_bf16(Wt).astype(np.float64)[:, t, :].T
+    assert np.max(np.abs(Y - want)) <= 2e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("base", [32, 64])
+def test_network_block_widths_agree(base):
+    """64 copies of one image (blocks of 64 channels) against the image alone (narrower blocks, which the oracle
+    checks): the same predictions, and the same gradients up to the order of FP32 sums (1 / 64 is exact)."""
+    rng, B, H, W = np.random.default_rng(base), 64, 40, 24
+    x = rng.uniform(0, 1, (1, H, W, 64)).astype(np.float32)
+    start = rng.uniform(0, 1, (1, 3, H, W)).astype(np.float32)
+    target = (start + 0.1 * rng.standard_normal(start.shape)).astype(np.float32)
+    got = []
+    for n in (1, B):
+        print(f"U-Net levels=3 base={base} B={n} {H}x{W}", flush=True)
+        net = Cnn(64, levels=3, base=base, max_batch=n, max_h=H, max_w=W, seed=5)
+        net.set_batch_host(*[np.repeat(a, n, axis=0) for a in (x, start, target)])
+        pred = net.forward()
+        loss = net.loss_grad()
+        got.append((pred, loss, net.get_grads()))
+    assert np.array_equal(got[1][0], np.repeat(got[0][0], B, axis=0))
+    assert abs(got[1][1] - got[0][1]) <= 1e-6 * got[0][1]
+    # sums of 64 H W terms in FP32: eps times the root of their number
+    assert rel_err(got[1][2], got[0][2]) <= 2e-5
