@@ -230,13 +230,21 @@ extern "C" lfrv_status lfrv_batch_run(lfrv_batch *b, lfrv_batch_result *res)
             const int ks = 3 + gk / 2;
             const bool grad = (gk & 1) != 0;
             const int b0 = (int)work.size();
+            std::vector<StripSize> sizes;  // the strips' height is chosen for the group's launch as a whole
+            for (int k = 0; k < ns; k++)
+                if (b->entries[sr_index[k]].ctx->ks == ks && (sr_items[k].da.beta > 0.0f) == grad)
+                    sizes.push_back({sr_items[k].W, sr_items[k].H});
+            if (sizes.empty()) continue;
+            const int rows = sr_strip_rows(ks, grad, sizes.data(), (int)sizes.size());
             for (int k = 0; k < ns; k++) {
                 if (b->entries[sr_index[k]].ctx->ks != ks || (sr_items[k].da.beta > 0.0f) != grad) continue;
                 const int idx = (int)items_sorted.size();
                 items_sorted.push_back(sr_items[k]);
                 items_sorted.back().theta = nullptr;  // set below, once the device array exists
                 items_sorted.back().NA = sr_items[k].NA;
-                for (int j = 0; j < sr_items[k].ntiles; j++) work.push_back(make_int2(idx, j));
+                const StripGeom sg = sr_strips(ks, grad, {sr_items[k].W, sr_items[k].H}, rows);
+                items_sorted.back().sg = sg;
+                for (int j = 0; j < sg.nblocks; j++) work.push_back(make_int2(idx, j));
                 max_steps = std::max(max_steps, sr_items[k].steps);
                 sorted_theta.push_back(theta_off[k]);
             }

@@ -8,8 +8,10 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <climits>
 #include <chrono>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace lfrv {
@@ -153,7 +155,7 @@ __global__ void __launch_bounds__(kPullMaxThreads) k_sr_dataterm(TileGeom g, Til
 // S, SE, SW planes; the others are the neighbours' couplings), G9' is the same
 // without omega (gw_type 0), bI = sum omega t v, bG = sum t lap v [* omega].
 // They are assembled once per set of weights (k_sr_assemble); every outer
-// step is then a tiled stencil (k_sr_dataterm_st): box sums, the 9-point
+// step is then a stencil (k_sr_step_st): box sums, the 9-point
 // couplings, and the box sums back onto the pixels.  The step weighs the two
 // terms' back-projections by constants of the parameters before adding them
 // per pixel (cI = alpha sigma^2, cG = -beta gradient_step [sigma^2]), and the
@@ -236,486 +238,401 @@ __global__ void __launch_bounds__(kPullMaxThreads) k_sr_assemble(TileGeom g, Til
     }
 }
 
-// One outer step's data term on a 32 x 16 pixel tile from the assembled
-// operator.  Every global load of the block (U with its halo, the couplings
-// and right-hand sides of the tile's anchors, coverage) is issued first; the
-// rest runs in LDS: lap U, the box sums BU / BL at the anchors (+1 ring), the
-// anchor residuals QI = G9 BU - bI (with the gradient term the weighted sum
-// cI G9 BU + cG dsf^2 G9' BL - b), then the box sums back onto the pixels,
-// split into rows and columns.
-constexpr int kStTW = 32, kStTH = 16;
+// ---- dsf >= 2: the outer step as a marching stencil -------------------------
+//
+// A wave owns a strip of the target, 64 columns wide with its halo, and
+// marches down its rows; everything between two rows stays in its registers,
+// and columns meet by DPP shifts of the wave (folded into the additions), so
+// the pass has neither LDS nor barriers.  Per row, from the row of U that
+// came last: lap U one row behind; the D-wide row sums of both (D = dsf), and
+// their D-high column sums BU, BL kept as D - 1 partial chains; the anchor
+// residuals one row behind those, q = G9 BU - bI (with the gradient term the
+// weighted sum cI G9 BU + cG dsf^2 G9' BL - b; G9 the 9-point anchor couplings,
+// of which five planes are stored and the other four are the neighbours' own,
+// shifted over); their row sums and
+// column chains back onto the pixels; the clamped gradient step F; the dual
+// and primal update.  The output row lags the U row by LAG = D (+ 1 with the
+// Laplacian), and LAG columns at each end of the wave are halo: 54 - 60 of the
+// 64 lanes have an output.
+// Bounds: at large targets the bytes of the step (25 views, 2048^2, dsf 4: 555
+// MB in 141 us, 3.9 TB/s; 188 us before), at small ones the latency of the rows
+// of one wave (256^2, dsf 2: 6.6 us per step; 7.1 before).  The tile form this
+// replaced (32 x 16 pixels, nine LDS phases, 2.1 x halo loads) was bound by its
+// LDS and address instructions.  Results are its own bit for bit: sums in its
+// order, the contractions written out.
+// Loads and stores go through buffer descriptors, and a lane or row outside
+// its plane takes the offset kOutside, past every buffer: it reads 0 and writes
+// nothing, without a compare per value.  Every row issues the same loads and
+// stores, outside any branch, so that the waits count exactly the younger ones
+// and the next two rows' loads stay in flight.  The rows before the first
+// output are peeled off (they need only part of the row's work).
+// The arithmetic of a pixel does not depend on the strip it falls in, so
+// strips of any height, and batches, give the same bits.
 
-// Every LDS plane of the tile has the row pitch P of the widest one (U with
-// its ring) and every pass maps consecutive threads to consecutive points of
-// that pitch (idle where x is past the pass's width), so a wave's accesses are
-// contiguous and free of bank conflicts; a pitch per plane made them jump at
-// each row wrap.
-// GRAD: the gradient-constraint term is on (dt_beta > 0): lap U, its box
-// sums and residuals are formed too (NC = 6 planes instead of 3).
-template <int KS, bool GRAD = true>
-struct StDims {
-    static constexpr int D = KS - 1, TW = kStTW, TH = kStTH, NT = TW * TH;
-    static constexpr int NC = GRAD ? 6 : 3;
-    static constexpr int QW = TW + D - 1, QH = TH + D - 1;  // anchor points x' = tx0 + qx
-    static constexpr int BW = QW + 2, BH = QH + 2;          // box sums at x' = tx0 - 1 + bx
-    static constexpr int LW = BW + D - 1, LH = BH + D - 1;  // pixels tx0 - D + lx (box sums' support)
-    static constexpr int SW = LW + 2, SH = LH + 2;          // U from tx0 - D - 1 (the Laplacian's ring)
-    static constexpr int P = SW;                            // the common row pitch
-    // The two LDS regions take turns: sa holds U and lap U, sb their row sums
-    // (D > 2); then the box sums BU, BL go to the region nobody reads any more
-    // (sa for D > 2, sb for D <= 2), the anchor residuals to the other one, and
-    // (D > 2) the residuals' row sums to sa again; sb ends with the duals of
-    // the primal-dual step (6 planes of (TH + 1) x (TW + 2)).
-    static constexpr int A1 = 3 * SH * P + (GRAD ? 3 * LH * P : 0), A2 = 3 * QH * P;  // (3 residual planes)
-    static constexpr int AREA = A1 > A2 ? A1 : A2;
-    static constexpr int HR = BH + D - 1;  // rows of the horizontal box sums
-    // D > 2: the row sums keep only the BW columns the column sums read (pitch
-    // BW: a wave's active lanes then write and read consecutive words);
-    // D <= 2: the box sums themselves
-    static constexpr int B1 = D > 2 ? NC * HR * BW : NC * BH * P, B2 = 6 * (TH + 1) * (TW + 2);
-    static constexpr int BAREA = B1 > B2 ? B1 : B2;  // sb
-    static constexpr int NQP = QH * P;               // anchor slots (qx < QW used)
-    static constexpr int NQT = (NQP + NT - 1) / NT, NST = (SH * P + NT - 1) / NT;
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        static_for<N, I + 1>(f);
+    }
+}
+
+constexpr int kStripGroup = 3;  // rows per turn of the loop
+
+template <int D, bool GRAD>
+struct Strip {
+    static constexpr int LAG = D + (GRAD ? 1 : 0), OW = 64 - 2 * LAG;  // output columns
 };
 
-// The data term of one 32 x 16 tile.  Every thread of the block calls it; on
-// return each thread holds F (the clamped gradient step) and U at its pixel,
-// and the pixel's coverage; sb is free for the caller at once, sa only after
-// a barrier.  With ur, the U values of
-// [tx0-1, tx0+TW] x [ty0-1, ty0+TH] (3 planes, pitch TW+2) are also left there.
-template <int KS, bool GRAD>
-__device__ __forceinline__ void sr_dataterm_tile(int W, int H, int Wc, int Hc, int tx0, int ty0, const DataTermArgs &da,
-                                                 const float *__restrict__ U, const float *__restrict__ ops, size_t NA,
-                                                 const float *__restrict__ coverage, float *sa, float *sb,
-                                                 float (&F)[3], float (&up)[3], float &cov, float *ur = nullptr)
+// The lane's left (x - 1) / right (x + 1) neighbour's value, 0 past the wave
+// (every lane has to take part: never inside a select).
+__device__ __forceinline__ float from_left(float v)
 {
-    using S = StDims<KS, GRAD>;
-    constexpr int D = S::D, TW = S::TW, NT = S::NT, QW = S::QW, QH = S::QH, BW = S::BW, BH = S::BH, LW = S::LW,
-                  LH = S::LH, SH = S::SH, P = S::P, NQP = S::NQP, NQT = S::NQT, NST = S::NST;
-    constexpr bool SEP = D > 2;  // separable box sums
-    static_assert(S::NC * BH * P <= (SEP ? S::AREA : S::BAREA) && 3 * NQP <= (SEP ? S::BAREA : S::AREA) &&
-                      3 * QH * TW <= S::AREA,
-                  "the box sums, residuals and row sums fit their LDS regions");
-    float *us = sa, *ls = sa + 3 * SH * P;
-    float *bus = SEP ? sa : sb, *bls = bus + 3 * BH * P;
-    float *qs = SEP ? sb : sa;
-    float *rs = sa;  // D > 2: the residuals' row sums, once BU and BL are read
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));  // wave_shr:1
+}
+__device__ __forceinline__ float from_right(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));  // wave_shl:1
+}
+
+constexpr int kOutside = (int)0x80000000;
+constexpr size_t kNarrowBytes = (size_t)1 << 31;  // kOutside lies past any buffer up to this size
+
+// Planes of `w`-wide rows, `stride` values apart.  Narrow: one descriptor for
+// all of them (at most kNarrowBytes), the row and plane in the scalar offset.
+// WIDE: a descriptor per row.
+template <bool WIDE>
+struct Planes {
+    const float *base;
+    size_t stride;
+    int w;
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Planes(const float *b, int n, size_t st, int width) : base(b), stride(st), w(width)
+    {
+        if constexpr (!WIDE) r = __builtin_amdgcn_make_buffer_rsrc((void *)b, 0, b ? (int)(4 * n * st) : 0, 0x00020000);
+    }
+    // plane c, row y (clamped at 0; a row outside comes with vo = kOutside)
+    __device__ __forceinline__ float load(int c, int y, int vo) const
+    {
+        if constexpr (WIDE) return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(row(c, y), vo, 0, 0));
+        else return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo, 4 * (c * (int)stride + max(y, 0) * w), 0));
+    }
+    __device__ __forceinline__ void store(float v, int c, int y, int vo) const
+    {
+        if constexpr (WIDE) __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), row(c, y), vo, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, vo, 4 * (c * (int)stride + max(y, 0) * w), 0);
+    }
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t row(int c, int y) const
+    {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(base + c * stride + (size_t)max(y, 0) * w), 0, base ? 4 * w : 0,
+                                                 0x00020000);
+    }
+};
+
+// n / d for finite values away from the ends of the range, correctly rounded:
+// a Newton step for the reciprocal, which several quotients of one divisor
+// share, then two for the quotient.
+struct Divisor {
+    float d, r;
+    __device__ __forceinline__ explicit Divisor(float div) : d(div), r(__builtin_amdgcn_rcpf(div))
+    {
+        r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    }
+    __device__ __forceinline__ float of(float n) const
+    {
+        float q = n * r;
+        q = fmaf(fmaf(-d, q, n), r, q);
+        return fmaf(fmaf(-d, q, n), r, q);
+    }
+};
+
+// The step's buffers (U read, the rest nullable where the caller's form skips it).
+struct StepBufs {
+    const float *U, *ops, *coverage, *px, *py, *g;
+    float *pxout, *pyout, *unew, *uq_relax, *gout, *norm_mask;
+};
+
+// Rows y0 .. y1 - 1 of the strip whose first output column is x0.  With PD the
+// data term and the first primal-dual iteration (k_pd_step's update, with
+// Uq = U as the step sets it, optimization.cu:1765-1767): the new primal goes
+// to unew, with uq_relax the over-relaxed one (vtv_rof.cu:28-45) there, with
+// gout F.  Without PD F goes to gout and U to uq_relax.  EXTRA: one of
+// uq_relax, gout and norm_mask is given.
+template <int D, bool GRAD, bool PD, bool EXTRA, bool WIDE>
+__device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, int Wc, int Hc, size_t NA,
+                                         const DataTermArgs &da, const PdArgs &pa, const StepBufs &sb)
+{
+    constexpr int LAG = Strip<D, GRAD>::LAG, OW = Strip<D, GRAD>::OW, RING = LAG < kStripGroup ? kStripGroup : 2 * kStripGroup, NB = 3, G = GRAD ? 1 : 0;
+    static_assert(LAG < RING && kStripGroup % NB == 0, "the ring holds the rows from the output row to the newest");
     const size_t N = (size_t)W * H;
-    constexpr bool grad = GRAD;  // da.beta > 0
-    const float *g9 = da.gw_type ? ops : ops + 8 * NA;  // couplings of the gradient term
+    const int lane = threadIdx.x & 63, x = x0 - LAG + lane;
+    const bool xin = x >= 0 && x < W;
+    const int vx = xin ? 4 * x : kOutside, vc = x >= 0 && x < Wc ? 4 * x : kOutside;
+    const int vs = lane >= LAG && lane < LAG + OW ? vx : kOutside;  // the lanes with an output
+    // cuda_laplacian_device (vtv_sr_kernels_unstructured.cu:720-761), no hole gating: the mean of the neighbours
+    // inside the image, on inner and on edge rows
+    const float nx = (x > 0 ? 1.0f : 0.0f) + (x < W - 1 ? 1.0f : 0.0f);
+    const float n_inner = xin ? nx + 2.0f : 1.0f, n_edge = xin ? nx + (H > 1 ? 1.0f : 0.0f) : 1.0f;
     const float ci = dt_intensity_weight(da), cgd = dt_gradient_weight(da) * da.dsf2;
-    const int tid = threadIdx.x;
+    const Divisor vden(pa.tau + pa.lam);
+    const float sgx = xin && x < W - 1 ? pa.sigma : 0.0f;
+    const float gnone = sb.g ? 0.0f : 1.0f;  // the TV weight where there is no map
+    const Planes<WIDE> bU(sb.U, 3, N, W), bC(sb.ops, 5, NA, Wc), bB(sb.ops + 5 * NA, 3, NA, Wc),
+        bE(da.gw_type ? sb.ops : sb.ops + 8 * NA, GRAD ? 5 : 0, NA, Wc), bPx(sb.px, 3, N, W), bPy(sb.py, 3, N, W),
+        bG(sb.g, 1, N, W), bCov(sb.coverage, 1, N, W), bPxo(sb.pxout, 3, N, W), bPyo(sb.pyout, 3, N, W),
+        bUn(sb.unew, 3, N, W), bUq(sb.uq_relax, 3, N, W), bGo(sb.gout, 3, N, W), bNm(sb.norm_mask, 1, N, W);
+    const int first = y0 - LAG, yend = y1 + LAG;  // rows of U
 
-    // ---- all global loads ----
-    float uv[NST][3];
+    // the loads of one row: U's new row, the operator one row behind the box sums, the output row's own
+    struct Loads {
+        float u[3], f[1 + G][5], b[3], p[PD ? 6 : 1], g, cov;
+    } ld[NB];
+    auto fetch = [&](Loads &l, int yn) __attribute__((always_inline)) {
+        const int yq = yn - G - 1, yo = yn - LAG;
+        const int vu = yn >= 0 && yn < min(H, yend) ? vx : kOutside;
+        const int vq = yq >= max(0, y0 - 1) && yq < Hc && yn < yend ? vc : kOutside;
+        const int vp = yo >= max(0, y0 - 1) && yo < y1 ? vx : kOutside;
 #pragma unroll
-    for (int k = 0; k < NST; k++) {
-        const int i = tid + k * NT;
-        const int x = tx0 - D - 1 + i % P, y = ty0 - D - 1 + i / P;
-        const bool in = i < SH * P && x >= 0 && x < W && y >= 0 && y < H;
-        const size_t o = in ? (size_t)y * W + x : 0;
+        for (int c = 0; c < 3; c++) l.u[c] = bU.load(c, yn, vu);
 #pragma unroll
-        for (int c = 0; c < 3; c++) uv[k][c] = in ? U[c * N + o] : 0.0f;
-    }
-    float cf[NQT][9], cg[NQT][9], bi[NQT][3];  // bi: bI, or b with the gradient term
-#pragma unroll
-    for (int k = 0; k < NQT; k++) {
-        const int i = tid + k * NT;
-        const int xq = tx0 + i % P, yq = ty0 + i / P;
-        const bool in = i < NQP && i % P < QW && xq < Wc && yq < Hc;
-        const int xc = min(xq, Wc - 1), yc = min(yq, Hc - 1);
-        const size_t o = (size_t)yc * Wc + xc;
-        const bool xm = xc > 0, ym = yc > 0, xp = xc < Wc - 1;
-        const size_t oE = xm ? o - 1 : o, oS = ym ? o - Wc : o, oSE = (xm && ym) ? o - Wc - 1 : o,
-                     oSW = (xp && ym) ? o - Wc + 1 : o;
-        auto load9 = [&](const float *Q, float(&f)[9]) {
-            f[0] = Q[o];
-            f[1] = Q[NA + o];
-            f[2] = Q[2 * NA + o];
-            f[3] = Q[3 * NA + o];
-            f[4] = Q[4 * NA + o];
-            const float e = Q[NA + oE], sn = Q[2 * NA + oS], se = Q[3 * NA + oSE], sw = Q[4 * NA + oSW];
-            f[5] = xm ? e : 0.0f;
-            f[6] = ym ? sn : 0.0f;
-            f[7] = (xm && ym) ? se : 0.0f;
-            f[8] = (xp && ym) ? sw : 0.0f;
-            if (!in)
-#pragma unroll
-                for (int q = 0; q < 9; q++) f[q] = 0.0f;
-        };
-        load9(ops, cf[k]);
-#pragma unroll
-        for (int c = 0; c < 3; c++) bi[k][c] = in ? ops[(size_t)(5 + c) * NA + o] : 0.0f;
-        if (grad) load9(g9, cg[k]);
-    }
-    const int px = tx0 + tid % TW, py = ty0 + tid / TW;
-    const bool pin = px < W && py < H;
-    const size_t po = pin ? (size_t)py * W + px : 0;
-    cov = pin ? coverage[po] : 0.0f;
-#pragma unroll
-    for (int c = 0; c < 3; c++) up[c] = pin ? U[c * N + po] : 0.0f;
-
-    // ---- U, lap U, box sums ----
-#pragma unroll
-    for (int k = 0; k < NST; k++) {
-        const int i = tid + k * NT;
-        if (i < SH * P)
-#pragma unroll
-            for (int c = 0; c < 3; c++) us[c * SH * P + i] = uv[k][c];
-        if (ur) {
-            // the ring of the primal-dual step: U tile coordinates (D, D) on
-            constexpr int RW = TW + 2, RH = S::TH + 2;
-            const int rx = i % P - D, ry = i / P - D;
-            if (i < SH * P && rx >= 0 && rx < RW && ry >= 0 && ry < RH)
-#pragma unroll
-                for (int c = 0; c < 3; c++) ur[(c * RH + ry) * RW + rx] = uv[k][c];
+        for (int k = 0; k < 5; k++) {
+            l.f[0][k] = bC.load(k, yq, vq);
+            if constexpr (GRAD) l.f[G][k] = bE.load(k, yq, vq);
         }
-    }
-    __syncthreads();
-    if (grad) {
-        // cuda_laplacian_device (vtv_sr_kernels_unstructured.cu:720-761), no hole gating
-        for (int i = tid; i < LH * P; i += NT) {
-            const int lx = i % P, ly = i / P;
-            if (lx >= LW) continue;
-            const int x = tx0 - D + lx, y = ty0 - D + ly;
-            const int ui = i + P + 1;  // the pixel in the U tile
+#pragma unroll
+        for (int c = 0; c < 3; c++) l.b[c] = bB.load(c, yq, vq);
+        l.cov = bCov.load(0, yo, vp);
+        if constexpr (PD) {
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                float v = 0.0f;
-                if (x >= 0 && x < W && y >= 0 && y < H) {
-                    const float *u = us + c * SH * P;
-                    float sm = 0.0f, wsum = 0.0f;
-                    if (x > 0) { sm += u[ui - 1]; wsum += 1.0f; }
-                    if (y > 0) { sm += u[ui - P]; wsum += 1.0f; }
-                    if (x < W - 1) { sm += u[ui + 1]; wsum += 1.0f; }
-                    if (y < H - 1) { sm += u[ui + P]; wsum += 1.0f; }
-                    v = sm / wsum - u[ui];
-                }
-                ls[c * LH * P + i] = v;
+                l.p[c] = bPx.load(c, yo, vp);
+                l.p[3 + c] = bPy.load(c, yo, vp);
+            }
+            l.g = bG.load(0, yo, vp);
+        }
+    };
+    float u[RING][3];                       // U's last rows
+    float bc[1 + G][3][D - 1];              // column chains of U's and lap U's row sums
+    // BU, BL of the two rows before the newest, at the lane's left, own and right anchor
+    float bm[1 + G][3][3], b0[1 + G][3][3];
+    // the operator row above: its south, the left neighbour's south-east, the right one's south-west
+    float s1[1 + G], s2[1 + G], s3[1 + G];
+    float qc[3][D - 1], py1[3];             // column chains of the residuals' row sums; the duals of the row above
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+#pragma unroll
+        for (int k = 0; k < RING; k++) u[k][c] = 0.0f;
+#pragma unroll
+        for (int t = 0; t <= G; t++) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) bm[t][c][d] = b0[t][c][d] = 0.0f;
+#pragma unroll
+            for (int d = 0; d < D - 1; d++) bc[t][c][d] = 0.0f;
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; d++) qc[c][d] = 0.0f;
+        py1[c] = 0.0f;
+    }
+#pragma unroll
+    for (int t = 0; t <= G; t++) s1[t] = s2[t] = s3[t] = 0.0f;
+    // the sum of the last D rows' values, added from the oldest on
+    auto chain = [](float(&ch)[D - 1], float v) __attribute__((always_inline)) {
+        const float sum = ch[D - 2] + v;
+#pragma unroll
+        for (int d = D - 2; d > 0; d--) ch[d] = ch[d - 1] + v;
+        ch[0] = v;
+        return sum;
+    };
+    // Row first + i with k = i modulo RING.  PHASE 0: box sums only; 1: and the residuals; 2: and the duals of
+    // row y0 - 1; 3: an output row.
+    auto row = [&](auto K, auto PHASE, int i) __attribute__((always_inline)) {
+        constexpr int k = decltype(K)::value, ph = decltype(PHASE)::value;
+        constexpr int ku = k % RING, k1 = (k + RING - 1) % RING, k2 = (k + RING - 2) % RING,
+                      ko = (k + RING - LAG) % RING;
+        const int yn = first + i, yb = yn - G, yo = yn - LAG;
+        const Loads &l = ld[k % NB];
+        fetch(ld[(k + 2) % NB], yn + 2);
+#pragma unroll
+        for (int c = 0; c < 3; c++) u[ku][c] = l.u[c];
+        // row sums of U and lap U at row yb, BU and BL of the anchor row yb
+        float bp[1 + G][3][3];
+        // (+: of the values; a choice between the captured variables would keep them all in memory)
+        const Divisor nn4(GRAD ? (yb > 0 && yb < H - 1 ? +n_inner : +n_edge) : 1.0f);
+        const bool bin = xin && yb >= 0 && yb < H;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const float uc = GRAD ? u[k1][c] : u[ku][c];
+            if constexpr (GRAD) {
+                const float sum = ((from_left(uc) + u[k2][c]) + from_right(uc)) + u[ku][c];
+                float t = nn4.of(sum) - uc;
+                t = bin ? t : 0.0f;
+                float rs = t;
+#pragma unroll
+                for (int d = 1; d < D; d++) rs = t + from_left(rs);
+                bp[G][c][1] = chain(bc[G][c], rs);
+            }
+            float rs = uc;
+#pragma unroll
+            for (int d = 1; d < D; d++) rs = uc + from_left(rs);
+            bp[0][c][1] = chain(bc[0][c], rs);
+#pragma unroll
+            for (int t = 0; t <= G; t++) {
+                bp[t][c][0] = from_left(bp[t][c][1]);
+                bp[t][c][2] = from_right(bp[t][c][1]);
             }
         }
-        __syncthreads();
-    }
-    // D x D box sums.  D <= 2: each box point reads its D x D values directly
-    // (as many reads as the separable form, one barrier instead of three; the
-    // sums are added in the separable form's order).  Larger D: separably,
-    // the row sums of U (rows 1.. of the U tile) and lap U (rows 0..) into sb,
-    // then their column sums into sa, which nothing reads any more.
-    if constexpr (D <= 2) {
-        for (int i = tid; i < BH * P; i += NT) {
-            if (i % P >= BW) continue;
+        float up[3] = {0, 0, 0}, acc[3] = {0, 0, 0};
+        if constexpr (ph >= 1) {
+            // residuals of the anchor row yb - 1, and back onto the pixels of row yo
+            float fw[1 + G];  // west: the left neighbour's own east
+#pragma unroll
+            for (int t = 0; t <= G; t++) fw[t] = from_left(l.f[t][1]);
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                float su = 0.0f, sl = 0.0f;
+                float st[1 + G];
 #pragma unroll
-                for (int l = 0; l < D; l++) {
-                    float ru = 0.0f, rl = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < D; k++) {
-                        ru += us[c * SH * P + i + (l + 1) * P + k + 1];
-                        if (grad) rl += ls[c * LH * P + i + l * P + k];
-                    }
-                    su += ru;
-                    sl += rl;
+                for (int t = 0; t <= G; t++) {
+                    const float *f = l.f[t], *m = bm[t][c], *z = b0[t][c], *p = bp[t][c];  // (left, own, right)
+                    float w = fmaf(f[0], z[1], f[1] * z[2]);
+                    w = fmaf(f[2], p[1], fmaf(fw[t], z[0], w));
+                    w = fmaf(f[3], p[2], fmaf(s1[t], m[1], w));
+                    w = fmaf(f[4], p[0], fmaf(s2[t], m[0], w));
+                    st[t] = fmaf(s3[t], m[2], w);
                 }
-                bus[c * BH * P + i] = su;
-                if (grad) bls[c * BH * P + i] = sl;
+                const float q = (GRAD ? fmaf(ci, st[0], cgd * st[G]) : st[0]) - l.b[c];
+                float rs = q, qr = q;
+#pragma unroll
+                for (int d = 1; d < D; d++) {
+                    qr = from_right(qr);
+                    rs += qr;
+                }
+                acc[c] = chain(qc[c], rs);
+                up[c] = u[ko][c];  // LAG rows ago
             }
         }
-        __syncthreads();
-    } else {
-    constexpr int HR = S::HR, NBT = (BH * P + NT - 1) / NT;
-    float *hsu = sb, *hsl = sb + 3 * HR * BW;  // pitch BW
-    for (int i = tid; i < HR * P; i += NT) {
-        if (i % P >= BW) continue;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            float su = 0.0f, sl = 0.0f;
-#pragma unroll
-            for (int k = 0; k < D; k++) {
-                su += us[c * SH * P + i + P + k + 1];
-                if (grad) sl += ls[c * LH * P + i + k];
-            }
-            const int h = i / P * BW + i % P;
-            hsu[c * HR * BW + h] = su;
-            if (grad) hsl[c * HR * BW + h] = sl;
-        }
-    }
-    __syncthreads();
-    float bsum[NBT][6];
-#pragma unroll
-    for (int k = 0; k < NBT; k++) {
-        const int i = tid + k * NT;
-#pragma unroll
-        for (int c = 0; c < 6; c++) bsum[k][c] = 0.0f;
-        if (i >= BH * P || i % P >= BW) continue;
-        const int h = i / P * BW + i % P;
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                bsum[k][c] += hsu[c * HR * BW + h + l * BW];
-                if (grad) bsum[k][3 + c] += hsl[c * HR * BW + h + l * BW];
-            }
-    }
-    // BU and BL go to sa, which the row sums no longer read: no barrier here
-#pragma unroll
-    for (int k = 0; k < NBT; k++) {
-        const int i = tid + k * NT;
-        if (i >= BH * P || i % P >= BW) continue;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            bus[c * BH * P + i] = bsum[k][c];
-            if (grad) bls[c * BH * P + i] = bsum[k][3 + c];  // (no room for BL without the gradient term)
-        }
-    }
-    __syncthreads();
-    }
-
-    // ---- anchor residuals ----
-#pragma unroll
-    for (int k = 0; k < NQT; k++) {
-        const int i = tid + k * NT;
-        if (i >= NQP || i % P >= QW) continue;
-        const int b = i + P + 1;  // the point in the box-sum tile
-        auto st9 = [&](const float *B, const float(&f)[9]) {
-            return f[0] * B[b] + f[1] * B[b + 1] + f[5] * B[b - 1] + f[2] * B[b + P] + f[6] * B[b - P] +
-                   f[3] * B[b + P + 1] + f[7] * B[b - P - 1] + f[4] * B[b + P - 1] + f[8] * B[b - P + 1];
-        };
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            if (grad)
-                qs[c * NQP + i] = ci * st9(bus + c * BH * P, cf[k]) + cgd * st9(bls + c * BH * P, cg[k]) - bi[k][c];
-            else
-                qs[c * NQP + i] = st9(bus + c * BH * P, cf[k]) - bi[k][c];
-        }
-    }
-    __syncthreads();
-    // rows: r(x, qy) = sum_k q(x + k, qy), stored with pitch TW for the pixel
-    // pass (D <= 2: the pixel pass reads its D x D residuals directly)
-    if constexpr (D > 2) {
-    for (int i = tid; i < QH * P; i += NT) {
-        const int lx = i % P, qy = i / P;
-        if (lx >= TW) continue;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            float sm = 0.0f;
-#pragma unroll
-            for (int k = 0; k < D; k++) sm += qs[c * NQP + i + k];
-            rs[(c * QH + qy) * TW + lx] = sm;
-        }
-    }
-    __syncthreads();
-    }
-
-    // ---- pixel: columns of the row sums, then the step of vtv_sr_ista_step_unstructured ----
-    const int lx = tid % TW, ly = tid / TW;
-    float acc[3];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        float sm = 0.0f;
-        if constexpr (D <= 2) {
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                float row = 0.0f;
-#pragma unroll
-                for (int k = 0; k < D; k++) row += qs[c * NQP + (ly + l) * P + lx + k];
-                sm += row;
-            }
-        } else {
-#pragma unroll
-            for (int l = 0; l < D; l++) sm += rs[(c * QH + ly + l) * TW + lx];
-        }
-        acc[c] = sm;
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        float G = 0.0f;
-        if (grad) {  // both terms, weighted in the residual
-            G = acc[c];
-            if (cov != 0.0f) G /= cov;
-        } else if (da.alpha > 0.0f) {
-            float gi = acc[c];
-            if (cov != 0.0f) gi /= cov;
-            gi *= da.sigma2;
-            G += da.alpha * gi;
-        }
-        G = fminf(1.0f, fmaxf(-1.0f, G));
-        G *= da.prox_factor;
-        G += up[c];
-        F[c] = fminf(1.0f, fmaxf(0.0f, G));
-    }
-    // no barrier here: sb is free since the residual phase's barrier, while
-    // other threads may still read sa
-}
-
-template <int KS, bool GRAD>
-__global__ void __launch_bounds__(kStTW * kStTH) k_sr_dataterm_st(int W, int H, int Wc, int Hc, int ntx, int ntiles,
-                                                                   DataTermArgs da, const float *__restrict__ U,
-                                                                   const float *__restrict__ ops, size_t NA,
-                                                                   const float *__restrict__ coverage,
-                                                                   float *__restrict__ Gout, float *__restrict__ Uq,
-                                                                   float *__restrict__ norm_mask, const int *halt)
-{
-    if (halt && *halt) return;  // a step enqueued behind a stopping rule that fired
-    __shared__ float sa[StDims<KS, GRAD>::AREA];
-    __shared__ float sb[StDims<KS, GRAD>::BAREA];
-    const int t = xcd_tile(blockIdx.x, ntiles);
-    const int tx0 = (t % ntx) * kStTW, ty0 = (t / ntx) * kStTH;
-    float F[3], up[3], cov;
-    sr_dataterm_tile<KS, GRAD>(W, H, Wc, Hc, tx0, ty0, da, U, ops, NA, coverage, sa, sb, F, up, cov);
-    const int px = tx0 + threadIdx.x % kStTW, py = ty0 + threadIdx.x / kStTW;
-    if (px >= W || py >= H) return;
-    const size_t N = (size_t)W * H, po = (size_t)py * W + px;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        Gout[c * N + po] = F[c];
-        Uq[c * N + po] = up[c];
-    }
-    if (da.alpha > 0.0f || da.beta > 0.0f) norm_mask[po] = cov;
-}
-
-
-// One outer step for dsf >= 2 in one pass: the data term of the tile, then
-// the first primal-dual iteration on it (k_pd_step's update, with Uq = U as the
-// step sets it, optimization.cu:1765-1767).  U is only read; the new primal
-// goes to unew.  With uq_relax (the step's only inner iteration) the
-// over-relaxation of vtv_rof.cu:28-45 is fused too: uq_relax <- U + theta (new -
-// U).  Gout (nullable) receives F for further inner iterations.  uq_relax and
-// norm_mask are nullable: a run of fixed steps reads neither between its steps
-// (the next step starts from the new primal, and the mask is the coverage
-// again), so only its last step writes them.
-// The step on tile t (of the W x H target's ntx-wide tile grid); every
-// thread of the block calls it.
-template <int KS, bool GRAD>
-__device__ __forceinline__ void sr_step_tile(int t, int W, int H, int Wc, int Hc, int ntx, const DataTermArgs &da,
-                                             const PdArgs &pa, const float *__restrict__ U,
-                                             const float *__restrict__ ops, size_t NA,
-                                             const float *__restrict__ coverage, const float *__restrict__ pxin,
-                                             const float *__restrict__ pyin, const float *__restrict__ g,
-                                             float *__restrict__ pxout, float *__restrict__ pyout,
-                                             float *__restrict__ unew, float *__restrict__ uq_relax,
-                                             float *__restrict__ Gout, float *__restrict__ norm_mask)
-{
-    constexpr int TW = kStTW, TH = kStTH, NT = TW * TH;
-    constexpr int UW = TW + 2, UH = TH + 2;  // U region [x0-1, x0+TW] x [y0-1, y0+TH]
-    constexpr int PW = TW + 1, PH = TH + 1;  // p region [x0-1, x0+TW-1] x [y0-1, y0+TH-1]
-    constexpr int NPP = PH * UW;             // p slots with the U region's pitch (x < PW used)
-    constexpr int NPT = (NPP + NT - 1) / NT;
-    static_assert(6 * NPP <= StDims<KS, GRAD>::BAREA, "primal-dual tiles exceed the data term's second LDS region");
-    static_assert(UW == kStTW + 2 && UH == kStTH + 2, "the ring the data term leaves");
-    __shared__ float sa[StDims<KS, GRAD>::AREA];
-    __shared__ float sb[StDims<KS, GRAD>::BAREA];
-    __shared__ float us[3 * UH * UW];  // U on the primal-dual step's ring, left by the data term's staging
-    const int tx0 = (t % ntx) * TW, ty0 = (t / ntx) * TH;
-    const size_t N = (size_t)W * H;
-    const int tid = threadIdx.x;
-    // the dual inputs of this thread's p points and the TV weight there, loaded
-    // first so that they arrive while the data term runs
-    float pa_in[NPT][6], gr[NPT];
-#pragma unroll
-    for (int k = 0; k < NPT; k++) {
-        const int i = tid + k * NT;
-        const int x = tx0 - 1 + i % UW, y = ty0 - 1 + i / UW;
-        const bool in = i < NPP && i % UW < PW && x >= 0 && x < W && y >= 0 && y < H;
-        const size_t o = in ? (size_t)y * W + x : 0;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            pa_in[k][c] = in ? pxin[c * N + o] : 0.0f;
-            pa_in[k][3 + c] = in ? pyin[c * N + o] : 0.0f;
-        }
-        gr[k] = (in && g) ? g[o] : 1.0f;
-    }
-    float F[3], up[3], cov;
-    sr_dataterm_tile<KS, GRAD>(W, H, Wc, Hc, tx0, ty0, da, U, ops, NA, coverage, sa, sb, F, up, cov, us);
-
-    // ---- the primal-dual iteration (vtv_rof.cu:118-147, 280-321; cuda_kernels.cu:504-532) ----
-    float *ps = sb;  // free once the data term returns (sa may still be read)
-#pragma unroll
-    for (int k = 0; k < NPT; k++) {
-        const int i = tid + k * NT;
-        if (i >= NPP || i % UW >= PW) continue;
-        const int lx = i % UW, ly = i / UW;
-        const int x = tx0 - 1 + lx, y = ty0 - 1 + ly;
         float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
-        if (x >= 0 && x < W && y >= 0 && y < H) {
+        if constexpr (PD && ph >= 2) {
+            // the duals (vtv_rof.cu:118-147, 280-321)
+            const float sgy = yo < H - 1 ? pa.sigma : 0.0f;
             float nn = 0.0f;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                // the p region and the U region share the origin (x0-1, y0-1)
-                const float *u = us + c * UH * UW;
-                const float uc = u[i];
-                const float gx = (x < W - 1) ? u[i + 1] - uc : 0.0f;
-                const float gy = (y < H - 1) ? u[i + UW] - uc : 0.0f;
-                a[c] = pa_in[k][c] + pa.sigma * gx;
-                b[c] = pa_in[k][3 + c] + pa.sigma * gy;
-                nn += a[c] * a[c] + b[c] * b[c];
+                a[c] = fmaf(sgx, from_right(up[c]) - up[c], l.p[c]);
+                b[c] = fmaf(sgy, u[(ko + 1) % RING][c] - up[c], l.p[3 + c]);
+                nn += fmaf(a[c], a[c], b[c] * b[c]);
             }
             nn = sqrtf(nn);
-            if (nn > gr[k]) {
-                const float sc = gr[k] / nn;
+            const float gr = l.g + gnone, ratio = gr / nn, sc = nn > gr ? ratio : 1.0f;
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    a[c] *= sc;
-                    b[c] *= sc;
-                }
+            for (int c = 0; c < 3; c++) {
+                a[c] *= sc;
+                b[c] *= sc;
             }
         }
+        if constexpr (ph == 3) {
+            // the step of vtv_sr_ista_step_unstructured, and the primal (cuda_kernels.cu:504-532)
+            const int vo = yo < y1 ? vs : kOutside;
+            const Divisor cov(l.cov != 0.0f ? l.cov : 1.0f);
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            ps[c * NPP + i] = a[c];
-            ps[(3 + c) * NPP + i] = b[c];
+            for (int c = 0; c < 3; c++) {
+                float Gv = cov.of(acc[c]);
+                if constexpr (!GRAD) Gv = da.alpha > 0.0f ? da.alpha * (Gv * da.sigma2) : 0.0f;
+                Gv = fminf(1.0f, fmaxf(-1.0f, Gv));
+                const float F = fminf(1.0f, fmaxf(0.0f, fmaf(Gv, da.prox_factor, up[c])));
+                float rel = up[c];
+                if constexpr (PD) {
+                    // (left of the image U and the duals read 0)
+                    const float step = a[c] + b[c] - from_left(a[c]) - py1[c];
+                    const float un = fmaf(pa.tau, step, up[c]);
+                    const float v = vden.of(fmaf(pa.tau, F, pa.lam * un));
+                    rel = fmaf(pa.theta, v - up[c], up[c]);
+                    bPxo.store(a[c], c, yo, vo);
+                    bPyo.store(b[c], c, yo, vo);
+                    bUn.store(v, c, yo, vo);
+                }
+                if constexpr (EXTRA) {
+                    bUq.store(rel, c, yo, vo);
+                    bGo.store(F, c, yo, vo);
+                }
+            }
+            if constexpr (EXTRA) bNm.store(l.cov, 0, yo, vo);
         }
-    }
-    __syncthreads();
-    const int lx = tid % TW, ly = tid / TW;
-    const int x = tx0 + lx, y = ty0 + ly;
-    if (x >= W || y >= H) return;
-    const size_t o = (size_t)y * W + x;
-    const int pi = (ly + 1) * UW + lx + 1;
+        if constexpr (PD && ph >= 2) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-        const float *pxs = ps + c * NPP, *pys = ps + (3 + c) * NPP;
-        const float pxv = pxs[pi], pyv = pys[pi];
-        pxout[c * N + o] = pxv;
-        pyout[c * N + o] = pyv;
-        float step = pxv + pyv;
-        if (x > 0) step -= pxs[pi - 1];
-        if (y > 0) step -= pys[pi - UW];
-        const float un = up[c] + pa.tau * step;
-        const float v = (pa.tau * F[c] + pa.lam * un) / (pa.tau + pa.lam);
-        unew[c * N + o] = v;
-        if (uq_relax) uq_relax[c * N + o] = up[c] + pa.theta * (v - up[c]);
-        if (Gout) Gout[c * N + o] = F[c];
+            for (int c = 0; c < 3; c++) py1[c] = ph == 3 || yo >= 0 ? b[c] : 0.0f;
+        }
+#pragma unroll
+        for (int t = 0; t <= G; t++) {
+            s1[t] = l.f[t][2];
+            s2[t] = from_left(l.f[t][3]);
+            s3[t] = from_right(l.f[t][4]);
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    bm[t][c][d] = b0[t][c][d];
+                    b0[t][c][d] = bp[t][c][d];
+                }
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < 2; k++) fetch(ld[k], first + k);
+    constexpr int WARM = 2 * LAG;  // rows before the first output
+    static_for<WARM>([&](auto K) __attribute__((always_inline)) {
+        constexpr int i = decltype(K)::value;
+        row(K, std::integral_constant<int, (i == WARM - 1 ? 2 : i > D + 2 * G ? 1 : 0)>(), i);
+    });
+    // whole groups of kStripGroup rows, those past y1 without bytes: a branch between rows would cost the state's
+    // registers a move each.  A ring of two groups changes halves after each, so that its indices stay the same.
+    for (int j0 = 0; j0 < y1 - y0; j0 += kStripGroup) {
+        static_for<kStripGroup>([&](auto J) __attribute__((always_inline)) {
+            constexpr int j = decltype(J)::value;
+            row(std::integral_constant<int, WARM + j>(), std::integral_constant<int, 3>(), WARM + j0 + j);
+        });
+        if constexpr (RING == 2 * kStripGroup)
+#pragma unroll
+            for (int k = 0; k < kStripGroup; k++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const float t = u[k][c];
+                    u[k][c] = u[k + kStripGroup][c];
+                    u[k + kStripGroup][c] = t;
+                }
     }
-    if (norm_mask && (da.alpha > 0.0f || da.beta > 0.0f)) norm_mask[o] = cov;
 }
 
-template <int KS, bool GRAD>
-__global__ void __launch_bounds__(kStTW * kStTH) k_sr_step_st(int W, int H, int Wc, int Hc, int ntx, int ntiles,
-                                                               DataTermArgs da, PdArgs pa, const float *__restrict__ U,
-                                                               const float *__restrict__ ops, size_t NA,
-                                                               const float *__restrict__ coverage,
-                                                               const float *__restrict__ pxin,
-                                                               const float *__restrict__ pyin,
-                                                               const float *__restrict__ g, float *__restrict__ pxout,
-                                                               float *__restrict__ pyout, float *__restrict__ unew,
-                                                               float *__restrict__ uq_relax, float *__restrict__ Gout,
-                                                               float *__restrict__ norm_mask, const int *halt)
+template <int D, bool GRAD, bool PD, bool EXTRA, bool WIDE>
+__device__ __forceinline__ void sr_block(int b, StripGeom sg, int W, int H, int Wc, int Hc, size_t NA,
+                                         const DataTermArgs &da, const PdArgs &pa, const StepBufs &sb)
+{
+    const int strip = __builtin_amdgcn_readfirstlane(4 * b + (int)(threadIdx.x >> 6));
+    const int sy = strip / sg.nx, sx = strip - sy * sg.nx, y0 = sy * sg.rows;
+    if (y0 >= H) return;
+    sr_strip<D, GRAD, PD, EXTRA, WIDE>(sx * Strip<D, GRAD>::OW, y0, min(y0 + sg.rows, H), W, H, Wc, Hc, NA, da, pa, sb);
+}
+
+// One outer step for dsf >= 2 (PD), or its data term alone.  U is only read.
+// uq_relax and norm_mask are nullable: a run of fixed steps reads neither
+// between its steps (the next step starts from the new primal, and the mask
+// is the coverage again), so only its last step writes them.
+template <int KS, bool GRAD, bool PD, bool EXTRA, bool WIDE>
+__global__ void __launch_bounds__(256) k_sr_step_st(int W, int H, int Wc, int Hc, StripGeom sg, DataTermArgs da, PdArgs pa,
+                                                    size_t NA, StepBufs sb, const int *halt)
 {
     if (halt && *halt) return;  // a step enqueued behind a stopping rule that fired
-    sr_step_tile<KS, GRAD>(xcd_tile(blockIdx.x, ntiles), W, H, Wc, Hc, ntx, da, pa, U, ops, NA, coverage, pxin, pyin, g,
-                     pxout, pyout, unew, uq_relax, Gout, norm_mask);
+    sr_block<KS - 1, GRAD, PD, EXTRA, WIDE>(xcd_tile(blockIdx.x, sg.nblocks), sg, W, H, Wc, Hc, NA, da, pa, sb);
 }
 
-// Step s of every IBR_color solve of a batch in one launch: block b runs tile
-// xcd_tile(j, ntiles) of solve k, (k, j) = work[b], exactly as block j of
-// that solve's own k_sr_step_st launch (the same tile, the same arithmetic),
-// on the buffers of step parity s & 1; a solve with fewer steps returns.
-// Only a solve's last step writes Uq and the norm mask, as in its own run.
+// Step s of every IBR_color solve of a batch in one launch: block b runs block
+// xcd_tile(j, nblocks) of solve k, (k, j) = work[b], as in that solve's own
+// k_sr_step_st launch (the same arithmetic), on the buffers of step parity
+// s & 1; a solve with fewer steps returns.  Only a solve's last step writes Uq
+// and the norm mask, as in its own run.
 template <int KS, bool GRAD>
-__global__ void __launch_bounds__(kStTW * kStTH) k_sr_step_st_batch(const SrBatchItem *__restrict__ items,
-                                                                     const int2 *__restrict__ work, int s)
+__global__ void __launch_bounds__(256) k_sr_step_st_batch(const SrBatchItem *__restrict__ items,
+                                                          const int2 *__restrict__ work, int s)
 {
     const int2 wk = work[blockIdx.x];
     const SrBatchItem &it = items[wk.x];
@@ -724,9 +641,13 @@ __global__ void __launch_bounds__(kStTW * kStTH) k_sr_step_st_batch(const SrBatc
     PdArgs pa = it.pa;
     pa.theta = it.theta[s];
     const bool last = s == it.steps - 1;
-    sr_step_tile<KS, GRAD>(xcd_tile(wk.y, it.ntiles), it.W, it.H, it.Wc, it.Hc, it.ntx, it.da, pa, it.U[p], it.ops, it.NA,
-                     it.coverage, it.PX[p], it.PY[p], it.g, it.PX[p ^ 1], it.PY[p ^ 1], it.U[p ^ 1],
-                     last ? it.uq : nullptr, nullptr, last ? it.norm_mask : nullptr);
+    const StepBufs sb{it.U[p],         it.ops,       it.coverage, it.PX[p], it.PY[p], it.g, it.PX[p ^ 1], it.PY[p ^ 1],
+                      it.U[p ^ 1], last ? it.uq : nullptr, nullptr,     last ? it.norm_mask : nullptr};
+    const StripGeom sg = it.sg;
+    if (last)
+        sr_block<KS - 1, GRAD, true, true, false>(xcd_tile(wk.y, sg.nblocks), sg, it.W, it.H, it.Wc, it.Hc, it.NA, it.da, pa, sb);
+    else
+        sr_block<KS - 1, GRAD, true, false, false>(xcd_tile(wk.y, sg.nblocks), sg, it.W, it.H, it.Wc, it.Hc, it.NA, it.da, pa, sb);
 }
 
 // theta over-relaxation (vtv_rof.cu:28-45): uq <- u + theta (uq - u); u <- uq_old
@@ -1024,6 +945,9 @@ lfrv_status ensure_sr_ops(lfrv_ctx *ctx)
     return LFRV_OK;
 }
 
+// Whether the step's planes outgrow one buffer descriptor (the five planes of a coupling set are the largest).
+bool sr_wide(int Wc, int Hc) { return 20 * (size_t)Wc * Hc >= kNarrowBytes; }
+
 // One FISTA step on the stream; with `halt` every launch of the step is a
 // no-op once a stopping rule has fired on the device.  A step that is not the
 // last of a fixed run (last = false) leaves Uq and the norm mask to the run's
@@ -1062,8 +986,19 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
         const size_t NA = (size_t)Wc * Hc;
         st = ensure_sr_ops(ctx);
         if (st != LFRV_OK) return st;
-        const int ntx = (ctx->W + kStTW - 1) / kStTW, ntiles = ntx * ((ctx->H + kStTH - 1) / kStTH);
+        const StripSize size{ctx->W, ctx->H};
+        const bool grad = da.beta > 0.0f;
+        const StripGeom sg = sr_strips(ctx->ks, grad, size, sr_strip_rows(ctx->ks, grad, &size, 1));
         const KernelEvents ev = kernel_events(ctx, 3);  // stamped by the dispatch itself
+#define STEP2(K, GR, PD, EX, WI) hipExtLaunchKernelGGL(k_sr_step_st<K, GR, PD, EX, WI>, dim3(sg.nblocks), dim3(256), 0, ctx->stream, ev.a, ev.b, 0, ctx->W, ctx->H, Wc, Hc, sg, da, pa, NA, sb, halt)
+#define STEP1(K, GR, PD, EX) do { if (sr_wide(Wc, Hc)) STEP2(K, GR, PD, EX, true); else STEP2(K, GR, PD, EX, false); } while (0)
+#define STEP(PD, EX)                                                              \
+    do {                                                                          \
+        if (ctx->ks == 3) { if (grad) STEP1(3, true, PD, EX); else STEP1(3, false, PD, EX); }      \
+        else if (ctx->ks == 4) { if (grad) STEP1(4, true, PD, EX); else STEP1(4, false, PD, EX); } \
+        else if (ctx->ks == 5) { if (grad) STEP1(5, true, PD, EX); else STEP1(5, false, PD, EX); } \
+        else return fail(ctx, LFRV_E_ARG, "dsf out of range");                    \
+    } while (0)
         if (inner > 0) {
             // the data term and the first primal-dual iteration in one pass: U is
             // read, the new primal goes to U2 (with one inner iteration the
@@ -1071,19 +1006,11 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
             PdArgs pa = pd_args(ctx);
             pa.theta = theta;
             const float *gw = ctx->has_reg_g ? ctx->reg_g : nullptr;
-            float *uq_relax = (inner == 1 && last) ? ctx->Uq : nullptr;
-            float *gout = inner > 1 ? ctx->G : nullptr;
-            float *nmask = (inner > 1 || last) ? ctx->norm_mask : nullptr;
-#define ST1(K, GR) hipExtLaunchKernelGGL(k_sr_step_st<K, GR>, dim3(ntiles), dim3(kStTW * kStTH), 0, ctx->stream, ev.a, ev.b, 0, ctx->W, ctx->H, Wc, Hc, ntx, ntiles, da, pa, (const float *)ctx->U, (const float *)ctx->sr_ops, NA, (const float *)ctx->coverage, (const float *)ctx->PX, (const float *)ctx->PY, gw, ctx->P2X, ctx->P2Y, ctx->U2, uq_relax, gout, nmask, halt)
-#define ST(K) do { if (da.beta > 0.0f) ST1(K, true); else ST1(K, false); } while (0)
-            switch (ctx->ks) {
-            case 3: ST(3); break;
-            case 4: ST(4); break;
-            case 5: ST(5); break;
-            default: return fail(ctx, LFRV_E_ARG, "dsf out of range");
-            }
-#undef ST
-#undef ST1
+            const StepBufs sb{ctx->U,    ctx->sr_ops, ctx->coverage, ctx->PX, ctx->PY, gw, ctx->P2X, ctx->P2Y, ctx->U2,
+                              (inner == 1 && last) ? ctx->Uq : nullptr, inner > 1 ? ctx->G : nullptr,
+                              (inner > 1 || last) ? ctx->norm_mask : nullptr};
+            if (sb.uq_relax || sb.gout || sb.norm_mask) STEP(true, true);
+            else STEP(true, false);
             record_kernel_events(ctx, 3, ev);
             LFRV_LAUNCH(ctx, "data term + primal-dual step");
             std::swap(ctx->PX, ctx->P2X);
@@ -1094,20 +1021,17 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
                 std::swap(ctx->Uq, ctx->U2);  // the remaining iterations start from Uq
             pd_done = true;
         } else {
-#define DT1(K, GR) hipExtLaunchKernelGGL(k_sr_dataterm_st<K, GR>, dim3(ntiles), dim3(kStTW * kStTH), 0, ctx->stream, ev.a, ev.b, 0, ctx->W, ctx->H, Wc, Hc, ntx, ntiles, da, (const float *)ctx->U, (const float *)ctx->sr_ops, NA, (const float *)ctx->coverage, ctx->G, ctx->Uq, ctx->norm_mask, halt)
-#define DT(K) do { if (da.beta > 0.0f) DT1(K, true); else DT1(K, false); } while (0)
-            switch (ctx->ks) {
-            case 3: DT(3); break;
-            case 4: DT(4); break;
-            case 5: DT(5); break;
-            default: return fail(ctx, LFRV_E_ARG, "dsf out of range");
-            }
-#undef DT
-#undef DT1
+            const PdArgs pa{};
+            const StepBufs sb{ctx->U,  ctx->sr_ops, ctx->coverage, nullptr, nullptr, nullptr,       nullptr, nullptr,
+                              nullptr, ctx->Uq,     ctx->G,        ctx->norm_mask};
+            STEP(false, true);
             record_kernel_events(ctx, 3, ev);
             LFRV_LAUNCH(ctx, "data term");
         }
     }
+#undef STEP
+#undef STEP1
+#undef STEP2
     if (pd_done) {
         if (inner > 1) {
             st = run_pd_steps(ctx, inner - 1, ctx->G, true, theta, halt);
@@ -1156,6 +1080,38 @@ EnergyCoef energy_coef(const lfrv_ctx *ctx)
 
 }  // namespace
 
+// Rows per strip for targets stepped in one launch.  A wave costs its rows and
+// the 2 LAG before the first output, and 2 waves per SIMD, 2048 in all, run at
+// once: the height (whole groups of rows) with the least rows per slot.  2048^2,
+// dsf 4 (38 strips across): 42 rows, 1862 waves, 141 us per step; 36 rows, 2166
+// waves, 173 us; 256^2, dsf 2: 3 rows 6.6 us, 12 rows 12.6 us.
+int sr_strip_rows(int ks, bool grad, const StripSize *sizes, int n)
+{
+    const int lag = ks - 1 + (grad ? 1 : 0);
+    int best = kStripGroup;
+    long best_cost = LONG_MAX;
+    for (int rows = kStripGroup; rows <= 96; rows += kStripGroup) {
+        long waves = 0;
+        for (int i = 0; i < n; i++) waves += 4L * sr_strips(ks, grad, sizes[i], rows).nblocks;
+        const long cost = (waves + 2047) / 2048 * (rows + 2 * lag);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = rows;
+        }
+    }
+    return best;
+}
+
+StripGeom sr_strips(int ks, bool grad, StripSize size, int rows)
+{
+    const int lag = ks - 1 + (grad ? 1 : 0), ow = 64 - 2 * lag;
+    StripGeom sg;
+    sg.nx = (size.W + ow - 1) / ow;
+    sg.rows = rows;
+    sg.nblocks = (sg.nx * ((size.H + rows - 1) / rows) + 3) / 4;
+    return sg;
+}
+
 lfrv_status run_fista(lfrv_ctx *ctx, bool last)
 {
     return enqueue_fista(ctx, nullptr, last);
@@ -1163,7 +1119,8 @@ lfrv_status run_fista(lfrv_ctx *ctx, bool last)
 
 bool sr_batchable(const lfrv_ctx *ctx)
 {
-    return ctx->p.mode == LFRV_MODE_COLOR_SR && ctx->ks >= 3 && ctx->ks <= 5 && ctx->p.inner_iterations == 1;
+    return ctx->p.mode == LFRV_MODE_COLOR_SR && ctx->ks >= 3 && ctx->ks <= 5 && ctx->p.inner_iterations == 1 &&
+           !sr_wide(ctx->W + ctx->ks - 1, ctx->H + ctx->ks - 1);
 }
 
 lfrv_status sr_batch_begin(lfrv_ctx *ctx, int steps, SrBatchItem *it, float *theta_host)
@@ -1178,8 +1135,6 @@ lfrv_status sr_batch_begin(lfrv_ctx *ctx, int steps, SrBatchItem *it, float *the
     it->H = ctx->H;
     it->Wc = Wc;
     it->Hc = Hc;
-    it->ntx = (ctx->W + kStTW - 1) / kStTW;
-    it->ntiles = it->ntx * ((ctx->H + kStTH - 1) / kStTH);
     it->steps = steps;
     it->da = data_term_args(ctx);
     it->pa = pd_args(ctx);
@@ -1225,7 +1180,7 @@ void sr_batch_end(lfrv_ctx *ctx, int steps)
 hipError_t launch_sr_batch_step(int ks, bool grad, const SrBatchItem *items, const int2 *work, int nblocks, int s,
                                 hipStream_t stream)
 {
-#define SB(K, G) k_sr_step_st_batch<K, G><<<nblocks, kStTW * kStTH, 0, stream>>>(items, work, s)
+#define SB(K, G) k_sr_step_st_batch<K, G><<<nblocks, 256, 0, stream>>>(items, work, s)
     switch (ks * 2 + (grad ? 1 : 0)) {
     case 6: SB(3, false); break;
     case 7: SB(3, true); break;

@@ -523,11 +523,22 @@ __host__ __device__ __forceinline__ float dt_gradient_weight(const DataTermArgs 
 struct PdArgs {
     float tau, lam, sigma, theta;
 };
+// How a target is cut into the strips of an IBR_color step (k_sr.hip): nx
+// across, `rows` rows each, four per block.
+struct StripSize {
+    int W, H;
+};
+struct StripGeom {
+    int nx, rows, nblocks;
+};
+int sr_strip_rows(int ks, bool grad, const StripSize *sizes, int n);
+StripGeom sr_strips(int ks, bool grad, StripSize size, int rows);
 // One solve's FISTA steps inside a batched launch: step s reads U[s & 1],
 // PX[s & 1], PY[s & 1] and writes the other parity (the pointer swaps of
 // the solve's own steps), with theta[s] of its FISTA sequence.
 struct SrBatchItem {
-    int W, H, Wc, Hc, ntx, ntiles, steps;
+    int W, H, Wc, Hc, steps;
+    StripGeom sg;
     DataTermArgs da;
     PdArgs pa;
     const float *theta;  // device, `steps` entries
@@ -541,7 +552,7 @@ struct SrBatchItem {
 // primal-dual iteration per step).
 bool sr_batchable(const lfrv_ctx *ctx);
 // Readies `steps` steps of ctx for a batched launch on ctx's stream (the
-// assembled operator, the entry weights) and fills `it` (all but `theta`)
+// assembled operator, the entry weights) and fills `it` (all but `theta` and `sg`)
 // and theta_host[0 .. steps).
 lfrv_status sr_batch_begin(lfrv_ctx *ctx, int steps, SrBatchItem *it, float *theta_host);
 // After the batched steps: the context's buffers and FISTA state as after

@@ -167,3 +167,16 @@ def test_sr_iterate_equals_single_steps(dsf, inner, beta):
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     assert np.abs(out[0][3].ravel() - out[0][0].ravel()).max() > 0  # the over-relaxed solution is not the solution
+
+
+@pytest.mark.parametrize("w,h,dsf,beta", [(29, 7, 2, 0.3),   # one strip to its last column, rows short of a group
+                                          (30, 8, 2, 0.0),
+                                          (31, 3, 2, 0.0),   # a second strip of two columns
+                                          (19, 16, 3, 0.3),  # a second strip of one column
+                                          (14, 5, 4, 0.3), (70, 4, 4, 0.0)])
+def test_sr_steps_at_strip_edges(w, h, dsf, beta):
+    """The marching step where its 64-column strips and 3-row groups end, against the oracle."""
+    d = lfrv.synth_desc(1, 3)
+    d.grid, d.w, d.h, d.dsf, d.render_scale = 3, w, h, dsf, dsf
+    d.focal, d.baseline = float(w), 0.7 * 4.0 / (w * dsf)
+    _steps_match_oracle(lfrv.synth(d), beta, 0, 1, metas=1, steps=3)
