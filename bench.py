@@ -449,9 +449,9 @@ def bench_color_sr(args, workload):
         NA = (scene["W"] + ks - 1) * (scene["H"] + ks - 1)
         dt_kernel = f"k_sr_step_st<{ks}, {'true' if beta > 0 else 'false'}>"  # <dsf + 1, gradient term>
         dt_bytes = 4 * NA * (8 + (5 if beta > 0 else 0)) + 80 * N
-    # fused PD step: Uq, px, py, g, F read; px, py, new primal written (88 B
-    # per pixel), with the outer step's over-relaxation fused in: U read, and
-    # U and the over-relaxed Uq written (+24 B)
+    # a pass of primal-dual iterations (up to four): Uq, px, py, g, F read; px, py,
+    # new primal written (88 B per pixel), with the outer step's over-relaxation
+    # fused in: U read, and U and the over-relaxed Uq written (+24 B)
     pd_bytes = 112 * N
     dt_s = dt_ms / max(dt_n, 1) / 1e3
     pd_s = pd_ms / max(pd_n, 1) / 1e3
@@ -460,9 +460,9 @@ def bench_color_sr(args, workload):
                               achieved_gbs=round(dt_bytes / dt_s / 1e9, 1), launches=dt_n),
     }
     if pd_n:  # separate primal-dual launches (dsf = 1; dsf >= 2 runs them inside the step pass)
-        kern["k_pd_step"] = dict(bytes_per_launch=pd_bytes, avg_launch_us=round(pd_s * 1e6, 2),
+        kern["k_pd_steps"] = dict(bytes_per_launch=pd_bytes, avg_launch_us=round(pd_s * 1e6, 2),
                                  achieved_gbs=round(pd_bytes / pd_s / 1e9, 1), launches=pd_n)
-    dom = dt_kernel if dt_ms >= pd_ms else "k_pd_step"
+    dom = dt_kernel if dt_ms >= pd_ms else "k_pd_steps"
     k = kern[dom]
     if nmeta:
         last = irls[-1]

@@ -235,14 +235,14 @@ extern "C" lfrv_status lfrv_batch_run(lfrv_batch *b, lfrv_batch_result *res)
                 if (b->entries[sr_index[k]].ctx->ks == ks && (sr_items[k].da.beta > 0.0f) == grad)
                     sizes.push_back({sr_items[k].W, sr_items[k].H});
             if (sizes.empty()) continue;
-            const int rows = sr_strip_rows(ks, grad, sizes.data(), (int)sizes.size());
+            const int rows = strip_rows(sr_lag(ks, grad), sizes.data(), (int)sizes.size());
             for (int k = 0; k < ns; k++) {
                 if (b->entries[sr_index[k]].ctx->ks != ks || (sr_items[k].da.beta > 0.0f) != grad) continue;
                 const int idx = (int)items_sorted.size();
                 items_sorted.push_back(sr_items[k]);
                 items_sorted.back().theta = nullptr;  // set below, once the device array exists
                 items_sorted.back().NA = sr_items[k].NA;
-                const StripGeom sg = sr_strips(ks, grad, {sr_items[k].W, sr_items[k].H}, rows);
+                const StripGeom sg = strips(sr_lag(ks, grad), {sr_items[k].W, sr_items[k].H}, rows);
                 items_sorted.back().sg = sg;
                 for (int j = 0; j < sg.nblocks; j++) work.push_back(make_int2(idx, j));
                 max_steps = std::max(max_steps, sr_items[k].steps);

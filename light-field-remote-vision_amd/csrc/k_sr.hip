@@ -16,10 +16,6 @@
 
 namespace lfrv {
 
-// k_stencil.hip; with `overrelax` the last step also does the over-relaxation
-lfrv_status run_pd_steps(lfrv_ctx *ctx, int iters, const float *F, bool overrelax = false, float theta = 0.0f,
-                         const int *halt = nullptr);
-
 namespace {
 
 
@@ -650,6 +646,147 @@ __global__ void __launch_bounds__(256) k_sr_step_st_batch(const SrBatchItem *__r
         sr_block<KS - 1, GRAD, true, false, false>(xcd_tile(wk.y, sg.nblocks), sg, it.W, it.H, it.Wc, it.Hc, it.NA, it.da, pa, sb);
 }
 
+// ---- further primal-dual iterations -------------------------------------------
+//
+// Inner iterations of vtv_sr_ista_step_unstructured (optimization.cu:1817-1828):
+//   dual:   p_c <- p_c + sigma grad+ Uq_c           (vtv_rof.cu:118-147)
+//   proj:   joint TV_F projection onto |p| <= g      (vtv_rof.cu:280-321; radius 1 without g, :237-275)
+//   primal: Uq_c <- (tau F_c + lam (Uq_c + tau div- p_c)) / (tau + lam)   (cuda_kernels.cu:504-532)
+// K of them in one pass of the marching strips: iteration j takes row y of the
+// iteration before it as soon as that row and the next are there, one row and
+// one column behind, so U, the duals, F and g cross memory once per K
+// iterations.  One pass of 431 x 322: 3 iterations in 12 us, where a pass per
+// iteration (64 x 4 tiles) took 8.2 us each.
+// With u_final (the last iterations of an outer step) the over-relaxation of
+// the outer step is fused in (vtv_rof.cu:28-45): u_final <- the new primal,
+// uout <- u_final_old + theta (new primal - u_final_old).
+struct PdBufs {
+    const float *uin, *px, *py, *F, *g;
+    float *uout, *pxout, *pyout, *u_final;
+};
+
+template <int K, bool WIDE>
+__device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, const PdArgs &pa, const PdBufs &pb)
+{
+    const size_t N = (size_t)W * H;
+    const int lane = threadIdx.x & 63, x = x0 - K + lane;
+    const bool xin = x >= 0 && x < W;
+    const int vx = xin ? 4 * x : kOutside, vs = lane >= K && lane < 64 - K ? vx : kOutside;
+    const Divisor vden(pa.tau + pa.lam);
+    const float sgx = xin && x < W - 1 ? pa.sigma : 0.0f;
+    const float gnone = pb.g ? 0.0f : 1.0f;
+    const Planes<WIDE> bU(pb.uin, 3, N, W), bPx(pb.px, 3, N, W), bPy(pb.py, 3, N, W), bF(pb.F, 3, N, W), bG(pb.g, 1, N, W),
+        bUo(pb.uout, 3, N, W), bPxo(pb.pxout, 3, N, W), bPyo(pb.pyout, 3, N, W), bUf(pb.u_final, 3, N, W);
+    const int first = y0 - K, yend = y1 + K;  // rows of U
+    struct Loads {
+        float u[3], p[6], F[3], g, uf[3];
+    } ld[3];
+    auto fetch = [&](Loads &l, int yn) __attribute__((always_inline)) {
+        const int yp = yn - 1, yo = yn - K;
+        const int vu = yn >= 0 && yn < min(H, yend) ? vx : kOutside;
+        const int vp = yp >= 0 && yp < H && yn < yend ? vx : kOutside;
+        const int vf = yo >= y0 && yo < y1 ? vs : kOutside;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            l.u[c] = bU.load(c, yn, vu);
+            l.p[c] = bPx.load(c, yp, vp);
+            l.p[3 + c] = bPy.load(c, yp, vp);
+            l.F[c] = bF.load(c, yp, vp);
+            l.uf[c] = bUf.load(c, yo, vf);
+        }
+        l.g = bG.load(0, yp, vp);
+    };
+    // iteration j: U's last row, and for j > 0 the duals, F and g of that row, as iteration j - 1 left them a turn
+    // ago; the y part of its own duals a row up
+    float u[K][3], p[K][6], F[K][3], g[K], py[K][3];
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        g[j] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 3; c++) u[j][c] = p[j][c] = p[j][3 + c] = py[j][c] = F[j][c] = 0.0f;
+    }
+    auto row = [&](auto B, int yn) __attribute__((always_inline)) {
+        constexpr int k = decltype(B)::value;
+        const Loads &l = ld[k % 3];
+        fetch(ld[(k + 2) % 3], yn + 2);
+        float un[3], cp[6], cF[3], cg = l.g + gnone;  // to iteration j: its new row of U; duals, F, g of the row above
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            un[c] = l.u[c];
+            cF[c] = l.F[c];
+            cp[c] = l.p[c];
+            cp[3 + c] = l.p[3 + c];
+        }
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            const int y = yn - 1 - j;  // the row this iteration completes
+            const bool yin = y >= 0 && y < H;
+            const float sgy = y < H - 1 ? pa.sigma : 0.0f;
+            if (j > 0) {
+                // what came from iteration j - 1 is for the next turn
+                const float tg = g[j];
+                g[j] = cg;
+                cg = tg;
+#pragma unroll
+                for (int c = 0; c < 6; c++) {
+                    const float t = p[j][c];
+                    p[j][c] = cp[c];
+                    cp[c] = t;
+                }
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const float t = F[j][c];
+                    F[j][c] = cF[c];
+                    cF[c] = t;
+                }
+            }
+            float nn = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                cp[c] = fmaf(sgx, from_right(u[j][c]) - u[j][c], cp[c]);
+                cp[3 + c] = fmaf(sgy, un[c] - u[j][c], cp[3 + c]);
+                nn += fmaf(cp[c], cp[c], cp[3 + c] * cp[3 + c]);
+            }
+            nn = sqrtf(nn);
+            const float ratio = cg / nn, in = nn > cg ? ratio : 1.0f;
+            const float sc = yin ? +in : 0.0f;  // (no duals outside the image; left and right of it all they read is 0)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                cp[c] *= sc;
+                cp[3 + c] *= sc;
+                const float step = cp[c] + cp[3 + c] - from_left(cp[c]) - py[j][c];
+                const float v = vden.of(fmaf(pa.tau, cF[c], pa.lam * fmaf(pa.tau, step, u[j][c])));
+                py[j][c] = cp[3 + c];
+                u[j][c] = un[c];
+                un[c] = xin && yin ? +v : 0.0f;
+            }
+        }
+        const int yo = yn - K, vo = yo >= y0 && yo < y1 ? vs : kOutside;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            bPxo.store(cp[c], c, yo, vo);
+            bPyo.store(cp[3 + c], c, yo, vo);
+            const float rel = fmaf(pa.theta, un[c] - l.uf[c], l.uf[c]);
+            bUo.store(pb.u_final ? rel : un[c], c, yo, vo);
+            bUf.store(un[c], c, yo, vo);
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < 2; k++) fetch(ld[k], first + k);
+    for (int yn = first; yn < yend; yn += kStripGroup)
+        static_for<kStripGroup>([&](auto B) __attribute__((always_inline)) { row(B, yn + decltype(B)::value); });
+}
+
+template <int K, bool WIDE>
+__global__ void __launch_bounds__(256) k_pd_steps(int W, int H, StripGeom sg, PdArgs pa, PdBufs pb, const int *halt)
+{
+    if (halt && *halt) return;  // a step enqueued behind a stopping rule that fired
+    const int strip = __builtin_amdgcn_readfirstlane(4 * xcd_tile(blockIdx.x, sg.nblocks) + (int)(threadIdx.x >> 6));
+    const int sy = strip / sg.nx, sx = strip - sy * sg.nx, y0 = sy * sg.rows;
+    if (y0 >= H) return;
+    pd_strip<K, WIDE>(sx * (64 - 2 * K), y0, min(y0 + sg.rows, H), W, H, pa, pb);
+}
+
 // theta over-relaxation (vtv_rof.cu:28-45): uq <- u + theta (uq - u); u <- uq_old
 __global__ void k_overrelax(size_t n3, float theta, float *__restrict__ uq, float *__restrict__ u, const int *halt)
 {
@@ -948,6 +1085,78 @@ lfrv_status ensure_sr_ops(lfrv_ctx *ctx)
 // Whether the step's planes outgrow one buffer descriptor (the five planes of a coupling set are the largest).
 bool sr_wide(int Wc, int Hc) { return 20 * (size_t)Wc * Hc >= kNarrowBytes; }
 
+}  // namespace
+
+int sr_lag(int ks, bool grad) { return ks - 1 + (grad ? 1 : 0); }
+
+// Rows per strip for targets stepped in one launch.  A wave costs its rows and
+// the 2 LAG before the first output, and 2 waves per SIMD, 2048 in all, run at
+// once: the height (whole groups of rows) with the least rows per slot.  2048^2,
+// dsf 4 (38 strips across): 42 rows, 1862 waves, 141 us per step; 36 rows, 2166
+// waves, 173 us; 256^2, dsf 2: 3 rows 6.6 us, 12 rows 12.6 us.
+int strip_rows(int lag, const StripSize *sizes, int n)
+{
+    int best = kStripGroup;
+    long best_cost = LONG_MAX;
+    for (int rows = kStripGroup; rows <= 96; rows += kStripGroup) {
+        long waves = 0;
+        for (int i = 0; i < n; i++) waves += 4L * strips(lag, sizes[i], rows).nblocks;
+        const long cost = (waves + 2047) / 2048 * (rows + 2 * lag);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = rows;
+        }
+    }
+    return best;
+}
+
+StripGeom strips(int lag, StripSize size, int rows)
+{
+    const int ow = 64 - 2 * lag;
+    StripGeom sg;
+    sg.nx = (size.W + ow - 1) / ow;
+    sg.rows = rows;
+    sg.nblocks = (sg.nx * ((size.H + rows - 1) / rows) + 3) / 4;
+    return sg;
+}
+
+namespace {
+
+// `iters` primal-dual iterations on F, up to four per pass, as even as they
+// come; with `overrelax` the last also does the over-relaxation.
+lfrv_status run_pd_steps(lfrv_ctx *ctx, int iters, const float *F, bool overrelax, float theta, const int *halt)
+{
+    const StripSize size{ctx->W, ctx->H};
+    PdArgs pa = pd_args(ctx);
+    pa.theta = theta;
+    const bool wide = 12 * (size_t)ctx->W * ctx->H >= kNarrowBytes;
+    int left = iters;
+    for (int passes = (iters + 3) / 4; passes > 0; passes--) {
+        const int k = (left + passes - 1) / passes;
+        left -= k;
+        const StripGeom sg = strips(k, size, strip_rows(k, &size, 1));
+        const PdBufs pb{ctx->Uq, ctx->PX,  ctx->PY,  F, ctx->has_reg_g ? ctx->reg_g : nullptr,
+                        ctx->U2, ctx->P2X, ctx->P2Y, overrelax && left == 0 ? ctx->U : nullptr};
+        const KernelEvents ev = kernel_events(ctx, 2);  // stamped by the dispatch itself
+#define PD1(K, WI) hipExtLaunchKernelGGL(k_pd_steps<K, WI>, dim3(sg.nblocks), dim3(256), 0, ctx->stream, ev.a, ev.b, 0, ctx->W, ctx->H, sg, pa, pb, halt)
+#define PD(K) case K: if (wide) PD1(K, true); else PD1(K, false); break
+        switch (k) {
+            PD(1);
+            PD(2);
+            PD(3);
+            PD(4);
+        }
+#undef PD
+#undef PD1
+        record_kernel_events(ctx, 2, ev);
+        std::swap(ctx->Uq, ctx->U2);
+        std::swap(ctx->PX, ctx->P2X);
+        std::swap(ctx->PY, ctx->P2Y);
+    }
+    LFRV_LAUNCH(ctx, "pd step");
+    return LFRV_OK;
+}
+
 // One FISTA step on the stream; with `halt` every launch of the step is a
 // no-op once a stopping rule has fired on the device.  A step that is not the
 // last of a fixed run (last = false) leaves Uq and the norm mask to the run's
@@ -988,7 +1197,7 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
         if (st != LFRV_OK) return st;
         const StripSize size{ctx->W, ctx->H};
         const bool grad = da.beta > 0.0f;
-        const StripGeom sg = sr_strips(ctx->ks, grad, size, sr_strip_rows(ctx->ks, grad, &size, 1));
+        const StripGeom sg = strips(sr_lag(ctx->ks, grad), size, strip_rows(sr_lag(ctx->ks, grad), &size, 1));
         const KernelEvents ev = kernel_events(ctx, 3);  // stamped by the dispatch itself
 #define STEP2(K, GR, PD, EX, WI) hipExtLaunchKernelGGL(k_sr_step_st<K, GR, PD, EX, WI>, dim3(sg.nblocks), dim3(256), 0, ctx->stream, ev.a, ev.b, 0, ctx->W, ctx->H, Wc, Hc, sg, da, pa, NA, sb, halt)
 #define STEP1(K, GR, PD, EX) do { if (sr_wide(Wc, Hc)) STEP2(K, GR, PD, EX, true); else STEP2(K, GR, PD, EX, false); } while (0)
@@ -1079,38 +1288,6 @@ EnergyCoef energy_coef(const lfrv_ctx *ctx)
 }
 
 }  // namespace
-
-// Rows per strip for targets stepped in one launch.  A wave costs its rows and
-// the 2 LAG before the first output, and 2 waves per SIMD, 2048 in all, run at
-// once: the height (whole groups of rows) with the least rows per slot.  2048^2,
-// dsf 4 (38 strips across): 42 rows, 1862 waves, 141 us per step; 36 rows, 2166
-// waves, 173 us; 256^2, dsf 2: 3 rows 6.6 us, 12 rows 12.6 us.
-int sr_strip_rows(int ks, bool grad, const StripSize *sizes, int n)
-{
-    const int lag = ks - 1 + (grad ? 1 : 0);
-    int best = kStripGroup;
-    long best_cost = LONG_MAX;
-    for (int rows = kStripGroup; rows <= 96; rows += kStripGroup) {
-        long waves = 0;
-        for (int i = 0; i < n; i++) waves += 4L * sr_strips(ks, grad, sizes[i], rows).nblocks;
-        const long cost = (waves + 2047) / 2048 * (rows + 2 * lag);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = rows;
-        }
-    }
-    return best;
-}
-
-StripGeom sr_strips(int ks, bool grad, StripSize size, int rows)
-{
-    const int lag = ks - 1 + (grad ? 1 : 0), ow = 64 - 2 * lag;
-    StripGeom sg;
-    sg.nx = (size.W + ow - 1) / ow;
-    sg.rows = rows;
-    sg.nblocks = (sg.nx * ((size.H + rows - 1) / rows) + 3) / 4;
-    return sg;
-}
 
 lfrv_status run_fista(lfrv_ctx *ctx, bool last)
 {

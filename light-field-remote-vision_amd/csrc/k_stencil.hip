@@ -274,103 +274,6 @@ __global__ void k_pp_finish(size_t N, const float *__restrict__ filled, float *_
     if (k < 3 * N) U[k] = filled[k] - U[k];
 }
 
-// ---- fused primal-dual ROF step --------------------------------------------
-// One inner iteration of vtv_sr_ista_step_unstructured (optimization.cu:1817-1828):
-//   dual:   p_c <- p_c + sigma grad+ Uq_c           (vtv_rof.cu:118-147)
-//   proj:   joint TV_F projection onto |p| <= g      (vtv_rof.cu:280-321; radius 1 without g, :237-275)
-//   primal: Uq_c <- (tau F_c + lam (Uq_c + tau div- p_c)) / (tau + lam)   (cuda_kernels.cu:504-532)
-// computed per tile: p_new on the tile plus its left/top halo, then Uq.
-// Inputs and outputs are separate buffers (neighbouring tiles read halos).
-constexpr int PD_TW = 64, PD_TH = 4;
-
-// With u_final (the last inner step of an outer step) the over-relaxation of
-// the outer step is fused in (vtv_rof.cu:28-45): u_final <- the new primal,
-// uout <- u_final_old + theta (new primal - u_final_old).
-// A non-null `halt` that holds nonzero makes the launch a no-op (a step
-// enqueued ahead of a stopping rule that has fired).
-__global__ void __launch_bounds__(256) k_pd_step(int W, int H, float tau, float lam, float sigma,
-                                                 const float *__restrict__ uin, float *__restrict__ uout,
-                                                 const float *__restrict__ pxin, const float *__restrict__ pyin,
-                                                 float *__restrict__ pxout, float *__restrict__ pyout,
-                                                 const float *__restrict__ F, const float *__restrict__ g,
-                                                 float *__restrict__ u_final, float theta, const int *halt)
-{
-    if (halt && *halt) return;
-    constexpr int UW = PD_TW + 2, UH = PD_TH + 2;  // Uq region [x0-1, x0+TW] x [y0-1, y0+TH]
-    constexpr int PW = PD_TW + 1, PH = PD_TH + 1;  // p region  [x0-1, x0+TW-1] x [y0-1, y0+TH-1]
-    __shared__ float us[3][UH][UW];
-    __shared__ float ps[6][PH][PW];
-    const size_t N = (size_t)W * H;
-    const int x0 = blockIdx.x * PD_TW, y0 = blockIdx.y * PD_TH;
-    for (int i = threadIdx.x; i < UW * UH; i += blockDim.x) {
-        const int lx = i % UW, ly = i / UW;
-        const int x = x0 - 1 + lx, y = y0 - 1 + ly;
-        const bool in = x >= 0 && x < W && y >= 0 && y < H;
-        const size_t o = in ? (size_t)y * W + x : 0;
-        for (int c = 0; c < 3; c++) us[c][ly][lx] = in ? uin[c * N + o] : 0.0f;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < PW * PH; i += blockDim.x) {
-        const int lx = i % PW, ly = i / PW;
-        const int x = x0 - 1 + lx, y = y0 - 1 + ly;
-        float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
-        if (x >= 0 && x < W && y >= 0 && y < H) {
-            const size_t o = (size_t)y * W + x;
-            float nn = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                // the p region and the Uq region share the origin (x0-1, y0-1)
-                const float uc = us[c][ly][lx];
-                const float gx = (x < W - 1) ? us[c][ly][lx + 1] - uc : 0.0f;
-                const float gy = (y < H - 1) ? us[c][ly + 1][lx] - uc : 0.0f;
-                a[c] = pxin[c * N + o] + sigma * gx;
-                b[c] = pyin[c * N + o] + sigma * gy;
-                nn += a[c] * a[c] + b[c] * b[c];
-            }
-            nn = sqrtf(nn);
-            const float rad = g ? g[o] : 1.0f;
-            if (nn > rad) {
-                const float s = rad / nn;
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    a[c] *= s;
-                    b[c] *= s;
-                }
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            ps[c][ly][lx] = a[c];
-            ps[3 + c][ly][lx] = b[c];
-        }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < PD_TW * PD_TH; i += blockDim.x) {
-        const int lx = i % PD_TW, ly = i / PD_TW;
-        const int x = x0 + lx, y = y0 + ly;
-        if (x >= W || y >= H) continue;
-        const size_t o = (size_t)y * W + x;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const float pxv = ps[c][ly + 1][lx + 1], pyv = ps[3 + c][ly + 1][lx + 1];
-            pxout[c * N + o] = pxv;
-            pyout[c * N + o] = pyv;
-            float step = pxv + pyv;
-            if (x > 0) step -= ps[c][ly + 1][lx];
-            if (y > 0) step -= ps[3 + c][ly][lx + 1];
-            const float unew = us[c][ly + 1][lx + 1] + tau * step;
-            const float v = (tau * F[c * N + o] + lam * unew) / (tau + lam);
-            if (u_final) {
-                const float uold = u_final[c * N + o];
-                u_final[c * N + o] = v;
-                uout[c * N + o] = uold + theta * (v - uold);
-            } else {
-                uout[c * N + o] = v;
-            }
-        }
-    }
-}
-
 }  // namespace
 
 lfrv_status run_hole_filling(lfrv_ctx *ctx, int iters, double eps, int *ran)
@@ -495,31 +398,6 @@ lfrv_status run_push_pull(lfrv_ctx *ctx, int levels)
         LFRV_HIP(ctx, hipMemcpyAsync(tmp + c * N, img + c * tot, N * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
     k_pp_finish<<<blocks_for(3 * N), kBlock, 0, ctx->stream>>>(N, tmp, ctx->U);
     LFRV_LAUNCH(ctx, "push-pull");
-    return LFRV_OK;
-}
-
-lfrv_status run_pd_steps(lfrv_ctx *ctx, int iters, const float *F, bool overrelax, float theta, const int *halt)
-{
-    const int W = ctx->W, H = ctx->H;
-    const float tau = (float)(0.3 / std::sqrt(8.0)), sigma = (float)(0.3 / std::sqrt(8.0));
-    const float L = (float)(1.0 / (double)ctx->p.lambda);
-    const float lam = (float)(1.0 / (double)L);
-    dim3 gs((W + PD_TW - 1) / PD_TW, (H + PD_TH - 1) / PD_TH);
-    const float *g = ctx->has_reg_g ? ctx->reg_g : nullptr;
-    for (int k = 0; k < iters; k++) {
-        float *uin = ctx->Uq, *uout = ctx->U2;
-        float *pxin = ctx->PX, *pyin = ctx->PY, *pxout = ctx->P2X, *pyout = ctx->P2Y;
-        float *ufin = (overrelax && k == iters - 1) ? ctx->U : nullptr;
-        const KernelEvents ev = kernel_events(ctx, 2);  // stamped by the dispatch itself
-        hipExtLaunchKernelGGL(k_pd_step, gs, dim3(256), 0, ctx->stream, ev.a, ev.b, 0, W, H, tau, lam, sigma,
-                              (const float *)uin, uout, (const float *)pxin, (const float *)pyin, pxout, pyout, F, g,
-                              ufin, theta, halt);
-        record_kernel_events(ctx, 2, ev);
-        std::swap(ctx->Uq, ctx->U2);
-        std::swap(ctx->PX, ctx->P2X);
-        std::swap(ctx->PY, ctx->P2Y);
-    }
-    LFRV_LAUNCH(ctx, "pd step");
     return LFRV_OK;
 }
 

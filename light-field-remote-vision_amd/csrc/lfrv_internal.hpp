@@ -531,8 +531,9 @@ struct StripSize {
 struct StripGeom {
     int nx, rows, nblocks;
 };
-int sr_strip_rows(int ks, bool grad, const StripSize *sizes, int n);
-StripGeom sr_strips(int ks, bool grad, StripSize size, int rows);
+int sr_lag(int ks, bool grad);  // a step's halo: rows and columns on each side
+int strip_rows(int lag, const StripSize *sizes, int n);
+StripGeom strips(int lag, StripSize size, int rows);
 // One solve's FISTA steps inside a batched launch: step s reads U[s & 1],
 // PX[s & 1], PY[s & 1] and writes the other parity (the pointer swaps of
 // the solve's own steps), with theta[s] of its FISTA sequence.

@@ -180,3 +180,15 @@ def test_sr_steps_at_strip_edges(w, h, dsf, beta):
     d.grid, d.w, d.h, d.dsf, d.render_scale = 3, w, h, dsf, dsf
     d.focal, d.baseline = float(w), 0.7 * 4.0 / (w * dsf)
     _steps_match_oracle(lfrv.synth(d), beta, 0, 1, metas=1, steps=3)
+
+
+@pytest.mark.parametrize("w,h,dsf,inner", [(62, 5, 1, 1),    # one strip of a pass of one iteration, exactly
+                                           (57, 7, 1, 4),    # four iterations per pass: a second strip of one column
+                                           (59, 9, 1, 5),    # three and two
+                                           (30, 4, 2, 4), (33, 3, 2, 9)])  # three after the first; four and four
+def test_pd_passes_at_strip_edges(w, h, dsf, inner):
+    """Several primal-dual iterations per pass where the strips end, against the oracle."""
+    d = lfrv.synth_desc(1, 3)
+    d.grid, d.w, d.h, d.dsf, d.render_scale = 3, w, h, dsf, dsf
+    d.focal, d.baseline = float(w), 0.7 * 4.0 / (w * dsf)
+    _steps_match_oracle(lfrv.synth(d), 0.3, 0, inner, metas=1, steps=2)
