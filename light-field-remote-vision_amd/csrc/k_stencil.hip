@@ -169,109 +169,147 @@ __global__ void k_conv_cols(int W, int H, Taps t, const float *__restrict__ in, 
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-__global__ void k_pp_reduce_rows(int Ws, int Hs, int hs, const float *__restrict__ in, float *__restrict__ tmp,
-                                 size_t in_cstride, size_t tmp_cstride)
+// Both passes of a reduction or expansion run in one kernel, which forms the
+// few row results that it needs again (the same sums in the same order), and
+// the levels of at most kPpTail pixels in one block per channel, in LDS: a
+// 256^2 image takes 5 launches where one per level, direction and pass, with
+// copies of level 0 around them, took 50 of some 3 us each.
+constexpr int kPpTail = 4096;
+
+// Weighted mean of the nonzero values among the five (0 if none).
+template <class At>
+__device__ __forceinline__ float pp_mean5(At at)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y, c = blockIdx.z;
-    if (j >= Ws || i >= hs) return;
     const float a = 0.4f;
     const float k[5] = {0.25f - 0.5f * a, 0.25f, a, 0.25f, 0.25f - 0.5f * a};
-    const int rows[5] = {max(2 * i - 2, 0), max(2 * i - 1, 0), 2 * i, min(2 * i + 1, Hs - 1), min(2 * i + 2, Hs - 1)};
-    const float *p = in + c * in_cstride;
     float s = 0.0f, wt = 0.0f;
+#pragma unroll
     for (int q = 0; q < 5; q++) {
-        const float v = p[(size_t)rows[q] * Ws + j];
+        const float v = at(q);
         if (v != 0.0f) { s += k[q] * v; wt += k[q]; }
     }
-    tmp[c * tmp_cstride + (size_t)i * Ws + j] = (wt == 0.0f) ? 0.0f : s / wt;
+    return (wt == 0.0f) ? 0.0f : s / wt;
 }
 
-__global__ void k_pp_reduce_cols(int Ws, int hs, int ws, const float *__restrict__ tmp, float *__restrict__ out,
-                                 size_t tmp_cstride, size_t out_cstride)
+__device__ __forceinline__ int pp_tap(int i, int q, int n) { return clampi(2 * i - 2 + q, 0, n - 1); }
+
+// Pixel (i, j) of the next coarser level of in (Ws x Hs): rows first.
+__device__ __forceinline__ float pp_reduce(const float *in, int Ws, int Hs, int i, int j)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y, c = blockIdx.z;
-    if (j >= ws || i >= hs) return;
+    return pp_mean5([&](int q) {
+        const float *col = in + pp_tap(j, q, Ws);
+        return pp_mean5([&](int r) { return col[(size_t)pp_tap(i, r, Hs) * Ws]; });
+    });
+}
+
+// Visibility there: OR over the same 5 x 5 support.
+template <class V>
+__device__ __forceinline__ uint8_t pp_reduce_vis(const V *vis, int Ws, int Hs, int i, int j)
+{
+    bool v = false;
+    for (int r = 0; r < 5; r++)
+        for (int q = 0; q < 5; q++) v |= vis[(size_t)pp_tap(i, r, Hs) * Ws + pp_tap(j, q, Ws)] != (V)0;
+    return v ? 1 : 0;
+}
+
+// Position i of a line of n coarser values, at twice the density.
+template <class At>
+__device__ __forceinline__ float pp_expand1(int i, int n, At at)
+{
     const float a = 0.4f;
     const float k[5] = {0.25f - 0.5f * a, 0.25f, a, 0.25f, 0.25f - 0.5f * a};
-    const int cols[5] = {max(2 * j - 2, 0), max(2 * j - 1, 0), 2 * j, min(2 * j + 1, Ws - 1), min(2 * j + 2, Ws - 1)};
-    const float *p = tmp + c * tmp_cstride + (size_t)i * Ws;
-    float s = 0.0f, wt = 0.0f;
-    for (int q = 0; q < 5; q++) {
-        const float v = p[cols[q]];
-        if (v != 0.0f) { s += k[q] * v; wt += k[q]; }
-    }
-    out[c * out_cstride + (size_t)i * ws + j] = (wt == 0.0f) ? 0.0f : s / wt;
-}
-
-// visibility pyramid: OR over the same 5 x 5 support
-__global__ void k_pp_reduce_vis(int Ws, int Hs, int ws, int hs, const uint8_t *__restrict__ in, uint8_t *__restrict__ out)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
-    if (j >= ws || i >= hs) return;
-    uint8_t v = 0;
-    const int rows[5] = {max(2 * i - 2, 0), max(2 * i - 1, 0), 2 * i, min(2 * i + 1, Hs - 1), min(2 * i + 2, Hs - 1)};
-    const int cols[5] = {max(2 * j - 2, 0), max(2 * j - 1, 0), 2 * j, min(2 * j + 1, Ws - 1), min(2 * j + 2, Ws - 1)};
-    for (int a = 0; a < 5; a++)
-        for (int b = 0; b < 5; b++) v |= in[(size_t)rows[a] * Ws + cols[b]] ? 1 : 0;
-    out[(size_t)i * ws + j] = v;
-}
-
-__global__ void k_pp_expand_rows(int ws, int hs, int Hs, const float *__restrict__ in, float *__restrict__ tmp,
-                                 size_t in_cstride, size_t tmp_cstride)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y, c = blockIdx.z;
-    if (j >= ws || i >= Hs) return;
-    const float a = 0.4f;
-    const float k[5] = {0.25f - 0.5f * a, 0.25f, a, 0.25f, 0.25f - 0.5f * a};
-    const float *p = in + c * in_cstride;
     float s = 0.0f;
     if (i % 2 == 0) {
-        const int r0 = max((i - 2) / 2, 0), r2 = min((i + 2) / 2, hs - 1);
-        s += 2.0f * k[0] * p[(size_t)r0 * ws + j];
-        s += 2.0f * k[2] * p[(size_t)min(i / 2, hs - 1) * ws + j];
-        s += 2.0f * k[4] * p[(size_t)r2 * ws + j];
+        s += 2.0f * k[0] * at(max((i - 2) / 2, 0));
+        s += 2.0f * k[2] * at(min(i / 2, n - 1));
+        s += 2.0f * k[4] * at(min((i + 2) / 2, n - 1));
     } else {
-        const int r1 = max((i - 1) / 2, 0), r3 = min((i + 1) / 2, hs - 1);
-        s += 2.0f * k[1] * p[(size_t)r1 * ws + j];
-        s += 2.0f * k[3] * p[(size_t)r3 * ws + j];
+        s += 2.0f * k[1] * at(max((i - 1) / 2, 0));
+        s += 2.0f * k[3] * at(min((i + 1) / 2, n - 1));
     }
-    tmp[c * tmp_cstride + (size_t)i * ws + j] = s;
+    return s;
 }
 
-__global__ void k_pp_expand_cols(int Ws, int Hs, int ws, const float *__restrict__ tmp, float *__restrict__ out,
-                                 const uint8_t *__restrict__ vis, size_t tmp_cstride, size_t out_cstride)
+// Pixel (i, j) of the next finer level of in (ws x hs): rows first.
+__device__ __forceinline__ float pp_expand(const float *in, int ws, int hs, int i, int j)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y, c = blockIdx.z;
-    if (j >= Ws || i >= Hs) return;
-    if (vis[(size_t)i * Ws + j]) return;
-    const float a = 0.4f;
-    const float k[5] = {0.25f - 0.5f * a, 0.25f, a, 0.25f, 0.25f - 0.5f * a};
-    const float *p = tmp + c * tmp_cstride + (size_t)i * ws;
-    float s = 0.0f;
-    if (j % 2 == 0) {
-        const int c0 = max((j - 2) / 2, 0), c2 = min((j + 2) / 2, ws - 1);
-        s += 2.0f * k[0] * p[c0];
-        s += 2.0f * k[2] * p[min(j / 2, ws - 1)];
-        s += 2.0f * k[4] * p[c2];
-    } else {
-        const int c1 = max((j - 1) / 2, 0), c3 = min((j + 1) / 2, ws - 1);
-        s += 2.0f * k[1] * p[c1];
-        s += 2.0f * k[3] * p[c3];
+    return pp_expand1(j, ws, [&](int x) { return pp_expand1(i, hs, [&](int y) { return in[(size_t)y * ws + x]; }); });
+}
+
+// One level down; V: the finer level's visibility is the target's float map (level 0) or bytes.
+template <class V>
+__global__ void k_pp_reduce(int Ws, int Hs, int ws, int hs, const float *__restrict__ in, size_t in_cstride,
+                            const V *__restrict__ vis, float *__restrict__ out, size_t out_cstride,
+                            uint8_t *__restrict__ vout)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y;
+    if (k >= ws * hs) return;
+    const int i = k / ws, j = k - i * ws;
+    out[c * out_cstride + k] = pp_reduce(in + c * in_cstride, Ws, Hs, i, j);
+    if (c == 0) vout[k] = pp_reduce_vis(vis, Ws, Hs, i, j);
+}
+
+// One level up, where nothing is visible.
+__global__ void k_pp_expand(int Ws, int Hs, int ws, int hs, const float *__restrict__ in, float *__restrict__ out,
+                            const uint8_t *__restrict__ vis, size_t cstride)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y;
+    if (k >= Ws * Hs || vis[k]) return;
+    const int i = k / Ws, j = k - i * Ws;
+    out[c * cstride + k] = pp_expand(in + c * cstride, ws, hs, i, j);
+}
+
+// The last level up, and U <- filled - U (optimization.cu:629-646); without levels (ws = 0) filled is U.
+__global__ void k_pp_finish(int W, int H, int ws, int hs, const float *__restrict__ in, size_t in_cstride,
+                            const float *__restrict__ vis, float *__restrict__ U)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y;
+    if (k >= W * H) return;
+    const int i = k / W, j = k - i * W;
+    const size_t o = (size_t)c * W * H + k;
+    const float u = U[o];
+    U[o] = (ws == 0 || vis[k] != 0.0f ? u : pp_expand(in + c * in_cstride, ws, hs, i, j)) - u;
+}
+
+// Every level below (w, h): down to the coarsest and back up to it, channel
+// blockIdx.x, in place.
+__global__ void __launch_bounds__(1024) k_pp_tail(int w, int h, int levels, float *__restrict__ img, size_t cstride,
+                                                  const uint8_t *__restrict__ vis)
+{
+    __shared__ float px[kPpTail + kPpTail / 2];  // the levels one behind the other: a quarter of the pixels each
+    __shared__ uint8_t vs[kPpTail + kPpTail / 2];
+    float *p = img + blockIdx.x * cstride;
+    for (int k = threadIdx.x; k < w * h; k += blockDim.x) {
+        px[k] = p[k];
+        vs[k] = vis[k];
     }
-    out[c * out_cstride + (size_t)i * Ws + j] = s;
-}
-
-__global__ void k_vis_to_u8(size_t N, const float *__restrict__ vis, uint8_t *__restrict__ out)
-{
-    const size_t o = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o < N) out[o] = vis[o] != 0.0f ? 1 : 0;
-}
-
-// U <- filled - U (optimization.cu:629-646)
-__global__ void k_pp_finish(size_t N, const float *__restrict__ filled, float *__restrict__ U)
-{
-    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < 3 * N) U[k] = filled[k] - U[k];
+    __syncthreads();
+    int o = 0, ws = w, hs = h;
+    for (int l = 0; l < levels; l++) {
+        const int on = o + ws * hs, wn = ws / 2, hn = hs / 2;
+        for (int k = threadIdx.x; k < wn * hn; k += blockDim.x) {
+            const int i = k / wn, j = k - i * wn;
+            px[on + k] = pp_reduce(px + o, ws, hs, i, j);
+            vs[on + k] = pp_reduce_vis(vs + o, ws, hs, i, j);
+        }
+        __syncthreads();
+        o = on;
+        ws = wn;
+        hs = hn;
+    }
+    for (int l = levels; l > 0; l--) {
+        const int wf = w >> (l - 1), hf = h >> (l - 1), of = o - wf * hf;
+        for (int k = threadIdx.x; k < wf * hf; k += blockDim.x) {
+            if (vs[of + k]) continue;
+            const int i = k / wf, j = k - i * wf;
+            px[of + k] = pp_expand(px + o, ws, hs, i, j);
+        }
+        __syncthreads();
+        o = of;
+        ws = wf;
+        hs = hf;
+    }
+    for (int k = threadIdx.x; k < w * h; k += blockDim.x) p[k] = px[k];
 }
 
 }  // namespace
@@ -372,31 +410,31 @@ lfrv_status run_push_pull(lfrv_ctx *ctx, int levels)
         tot += (size_t)wsn * hsn;
         top = s;
     }
-    // scratch: pyramid images (3 * tot floats) + row temp (3 * N floats) + vis pyramid (tot bytes)
-    const size_t need = 3 * tot + 3 * N + (tot + 3) / 4 + 1;
+    // scratch: pyramid images (3 * tot floats) + vis pyramid (tot bytes); level 0 stays in U and the target's map
+    const size_t need = 3 * tot + (tot + 3) / 4 + 1;
     if (need > ctx->pp_cap) return fail(ctx, LFRV_E_ARG, "push-pull scratch too small");
-    float *img = ctx->pp_scratch, *tmp = img + 3 * tot;
-    uint8_t *vis = reinterpret_cast<uint8_t *>(tmp + 3 * N);
-    for (int c = 0; c < 3; c++)
-        LFRV_HIP(ctx, hipMemcpyAsync(img + c * tot, ctx->U + c * N, N * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
-    k_vis_to_u8<<<blocks_for(N), kBlock, 0, ctx->stream>>>(N, ctx->visibility, vis);
-    for (int s = 1; s <= top; s++) {
-        const int Ws = ws[s - 1], Hs = hs[s - 1], wsn = ws[s], hsn = hs[s];
-        dim3 g1((Ws + 255) / 256, hsn, 3), g2((wsn + 255) / 256, hsn, 3), g3((wsn + 255) / 256, hsn, 1);
-        k_pp_reduce_rows<<<g1, 256, 0, ctx->stream>>>(Ws, Hs, hsn, img + off[s - 1], tmp, tot, N);
-        k_pp_reduce_cols<<<g2, 256, 0, ctx->stream>>>(Ws, hsn, wsn, tmp, img + off[s], N, tot);
-        k_pp_reduce_vis<<<g3, 256, 0, ctx->stream>>>(Ws, Hs, wsn, hsn, vis + off[s - 1], vis + off[s]);
+    float *img = ctx->pp_scratch;
+    uint8_t *vis = reinterpret_cast<uint8_t *>(img + 3 * tot);
+    auto grid = [](int w, int h) { return dim3(blocks_for((size_t)w * h), 3); };
+    // the levels from `tail` on in one launch
+    int tail = 1;
+    while (tail < top && (size_t)ws[tail] * hs[tail] > kPpTail) tail++;
+    for (int s = 1; s <= tail && s <= top; s++) {
+        if (s == 1)
+            k_pp_reduce<<<grid(ws[1], hs[1]), kBlock, 0, ctx->stream>>>(W, H, ws[1], hs[1], ctx->U, N, ctx->visibility,
+                                                                        img + off[1], tot, vis + off[1]);
+        else
+            k_pp_reduce<<<grid(ws[s], hs[s]), kBlock, 0, ctx->stream>>>(ws[s - 1], hs[s - 1], ws[s], hs[s],
+                                                                        img + off[s - 1], tot, vis + off[s - 1],
+                                                                        img + off[s], tot, vis + off[s]);
     }
-    for (int s = top; s > 0; s--) {
-        const int Ws = ws[s - 1], Hs = hs[s - 1], wsn = ws[s], hsn = hs[s];
-        dim3 g1((wsn + 255) / 256, Hs, 3), g2((Ws + 255) / 256, Hs, 3);
-        k_pp_expand_rows<<<g1, 256, 0, ctx->stream>>>(wsn, hsn, Hs, img + off[s], tmp, tot, N);
-        k_pp_expand_cols<<<g2, 256, 0, ctx->stream>>>(Ws, Hs, wsn, tmp, img + off[s - 1], vis + off[s - 1], N, tot);
-    }
-    // gather the three level-0 planes contiguously, then U <- filled - U
-    for (int c = 0; c < 3; c++)
-        LFRV_HIP(ctx, hipMemcpyAsync(tmp + c * N, img + c * tot, N * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
-    k_pp_finish<<<blocks_for(3 * N), kBlock, 0, ctx->stream>>>(N, tmp, ctx->U);
+    if (tail < top)
+        k_pp_tail<<<3, 1024, 0, ctx->stream>>>(ws[tail], hs[tail], top - tail, img + off[tail], tot, vis + off[tail]);
+    for (int s = std::min(tail, top); s > 1; s--)
+        k_pp_expand<<<grid(ws[s - 1], hs[s - 1]), kBlock, 0, ctx->stream>>>(
+            ws[s - 1], hs[s - 1], ws[s], hs[s], img + off[s], img + off[s - 1], vis + off[s - 1], tot);
+    k_pp_finish<<<grid(W, H), kBlock, 0, ctx->stream>>>(W, H, top ? ws[1] : 0, top ? hs[1] : 0,
+                                                        img + (top ? off[1] : 0), tot, ctx->visibility, ctx->U);
     LFRV_LAUNCH(ctx, "push-pull");
     return LFRV_OK;
 }
