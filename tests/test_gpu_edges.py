@@ -104,3 +104,23 @@ def test_color_sr_ragged_inputs(w, h, dsf, inner):
         e, _ = ctx.sr_primal_energy()
         oe, _ = oracle.sr_energy(W, H, dsf, tx, ty, s["views"], om, sig, lam, 1.0, beta, 0, vis, st.U)
         assert abs(e - oe) <= 1e-4 * max(oe, 1e-12)
+
+
+@pytest.mark.parametrize("w,h,dead", [(17, 33, (0, 17, 0, 16)),    # holes to three image edges, one tile past the second
+                                      (48, 40, (8, 40, 8, 24)),    # whole tiles of holes
+                                      (65, 20, (60, 65, 3, 20))])  # one column in the last tile
+def test_hole_sweeps_at_tile_edges(w, h, dead):
+    """The Poisson diffusion in tiles of 16 x 16 and eight sweeps per launch, against sweep after sweep in FP64."""
+    print(f"hole filling {w}x{h} holes {dead}", flush=True)
+    d = lfrv.synth_desc(2, 11)
+    d.grid, d.w, d.h, d.focal = 2, w, h, 1000.0 * w / 1024.0
+    s = lfrv.synth(d)
+    s["depths"] = s["depths"].copy()
+    s["depths"][:, dead[2]:dead[3], dead[0]:dead[1]] = 0.0
+    with lfrv.Context(pipelines.gradient_ibr_params(s)) as ctx:
+        pipelines.load_scene(ctx, s)
+        pipelines.gradient_ibr_solve(ctx, 1e-5, 3000)
+        U = ctx.get_solution()
+    r = oracle.gibr_pipeline(s["views"], s["depths"], s["P_views"], s["P_target"], 1, 1 / 255.0, 1.0, 1.0, 0.5, 1e-5, 3000)
+    # two solves to a relative residual of 1e-5
+    assert rel_err(U, r["U"]) < 1e-3
