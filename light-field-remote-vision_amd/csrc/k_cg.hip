@@ -9,6 +9,7 @@
 //   k_cg_update x += alpha d, r -= alpha q, per-block r.r and r.z; a one-block
 //               kernel sums them, tests convergence and computes beta.
 // d is double-buffered because neighbouring tiles read it in their halos.
+#include "strip_common.hpp"
 #include "tile_common.hpp"
 
 #include <hip/hip_ext.h>
@@ -1133,12 +1134,11 @@ constexpr int box_lds_floats()
     return 3 * (S::LW * S::LH + S::LH * S::BW + S::BH * S::BW + S::QW * S::QH);
 }
 
-enum : int { kBoxResInit = 0, kBoxBegin = 1, kBoxOp = 2, kBoxResid = 3 };
+enum : int { kBoxResInit = 0, kBoxBegin = 1, kBoxResid = 2 };
 
 // One box-operator pass over the tiles.
 //   kBoxResInit: r = b - A x, u = Minv r (no sums)
 //   kBoxBegin:   w = A u; 12 sums r.r, r.u, b.b, w.u (the begin pass)
-//   kBoxOp:      w = A u; 9 sums r.u, w.u, r.r (a PCG iteration)
 //   kBoxResid:   3 sums |b - A x|^2 (the true residual)
 // `in` is x (ResInit, Resid) or u (Begin, Op).  A solve already done returns.
 template <int KS, int MODE>
@@ -1150,13 +1150,12 @@ __global__ void __launch_bounds__(kBoxTW * kBoxTH) k_box_pass(int W, int H, int 
                                                                 const float *__restrict__ r,
                                                                 const float *__restrict__ minv,
                                                                 float *__restrict__ out, float *__restrict__ out2,
-                                                                const CgState *st, double *partials)
+                                                                double *partials)
 {
     constexpr int NL = box_lds_floats<KS>();
     __shared__ float lds[NL];
     __shared__ double red[12 * 16];
     using S = BoxDims<KS>;
-    if (MODE == kBoxOp && st->done) return;
     float *su = lds, *sh = su + 3 * S::LW * S::LH, *sb = sh + 3 * S::LH * S::BW, *sq = sb + 3 * S::BH * S::BW;
     const int t = xcd_tile(blockIdx.x, ntiles);
     const int tx0 = (t % ntx) * S::TW, ty0 = (t / ntx) * S::TH;
@@ -1165,7 +1164,7 @@ __global__ void __launch_bounds__(kBoxTW * kBoxTH) k_box_pass(int W, int H, int 
     const size_t N = (size_t)W * H, o = pin ? (size_t)y * W + x : 0;
     float av[3], uv[3];
     box_apply_tile<KS>(W, H, Wc, Hc, tx0, ty0, wscale, c0, beta_reg, ops, NA, in, su, sh, sb, sq, av, uv);
-    constexpr int NQS = MODE == kBoxBegin ? 12 : MODE == kBoxOp ? 9 : 3;
+    constexpr int NQS = MODE == kBoxBegin ? 12 : 3;
     double v[NQS];
 #pragma unroll
     for (int q = 0; q < NQS; q++) v[q] = 0.0;
@@ -1184,33 +1183,37 @@ __global__ void __launch_bounds__(kBoxTW * kBoxTH) k_box_pass(int W, int H, int 
             } else {
                 out[k] = av[c];
                 const double rr = r[k], uu = uv[c], ww = av[c];
-                if (MODE == kBoxBegin) {
-                    const double bb = b[k];
-                    v[c] += rr * rr;
-                    v[3 + c] += rr * uu;
-                    v[6 + c] += bb * bb;
-                    v[9 + c] += ww * uu;
-                } else {
-                    v[c] += rr * uu;
-                    v[3 + c] += ww * uu;
-                    v[6 + c] += rr * rr;
-                }
+                const double bb = b[k];
+                v[c] += rr * rr;
+                v[3 + c] += rr * uu;
+                v[6 + c] += bb * bb;
+                v[9 + c] += ww * uu;
             }
         }
     }
     if (MODE != kBoxResInit) block_partials<NQS>(v, partials, red);
 }
 
-// The vector updates of a PCG iteration from the scalars of the state:
-// s_i = w_i + beta s_{i-1}, p_i = Minv r_i + beta p_{i-1}, x += alpha p_i,
-// r_{i+1} = r_i - alpha s_i, u_{i+1} = Minv r_{i+1} (the operand of the next
-// box pass), per pixel and channel (the same updates as k_cgcg_st2's).
-__global__ void __launch_bounds__(256) k_box_update(size_t N, const CgState *st, const float *__restrict__ minv,
-                                                    const float *__restrict__ r_in, const float *__restrict__ w_in,
-                                                    const float *__restrict__ s_in, float *__restrict__ r_out,
-                                                    float *__restrict__ s_out, float *__restrict__ p,
-                                                    float *__restrict__ x, float *__restrict__ u)
+// One PCG iteration on the box operator as a marching strip: the vector updates
+// of s, p, x, r and u = Minv r (the same as k_cgcg_st2's, formed for the halo
+// too), then w = A u of the row D behind (row sums by wave shifts, column sums
+// as partial chains, the couplings G, the sums back) and the iteration's sums.
+// It replaced an update kernel and a 32 x 16 tile pass with six LDS phases,
+// which passed u through memory: 25 views, 1024^2, dsf 4: 21 + 34 us, now 36
+// us for 166 N bytes (4.8 TB/s).
+struct BoxIter {
+    const float *r_in, *w_in, *s_in, *minv, *ops;
+    float *r_out, *w_out, *s_out, *p, *x;
+};
+
+template <int D, bool WIDE>
+__global__ void __launch_bounds__(256) k_box_iter(int W, int H, int Wc, int Hc, StripGeom sg, float wscale, float c0,
+                                                  float beta_reg, size_t NA, BoxIter a, const CgState *st,
+                                                  double *partials)
 {
+    constexpr int RING = D < kStripGroup ? kStripGroup : 2 * kStripGroup, WARM = 2 * D;
+    static_assert(D < RING, "the ring holds the rows from the output row to the newest");
+    __shared__ double red[9 * 16];
     const int done = st->done, first = st->first;
     float al[3], be[3];
     for (int c = 0; c < 3; c++) {
@@ -1218,23 +1221,158 @@ __global__ void __launch_bounds__(256) k_box_update(size_t N, const CgState *st,
         be[c] = (float)st->beta[c];
     }
     if (done) return;
-    for (size_t o = (size_t)blockIdx.x * blockDim.x + threadIdx.x; o < N; o += (size_t)gridDim.x * blockDim.x) {
-        const float mi = minv[o];
+    const size_t N = (size_t)W * H;
+    const int strip = __builtin_amdgcn_readfirstlane(4 * xcd_tile(blockIdx.x, sg.nblocks) + (int)(threadIdx.x >> 6));
+    const int sy = strip / sg.nx, sx = strip - sy * sg.nx, y0 = sy * sg.rows, y1 = min(y0 + sg.rows, H);
+    double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (y0 < H) {  // (a block's last strips may lie below the target; its sums take all four)
+        const int lane = threadIdx.x & 63, x = sx * (64 - 2 * D) - D + lane;
+        const bool xin = x >= 0 && x < W, own = xin && lane >= D && lane < 64 - D;
+        const int vx = xin ? 4 * x : kOutside, vs = own ? vx : kOutside, vc = x >= 0 && x < Wc ? 4 * x : kOutside;
+        const float kx = W > 1 ? (x > 0 && x < W - 1 ? 2.0f : 1.0f) : 0.0f;
+        const Planes<WIDE> bR(a.r_in, 3, N, W), bW(a.w_in, 3, N, W), bS(a.s_in, 3, N, W), bM(a.minv, 1, N, W),
+            bC(a.ops, 5, NA, Wc), bP(a.p, 3, N, W), bX(a.x, 3, N, W), bRo(a.r_out, 3, N, W), bWo(a.w_out, 3, N, W),
+            bSo(a.s_out, 3, N, W);
+        const int row0 = y0 - D, yend = y1 + D;  // rows of u
+        struct Loads {
+            float r[3], w[3], s[3], p[3], x[3], mi, f[5];
+        } ld[3];
+        auto fetch = [&](Loads &l, int yn) __attribute__((always_inline)) {
+            const int yq = yn - 1;
+            const int vu = yn >= 0 && yn < min(H, yend) ? vx : kOutside;
+            const int vq = yq >= max(0, y0 - 1) && yq < Hc && yn < yend ? vc : kOutside;
+            const int vp = yn >= y0 && yn < y1 ? vs : kOutside;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                l.r[c] = bR.load(c, yn, vu);
+                l.w[c] = bW.load(c, yn, vu);
+                l.s[c] = bS.load(c, yn, vu);
+                l.p[c] = bP.load(c, yn, vp);
+                l.x[c] = bX.load(c, yn, vp);
+            }
+            l.mi = bM.load(0, yn, vu);
+#pragma unroll
+            for (int k = 0; k < 5; k++) l.f[k] = bC.load(k, yq, vq);
+        };
+        float u[RING][3], rn[RING][3];     // the last rows of u and r
+        float bc[3][D - 1], qc[3][D - 1];  // column chains of the row sums of u and of G's results
+        float bm[3][3], b0[3][3];          // box sums of the two rows before the newest, left, own, right
+        float s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;  // the coupling row above: south, left's south-east, right's south-west
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const size_t k = c * N + o;
-            const float rv = r_in[k];
-            const float s = first ? w_in[k] : w_in[k] + be[c] * s_in[k];
-            const float uo = mi * rv;
-            const float pn = first ? uo : uo + be[c] * p[k];
-            const float rn = rv - al[c] * s;
-            p[k] = pn;
-            x[k] += al[c] * pn;
-            s_out[k] = s;
-            r_out[k] = rn;
-            u[k] = mi * rn;
+#pragma unroll
+            for (int k = 0; k < RING; k++) u[k][c] = rn[k][c] = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 3; d++) bm[c][d] = b0[c][d] = 0.0f;
+#pragma unroll
+            for (int d = 0; d < D - 1; d++) bc[c][d] = qc[c][d] = 0.0f;
+        }
+        auto chain = [](float(&ch)[D - 1], float val) __attribute__((always_inline)) {
+            const float sum = ch[D - 2] + val;
+#pragma unroll
+            for (int d = D - 2; d > 0; d--) ch[d] = ch[d - 1] + val;
+            ch[0] = val;
+            return sum;
+        };
+        auto row = [&](auto K, auto PHASE, int yn) __attribute__((always_inline)) {
+            constexpr int k = decltype(K)::value, ph = decltype(PHASE)::value;  // 0: box sums only; 1: and G; 2: output
+            constexpr int ku = k % RING, ko = (k + RING - D) % RING;
+            constexpr int kup = (ko + RING - 1) % RING, kdn = (ko + 1) % RING;  // the rows above and below the output row
+            const Loads &l = ld[k % 3];
+            fetch(ld[(k + 2) % 3], yn + 2);
+            const int vo = yn >= y0 && yn < y1 ? vs : kOutside;
+            float up1[3];  // (the row above the output row: overwritten below where the ring is only just long enough)
+#pragma unroll
+            for (int c = 0; c < 3; c++) up1[c] = u[kup][c];
+            float bp[3][3];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const float sv = first ? l.w[c] : fmaf(be[c], l.s[c], l.w[c]);
+                const float uo = l.mi * l.r[c], pn = first ? uo : fmaf(be[c], l.p[c], uo);
+                const float rv = fmaf(-al[c], sv, l.r[c]), uc = l.mi * rv;
+                bP.store(pn, c, yn, vo);
+                bX.store(fmaf(al[c], pn, l.x[c]), c, yn, vo);
+                bSo.store(sv, c, yn, vo);
+                bRo.store(rv, c, yn, vo);
+                u[ku][c] = uc;
+                rn[ku][c] = rv;
+                float rs = uc;
+#pragma unroll
+                for (int d = 1; d < D; d++) rs = uc + from_left(rs);
+                bp[c][1] = chain(bc[c], rs);
+                bp[c][0] = from_left(bp[c][1]);
+                bp[c][2] = from_right(bp[c][1]);
+            }
+            if constexpr (ph >= 1) {
+                const float fw = from_left(l.f[1]);
+                const int yo = yn - D, vw = yo < y1 ? vs : kOutside;
+                const bool mine = own && yo < y1;
+                const float ky = H > 1 ? (yo > 0 && yo < H - 1 ? 2.0f : 1.0f) : 0.0f;
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const float *m = bm[c], *z = b0[c], *p = bp[c];
+                    float w = fmaf(l.f[0], z[1], l.f[1] * z[2]);
+                    w = fmaf(l.f[2], p[1], fmaf(fw, z[0], w));
+                    w = fmaf(l.f[3], p[2], fmaf(s1, m[1], w));
+                    w = fmaf(l.f[4], p[0], fmaf(s2, m[0], w));
+                    const float q = fmaf(s3, m[2], w);
+                    float rs = q, qr = q;
+#pragma unroll
+                    for (int d = 1; d < D; d++) {
+                        qr = from_right(qr);
+                        rs += qr;
+                    }
+                    const float acc = chain(qc[c], rs);
+                    if constexpr (ph == 2) {
+                        // D^T D u with Neumann boundary: outside the image u is 0 and the centre counts once
+                        const float dv = u[ko][c];
+                        const float lx = kx * dv - from_left(dv) - from_right(dv);
+                        const float lap = lx + (ky * dv - up1[c] - u[kdn][c]);
+                        const float av = fmaf(beta_reg, lap, fmaf(c0, dv, wscale * acc));
+                        bWo.store(av, c, yo, vw);
+                        const double rr = mine ? rn[ko][c] : 0.0f, uu = mine ? dv : 0.0f, ww = av;
+                        v[c] += rr * uu;
+                        v[3 + c] += ww * uu;
+                        v[6 + c] += rr * rr;
+                    }
+                }
+            }
+            s1 = l.f[2];
+            s2 = from_left(l.f[3]);
+            s3 = from_right(l.f[4]);
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    bm[c][d] = b0[c][d];
+                    b0[c][d] = bp[c][d];
+                }
+        };
+#pragma unroll
+        for (int k = 0; k < 2; k++) fetch(ld[k], row0 + k);
+        static_for<WARM>([&](auto K) __attribute__((always_inline)) {
+            constexpr int i = decltype(K)::value;
+            row(K, std::integral_constant<int, (i > D ? 1 : 0)>(), row0 + i);
+        });
+        for (int j0 = 0; j0 < y1 - y0; j0 += kStripGroup) {
+            static_for<kStripGroup>([&](auto J) __attribute__((always_inline)) {
+                constexpr int j = decltype(J)::value;
+                row(std::integral_constant<int, WARM + j>(), std::integral_constant<int, 2>(), row0 + WARM + j0 + j);
+            });
+            if constexpr (RING == 2 * kStripGroup)
+#pragma unroll
+                for (int k = 0; k < kStripGroup; k++)
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        const float t = u[k][c], q = rn[k][c];
+                        u[k][c] = u[k + kStripGroup][c];
+                        rn[k][c] = rn[k + kStripGroup][c];
+                        u[k + kStripGroup][c] = t;
+                        rn[k + kStripGroup][c] = q;
+                    }
         }
     }
+    block_partials<9>(v, partials, red);
 }
 
 }  // namespace
@@ -1337,7 +1475,7 @@ lfrv_status run_cg(lfrv_ctx *ctx, double alpha, double c0, double beta, bool use
         // r_0 = b - A x_0 and u_0 = Minv r_0, then w_0 = A u_0 with the start sums
         float *u = ctx->cg_extra + 9 * N;
         TimedRegion tr(ctx, 5);
-#define BP(K, M, IN, R, OUT, OUT2) k_box_pass<K, M><<<box_tiles, kBoxTW * kBoxTH, 0, ctx->stream>>>(ctx->W, ctx->H, Wc, Hc, box_ntx, box_tiles, wscale, (float)c0, (float)beta, ctx->box_ops, NA, IN, ctx->cg_b, R, minv, OUT, OUT2, stt, part)
+#define BP(K, M, IN, R, OUT, OUT2) k_box_pass<K, M><<<box_tiles, kBoxTW * kBoxTH, 0, ctx->stream>>>(ctx->W, ctx->H, Wc, Hc, box_ntx, box_tiles, wscale, (float)c0, (float)beta, ctx->box_ops, NA, IN, ctx->cg_b, R, minv, OUT, OUT2, part)
         switch (ctx->ks) {
         case 3: BP(3, kBoxResInit, x, nullptr, r, u); BP(3, kBoxBegin, u, r, ctx->cg_q, nullptr); break;
         case 4: BP(4, kBoxResInit, x, nullptr, r, u); BP(4, kBoxBegin, u, r, ctx->cg_q, nullptr); break;
@@ -1436,8 +1574,10 @@ lfrv_status run_cg(lfrv_ctx *ctx, double alpha, double c0, double beta, bool use
         float *rbuf[2] = {ctx->cg_r, ctx->cg_extra};
         float *sbuf[2] = {ctx->cg_extra + 3 * N, ctx->tmp3N};
         float *wbuf[2] = {ctx->cg_q, ctx->cg_extra + 6 * N};
-        float *u = ctx->cg_extra + 9 * N;
-        const unsigned int ub = (unsigned int)std::min<size_t>((N + 255) / 256, 8192);
+        const StripSize size{ctx->W, ctx->H};
+        const StripGeom sg = strips(ctx->ks - 1, size, strip_rows(ctx->ks - 1, &size, 1));
+        const bool wide = 20 * NA >= kNarrowBytes;
+        if ((size_t)sg.nblocks * 9 > ctx->partials_cap) return fail(ctx, LFRV_E_STATE, "partials buffer too small");
         auto box_poll = [&]() -> lfrv_status {
             {
                 TimedRegion tr(ctx, 5);
@@ -1461,19 +1601,20 @@ lfrv_status run_cg(lfrv_ctx *ctx, double alpha, double c0, double beta, bool use
             next_chunk = 4;
             for (int k = 0; k < nk; k++) {
                 {
-                    TimedRegion tr(ctx, 1);
-                    k_box_update<<<ub, 256, 0, ctx->stream>>>(N, stt, minv, rbuf[cur], wbuf[cur], sbuf[cur],
-                                                              rbuf[cur ^ 1], sbuf[cur ^ 1], ctx->cg_d, x, u);
-                }
-                {
                     TimedRegion tr(ctx, 0);
+                    const BoxIter bi{rbuf[cur],     wbuf[cur],     sbuf[cur],     minv,       ctx->box_ops,
+                                     rbuf[cur ^ 1], wbuf[cur ^ 1], sbuf[cur ^ 1], ctx->cg_d, x};
+#define BI1(D, WI) k_box_iter<D, WI><<<sg.nblocks, 256, 0, ctx->stream>>>(ctx->W, ctx->H, Wc, Hc, sg, wscale, (float)c0, (float)beta, NA, bi, stt, part)
+#define BI(D) case D + 1: if (wide) BI1(D, true); else BI1(D, false); break
                     switch (ctx->ks) {
-                    case 3: BP(3, kBoxOp, u, rbuf[cur ^ 1], wbuf[cur ^ 1], nullptr); break;
-                    case 4: BP(4, kBoxOp, u, rbuf[cur ^ 1], wbuf[cur ^ 1], nullptr); break;
-                    case 5: BP(5, kBoxOp, u, rbuf[cur ^ 1], wbuf[cur ^ 1], nullptr); break;
+                        BI(2);
+                        BI(3);
+                        BI(4);
                     }
+#undef BI
+#undef BI1
                 }
-                k_cgcg_step<<<1, kFinalizeThreads, 0, ctx->stream>>>(stt, part, box_tiles);
+                k_cgcg_step<<<1, kFinalizeThreads, 0, ctx->stream>>>(stt, part, sg.nblocks);
                 cur ^= 1;
             }
             LFRV_LAUNCH(ctx, "cg iteration");

@@ -334,7 +334,7 @@ __device__ __forceinline__ bf8v lds_transpose8(const char *p, int pitch)
 
 // grid (splits, co blocks, ci blocks); split k takes stages k, k + splits, ...
 template <int NCO, int WCO, int WCI>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, WCI == 4 ? 1 : 2)  // (its LDS fits twice in a CU but with 64 input channels)
 k_conv3x3_wgrad(const uint16_t *__restrict__ dU, const uint16_t *__restrict__ X, float *__restrict__ dW,
                 float *__restrict__ db, float *__restrict__ ws, int B, int H, int W, int Cin, int Cout, int up)
 {

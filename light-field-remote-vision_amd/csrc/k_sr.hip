@@ -3,6 +3,7 @@
 // assembled anchor-grid operator as a stencil, fused with the first
 // primal-dual iteration), the primal energy, and the re-weighting loop with
 // its stopping rules on the device.
+#include "strip_common.hpp"
 #include "tile_common.hpp"
 
 #include <hip/hip_ext.h>
@@ -11,7 +12,6 @@
 #include <climits>
 #include <chrono>
 #include <cmath>
-#include <type_traits>
 #include <vector>
 
 namespace lfrv {
@@ -265,83 +265,9 @@ __global__ void __launch_bounds__(kPullMaxThreads) k_sr_assemble(TileGeom g, Til
 // The arithmetic of a pixel does not depend on the strip it falls in, so
 // strips of any height, and batches, give the same bits.
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>());
-        static_for<N, I + 1>(f);
-    }
-}
-
-constexpr int kStripGroup = 3;  // rows per turn of the loop
-
 template <int D, bool GRAD>
 struct Strip {
     static constexpr int LAG = D + (GRAD ? 1 : 0), OW = 64 - 2 * LAG;  // output columns
-};
-
-// The lane's left (x - 1) / right (x + 1) neighbour's value, 0 past the wave
-// (every lane has to take part: never inside a select).
-__device__ __forceinline__ float from_left(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));  // wave_shr:1
-}
-__device__ __forceinline__ float from_right(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));  // wave_shl:1
-}
-
-constexpr int kOutside = (int)0x80000000;
-constexpr size_t kNarrowBytes = (size_t)1 << 31;  // kOutside lies past any buffer up to this size
-
-// Planes of `w`-wide rows, `stride` values apart.  Narrow: one descriptor for
-// all of them (at most kNarrowBytes), the row and plane in the scalar offset.
-// WIDE: a descriptor per row.
-template <bool WIDE>
-struct Planes {
-    const float *base;
-    size_t stride;
-    int w;
-    __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ Planes(const float *b, int n, size_t st, int width) : base(b), stride(st), w(width)
-    {
-        if constexpr (!WIDE) r = __builtin_amdgcn_make_buffer_rsrc((void *)b, 0, b ? (int)(4 * n * st) : 0, 0x00020000);
-    }
-    // plane c, row y (clamped at 0; a row outside comes with vo = kOutside)
-    __device__ __forceinline__ float load(int c, int y, int vo) const
-    {
-        if constexpr (WIDE) return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(row(c, y), vo, 0, 0));
-        else return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo, 4 * (c * (int)stride + max(y, 0) * w), 0));
-    }
-    __device__ __forceinline__ void store(float v, int c, int y, int vo) const
-    {
-        if constexpr (WIDE) __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), row(c, y), vo, 0, 0);
-        else __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, vo, 4 * (c * (int)stride + max(y, 0) * w), 0);
-    }
-    __device__ __forceinline__ __amdgpu_buffer_rsrc_t row(int c, int y) const
-    {
-        return __builtin_amdgcn_make_buffer_rsrc((void *)(base + c * stride + (size_t)max(y, 0) * w), 0, base ? 4 * w : 0,
-                                                 0x00020000);
-    }
-};
-
-// n / d for finite values away from the ends of the range, correctly rounded:
-// a Newton step for the reciprocal, which several quotients of one divisor
-// share, then two for the quotient.
-struct Divisor {
-    float d, r;
-    __device__ __forceinline__ explicit Divisor(float div) : d(div), r(__builtin_amdgcn_rcpf(div))
-    {
-        r = fmaf(fmaf(-d, r, 1.0f), r, r);
-    }
-    __device__ __forceinline__ float of(float n) const
-    {
-        float q = n * r;
-        q = fmaf(fmaf(-d, q, n), r, q);
-        return fmaf(fmaf(-d, q, n), r, q);
-    }
 };
 
 // The step's buffers (U read, the rest nullable where the caller's form skips it).

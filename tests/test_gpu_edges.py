@@ -124,3 +124,19 @@ def test_hole_sweeps_at_tile_edges(w, h, dead):
     r = oracle.gibr_pipeline(s["views"], s["depths"], s["P_views"], s["P_target"], 1, 1 / 255.0, 1.0, 1.0, 0.5, 1e-5, 3000)
     # two solves to a relative residual of 1e-5
     assert rel_err(U, r["U"]) < 1e-3
+
+
+@pytest.mark.parametrize("w,h,dsf", [(30, 7, 2), (31, 5, 2),    # one strip of 60 columns exactly, and two columns more
+                                     (29, 4, 3), (14, 9, 4), (15, 3, 4)])
+def test_box_iterations_at_strip_edges(w, h, dsf):
+    """The marching PCG iteration of the box operator where its strips and row groups end, against the oracle."""
+    s = _planes(w, h, dsf, 3, 5)
+    print(f"PCG {w}x{h} dsf {dsf}", flush=True)
+    with lfrv.Context(pipelines.gradient_ibr_params(s)) as ctx:
+        pipelines.load_scene(ctx, s)
+        st = pipelines.gradient_ibr_solve(ctx, 1e-6, 3000)
+        U = ctx.get_solution()
+    assert all(st["converged"])
+    r = oracle.gibr_pipeline(s["views"], s["depths"], s["P_views"], s["P_target"], dsf, 1 / 255.0, 1.0, 1.0, 0.5, 1e-6, 3000)
+    # two solves to a relative residual of 1e-6 of a system whose condition number is below 1e3
+    assert rel_err(U, r["U"]) < 1e-3
