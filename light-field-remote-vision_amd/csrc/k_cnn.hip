@@ -173,12 +173,13 @@ __device__ __forceinline__ void conv_epilogue(const CnnConv &a, f4v (&v)[4], int
 // against 2.92 (the masks, skips, fills and resamplings of the backward pass
 // took 0.75 ms).
 template <int EPI, int NJ>
-__global__ void __launch_bounds__(256, NJ == 4 ? 2 : 3) k_conv3x3(CnnConv a)
+__global__ void __launch_bounds__(256, NJ == 4 ? 2 : NJ == 2 ? 3 : 4) k_conv3x3(CnnConv a)
 {
     constexpr int FM = 4, TH = 16, TW = 16, HX = TW + 2, HP = HX * (TH + 2), BN = 16 * NJ;
     constexpr int NA = (HP * 4 + 255) / 256, NB = (36 * BN + 255) / 256;
     __shared__ __align__(16) uint16_t As[HP * kCvPitch];
     __shared__ __align__(16) uint16_t Bs[9 * BN * kCvPitch];
+    __shared__ __align__(16) float bias[BN];
     const int H = a.H, W = a.W, Cin = a.Cin, Cout = a.Cout;
     const int ntx = (W + TW - 1) / TW, nty = (H + TH - 1) / TH, ntiles = a.B * ntx * nty;
     const int co0 = blockIdx.y * BN;
@@ -227,14 +228,7 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 2 : 3) k_conv3x3(CnnConv a)
     };
     const uint16_t *al = As + (wv * FM * HX + (lane & 15)) * kCvPitch + 8 * (lane >> 4);
     const uint16_t *bl = Bs + (lane & 15) * kCvPitch + 8 * (lane >> 4);
-    f4v bias[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int co = co0 + 16 * j + 4 * (lane >> 4) + r;
-            bias[j][r] = a.bias && co < Cout ? a.bias[co] : 0.0f;
-        }
+    if (tid < BN) bias[tid] = a.bias && co0 + tid < Cout ? a.bias[co0 + tid] : 0.0f;
     bool weights = true;
     load(blockIdx.x, 0);
     load_weights(0);
@@ -243,7 +237,7 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 2 : 3) k_conv3x3(CnnConv a)
 #pragma unroll
         for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int i = 0; i < FM; i++) acc[j][i] = bias[j];
+            for (int i = 0; i < FM; i++) acc[j][i] = f4v{0.f, 0.f, 0.f, 0.f};
         for (int cc = 0; cc < ncc; cc++) {
             __syncthreads();  // the former chunk is multiplied out
             store(weights);
@@ -254,33 +248,39 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 2 : 3) k_conv3x3(CnnConv a)
                 load(nt, nc);
                 if (weights) load_weights(nc);
             }
+            bf8v px[FM][3], w[2][NJ];  // halo row r at px[r % FM]; tap t's weights at w[t % 2]
+            auto load_tap = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int dx = 0; dx < 3; dx++) {
-                if (NJ > 1) __builtin_amdgcn_sched_barrier(0);  // one column's weights in registers at a time: no spills
-                bf8v w[3][NJ];
+                for (int j = 0; j < NJ; j++) w[t % 2][j] = *(const bf8v *)(bl + (t * BN + 16 * j) * kCvPitch);
+            };
+            auto load_row = [&](int r) __attribute__((always_inline)) {
 #pragma unroll
-                for (int dy = 0; dy < 3; dy++)
+                for (int dx = 0; dx < 3; dx++) px[r % FM][dx] = *(const bf8v *)(al + (r * HX + dx) * kCvPitch);
+            };
+            load_tap(0);
+#pragma unroll
+            for (int r = 0; r < FM; r++) load_row(r);
+#pragma unroll
+            for (int t = 0; t < 9; t++) {
+                const int dy = t / 3, dx = t % 3;
+                if (t < 8) load_tap(t + 1);
+                __builtin_amdgcn_sched_barrier(0);  // the next tap's weights in registers, none beyond
+#pragma unroll
+                for (int i = 0; i < FM; i++)
 #pragma unroll
                     for (int j = 0; j < NJ; j++)
-                        w[dy][j] = *(const bf8v *)(bl + ((3 * dy + dx) * BN + 16 * j) * kCvPitch);
-#pragma unroll
-                for (int hr = 0; hr < FM + 2; hr++) {
-                    const bf8v px = *(const bf8v *)(al + (hr * HX + dx) * kCvPitch);
-#pragma unroll
-                    for (int dy = 0; dy < 3; dy++) {
-                        if (hr - dy < 0 || hr - dy >= FM) continue;
-#pragma unroll
-                        for (int j = 0; j < NJ; j++)
-                            acc[j][hr - dy] =
-                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dy][j], px, acc[j][hr - dy], 0, 0, 0);
-                    }
-                }
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t % 2][j], px[(i + dy) % FM][dx], acc[j][i], 0, 0, 0);
+                if (dx == 2 && dy < 2) load_row(dy + FM);
             }
         }
         const int img = tile / (ntx * nty), trem = tile - img * ntx * nty, ty = trem / ntx, tx = trem - ty * ntx;
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
+        for (int j = 0; j < NJ; j++) {
+            const f4v b = *(const f4v *)(bias + 16 * j + 4 * (lane >> 4));
+#pragma unroll
+            for (int i = 0; i < FM; i++) acc[j][i] += b;
             conv_epilogue<EPI>(a, acc[j], img, ty * TH + wv * FM, tx * TW + (lane & 15), co0 + 16 * j + 4 * (lane >> 4));
+        }
     }
 }
 

@@ -343,3 +343,25 @@ def test_network_block_widths_agree(base):
     assert abs(got[1][1] - got[0][1]) <= 1e-6 * got[0][1]
     # sums of 64 H W terms in FP32: eps times the root of their number
     assert rel_err(got[1][2], got[0][2]) <= 2e-5
+
+
+@pytest.mark.parametrize("Cin,Cout", [(32, 32), (32, 72), (96, 20), (64, 200)])
+def test_conv3x3_sums_in_a_fixed_order(Cin, Cout):
+    """Every block width adds up alike: chunks of 32 input channels, in each the taps row by row, the bias last.
+    Per output channel the terms are 1 but for one of 2^30 and a later one of -2^30, between which a 1 is lost and
+    after which none is: the sum counts the terms behind the second."""
+    print(f"conv3x3 order {Cin}->{Cout}", flush=True)
+    L, rng, B, H, W = cnn_lib(), np.random.default_rng([Cin, Cout]), 2, 90, 70
+    terms = [(t, 32 * k + int(rng.integers(32))) for k in range(Cin // 32) for t in range(9)]
+    Wt, b = np.zeros((Cout, 9, Cin), np.float32), rng.standard_normal(Cout).astype(np.float32)
+    want = np.zeros(Cout, np.float32)
+    for co in range(Cout):
+        first, second = sorted(rng.choice(len(terms), 2, replace=False))
+        for k, (t, ci) in enumerate(terms):
+            Wt[co, t, ci] = 2.0 ** 30 if k == first else -2.0 ** 30 if k == second else 1.0
+        want[co] = len(terms) - 1 - second + b[co]
+    dX, dW, db, dY = Raw(to_bf16(np.ones((B, H, W, Cin), np.float32))), Raw(to_bf16(Wt)), Raw(b), Raw(B * H * W * Cout * 4)
+    assert L.lfrv_op_conv3x3(B, H, W, Cin, Cout, dX.ptr, dW.ptr, db.ptr, dY.ptr, None) == 0
+    lfrv.device_sync()
+    inner = dY.get(np.float32, (B, H, W, Cout))[:, 1:-1, 1:-1]  # (where every term lies in the image)
+    assert np.array_equal(inner, np.broadcast_to(want, inner.shape))
