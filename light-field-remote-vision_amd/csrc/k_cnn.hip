@@ -158,20 +158,21 @@ __device__ __forceinline__ void conv_epilogue(const CnnConv &a, f4v (&v)[4], int
 // v[p][co] = sum_{t,ci} W[co][t][ci] X[p + off(t)][ci] + bias[co], then the epilogue EPI.
 // A block owns 16 x 16 pixels (a wave 4 rows of 16) and BN = 16 NJ output
 // channels.  Per chunk of 32 input channels the tile's 18 x 18 halo and the
-// weights of all 9 taps go to LDS once.  A wave reads each halo row once per
-// column offset and multiplies it with the (up to) three taps of that column,
-// whose weights it holds in registers: 18 + 9 NJ LDS reads for 36 NJ MFMAs
+// weights of all 9 taps go to LDS once.  The sums run by chunk, in a chunk by
+// tap in row order, and take the bias last, whatever NJ: in bf16 the network
+// amplifies a sum's last bit, so the order is part of the result.  A wave
+// holds the four halo rows that a row of taps meets, three operands each, and
+// a row of taps on replaces one of them: 18 + 9 NJ LDS reads for 36 NJ MFMAs
 // (reading per tap would be 36 + 9 NJ), so that NJ = 4 is bound by the matrix
 // units and not by LDS.  The weights are the MFMA's first operand, so a lane
 // ends with 4 consecutive channels of one pixel and stores them at once.  The
 // next chunk's (or tile's) loads are in flight while this one is multiplied; a
 // block runs through its tiles, and with 32 input channels keeps the weights.
 // With up, X is half the image's size and read as its 2x nearest upsampling.
-// One image of 1024 x 1024: the 15 layers 757 us (500 TFLOP/s) with what rides
-// on them, against 988 us and 382 us of pooling, upsampling and prediction
-// passes before; 8 of 256 x 256 forwards and backwards: the step 1.76 ms
-// against 2.92 (the masks, skips, fills and resamplings of the backward pass
-// took 0.75 ms).
+// One image of 1024 x 1024: the forward of 15 layers, with what rides on them,
+// 0.79 ms; 1.41 with pooling, upsampling and prediction as passes of their own;
+// 8 of 256 x 256 forwards and backwards: the step 1.71 ms against 5.66, of
+// which the weight gradient took 2.7.
 template <int EPI, int NJ>
 __global__ void __launch_bounds__(256, NJ == 4 ? 2 : NJ == 2 ? 3 : 4) k_conv3x3(CnnConv a)
 {
@@ -189,8 +190,16 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 2 : NJ == 2 ? 3 : 4) k_conv3x3(
     // loads always read a valid address; what lies outside is zeroed on its way to LDS
     u32x4 ar[NA], br[NB];
     unsigned amask = 0;
+    // (a value that the compiler does not see through: the staging's addresses are formed per chunk and not
+    // kept, or spilled, over the whole loop)
+    auto own_tid = [&]() {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        return t;
+    };
     auto load = [&](int tile, int cc) {
         const int img = tile / (ntx * nty), trem = tile - img * ntx * nty, ty = trem / ntx, tx = trem - ty * ntx;
+        const int tid = own_tid();
         amask = 0;
 #pragma unroll
         for (int j = 0; j < NA; j++) {
@@ -203,6 +212,7 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 2 : NJ == 2 ? 3 : 4) k_conv3x3(
         }
     };
     auto load_weights = [&](int cc) {
+        const int tid = own_tid();
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             const int idx = tid + 256 * j, t = idx / (4 * BN), r = (idx >> 2) - t * BN;
@@ -213,6 +223,7 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 2 : NJ == 2 ? 3 : 4) k_conv3x3(
     };
     const u32x4 z = {0u, 0u, 0u, 0u};
     auto store = [&](bool weights) {
+        const int tid = own_tid();
 #pragma unroll
         for (int j = 0; j < NA; j++) {
             const int idx = tid + 256 * j;
