@@ -956,6 +956,13 @@ DataTermArgs data_term_args(const lfrv_ctx *ctx)
     return da;
 }
 
+// The normalisation buffer that a step leaves the coverage in, as its data
+// terms do (optimization.cu:1835-2116): without either term it stays as it is.
+float *step_norm_mask(const lfrv_ctx *ctx)
+{
+    return ctx->p.dt_alpha > 0.0f || ctx->p.dt_beta > 0.0f ? ctx->norm_mask : nullptr;
+}
+
 // FISTA weights (optimization.cu:1744-1746): alpha_new is a cuflt (float)
 // there, theta the float of the double quotient.  Returns theta of the step
 // that starts at alpha; `an` receives alpha_new.
@@ -1143,7 +1150,7 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
             const float *gw = ctx->has_reg_g ? ctx->reg_g : nullptr;
             const StepBufs sb{ctx->U,    ctx->sr_ops, ctx->coverage, ctx->PX, ctx->PY, gw, ctx->P2X, ctx->P2Y, ctx->U2,
                               (inner == 1 && last) ? ctx->Uq : nullptr, inner > 1 ? ctx->G : nullptr,
-                              (inner > 1 || last) ? ctx->norm_mask : nullptr};
+                              (inner > 1 || last) ? step_norm_mask(ctx) : nullptr};
             if (sb.uq_relax || sb.gout || sb.norm_mask) STEP(true, true);
             else STEP(true, false);
             record_kernel_events(ctx, 3, ev);
@@ -1158,7 +1165,7 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
         } else {
             const PdArgs pa{};
             const StepBufs sb{ctx->U,  ctx->sr_ops, ctx->coverage, nullptr, nullptr, nullptr,       nullptr, nullptr,
-                              nullptr, ctx->Uq,     ctx->G,        ctx->norm_mask};
+                              nullptr, ctx->Uq,     ctx->G,        step_norm_mask(ctx)};
             STEP(false, true);
             record_kernel_events(ctx, 3, ev);
             LFRV_LAUNCH(ctx, "data term");
@@ -1253,7 +1260,7 @@ lfrv_status sr_batch_begin(lfrv_ctx *ctx, int steps, SrBatchItem *it, float *the
     it->PY[0] = ctx->PY;
     it->PY[1] = ctx->P2Y;
     it->uq = ctx->Uq;
-    it->norm_mask = ctx->norm_mask;
+    it->norm_mask = step_norm_mask(ctx);
     double a = ctx->fista_alpha;
     for (int k = 0; k < steps; k++) {
         float an;

@@ -6,6 +6,7 @@ import pytest
 import lfrv
 import oracle
 from lfrv import pipelines
+from lfrv.batch import Batch
 from conftest import rel_err
 
 pytestmark = pytest.mark.gpu
@@ -192,3 +193,28 @@ def test_pd_passes_at_strip_edges(w, h, dsf, inner):
     d.grid, d.w, d.h, d.dsf, d.render_scale = 3, w, h, dsf, dsf
     d.focal, d.baseline = float(w), 0.7 * 4.0 / (w * dsf)
     _steps_match_oracle(lfrv.synth(d), 0.3, 0, inner, metas=1, steps=2)
+
+
+@pytest.mark.parametrize("dsf,inner", [(1, 1), (2, 1), (2, 0), (2, 3), (4, 1)])
+def test_step_without_data_terms_keeps_the_norm_mask(dsf, inner):
+    """dt_alpha = dt_beta = 0: no data term runs, so the normalisation buffer stays, in single steps, in a fixed run
+    and in a batch (whose set-up leaves the mask that the same calls leave here)."""
+    s = _scene(dsf=dsf, kind=2 if dsf == 1 else 1)
+    print(f"norm mask without data terms dsf={dsf} inner={inner}", flush=True)
+    prm = pipelines.color_sr_params(s, inner_iterations=inner, dt_alpha=0.0, dt_beta=0.0)
+    with lfrv.Context(prm) as ctx, lfrv.Context(prm) as other:
+        for c in (ctx, other):
+            pipelines.load_scene(c, s)
+        pipelines.color_sr_setup(ctx)
+        ctx.sr_init_regularizer_weight()
+        before = ctx.get_buffer("NORM_MASK")
+        assert rel_err(before, ctx.get_buffer("COVERAGE")) > 0.1
+        ctx.sr_iteration_fista()
+        ctx.sr_iterate(3)
+        assert np.array_equal(ctx.get_buffer("NORM_MASK"), before)
+        b = Batch()
+        b.add_pd(other, 4)
+        b.run()
+        b.close()
+        assert np.array_equal(other.get_buffer("NORM_MASK"), before)
+        assert np.array_equal(other.get_solution(), ctx.get_solution())
