@@ -299,7 +299,7 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
     const float n_inner = xin ? nx + 2.0f : 1.0f, n_edge = xin ? nx + (H > 1 ? 1.0f : 0.0f) : 1.0f;
     const float ci = dt_intensity_weight(da), cgd = dt_gradient_weight(da) * da.dsf2;
     const Divisor vden(pa.tau + pa.lam);
-    const float sgx = xin && x < W - 1 ? pa.sigma : 0.0f;
+    const bool has_right = xin && x < W - 1;
     const float gnone = sb.g ? 0.0f : 1.0f;  // the TV weight where there is no map
     const Planes<WIDE> bU(sb.U, 3, N, W), bC(sb.ops, 5, NA, Wc), bB(sb.ops + 5 * NA, 3, NA, Wc),
         bE(da.gw_type ? sb.ops : sb.ops + 8 * NA, GRAD ? 5 : 0, NA, Wc), bPx(sb.px, 3, N, W), bPy(sb.py, 3, N, W),
@@ -381,7 +381,7 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         // row sums of U and lap U at row yb, BU and BL of the anchor row yb
         float bp[1 + G][3][3];
         // (+: of the values; a choice between the captured variables would keep them all in memory)
-        const Divisor nn4(GRAD ? (yb > 0 && yb < H - 1 ? +n_inner : +n_edge) : 1.0f);
+        const Divisor nn4(GRAD ? (yb > 0 && yb < H - 1 ? +n_inner : +n_edge) : 1.0f, 1.0f);
         const bool bin = xin && yb >= 0 && yb < H;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -437,12 +437,13 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
         if constexpr (PD && ph >= 2) {
             // the duals (vtv_rof.cu:118-147, 280-321)
-            const float sgy = yo < H - 1 ? pa.sigma : 0.0f;
+            const bool has_below = yo >= 0 && yo < H - 1;
             float nn = 0.0f;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                a[c] = fmaf(sgx, from_right(up[c]) - up[c], l.p[c]);
-                b[c] = fmaf(sgy, u[(ko + 1) % RING][c] - up[c], l.p[3 + c]);
+                const float gx = from_right(up[c]) - up[c], gy = u[(ko + 1) % RING][c] - up[c];
+                a[c] = fmaf(pa.sigma, has_right ? gx : 0.0f, l.p[c]);
+                b[c] = fmaf(pa.sigma, has_below ? gy : 0.0f, l.p[3 + c]);
                 nn += fmaf(a[c], a[c], b[c] * b[c]);
             }
             nn = sqrtf(nn);
@@ -483,7 +484,7 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         }
         if constexpr (PD && ph >= 2) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) py1[c] = ph == 3 || yo >= 0 ? b[c] : 0.0f;
+            for (int c = 0; c < 3; c++) py1[c] = b[c];
         }
 #pragma unroll
         for (int t = 0; t <= G; t++) {
@@ -599,7 +600,7 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
     const bool xin = x >= 0 && x < W;
     const int vx = xin ? 4 * x : kOutside, vs = lane >= K && lane < 64 - K ? vx : kOutside;
     const Divisor vden(pa.tau + pa.lam);
-    const float sgx = xin && x < W - 1 ? pa.sigma : 0.0f;
+    const bool has_right = xin && x < W - 1;
     const float gnone = pb.g ? 0.0f : 1.0f;
     const Planes<WIDE> bU(pb.uin, 3, N, W), bPx(pb.px, 3, N, W), bPy(pb.py, 3, N, W), bF(pb.F, 3, N, W), bG(pb.g, 1, N, W),
         bUo(pb.uout, 3, N, W), bPxo(pb.pxout, 3, N, W), bPyo(pb.pyout, 3, N, W), bUf(pb.u_final, 3, N, W);
@@ -647,7 +648,7 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
         for (int j = 0; j < K; j++) {
             const int y = yn - 1 - j;  // the row this iteration completes
             const bool yin = y >= 0 && y < H;
-            const float sgy = y < H - 1 ? pa.sigma : 0.0f;
+            const bool has_below = y >= 0 && y < H - 1;
             if (j > 0) {
                 // what came from iteration j - 1 is for the next turn
                 const float tg = g[j];
@@ -669,13 +670,13 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
             float nn = 0.0f;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                cp[c] = fmaf(sgx, from_right(u[j][c]) - u[j][c], cp[c]);
-                cp[3 + c] = fmaf(sgy, un[c] - u[j][c], cp[3 + c]);
+                const float gx = from_right(u[j][c]) - u[j][c], gy = un[c] - u[j][c];
+                cp[c] = fmaf(pa.sigma, has_right ? gx : 0.0f, cp[c]);
+                cp[3 + c] = fmaf(pa.sigma, has_below ? gy : 0.0f, cp[3 + c]);
                 nn += fmaf(cp[c], cp[c], cp[3 + c] * cp[3 + c]);
             }
             nn = sqrtf(nn);
-            const float ratio = cg / nn, in = nn > cg ? ratio : 1.0f;
-            const float sc = yin ? +in : 0.0f;  // (no duals outside the image; left and right of it all they read is 0)
+            const float ratio = cg / nn, sc = nn > cg ? ratio : 1.0f;  // (outside the image the duals read and stay 0)
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 cp[c] *= sc;

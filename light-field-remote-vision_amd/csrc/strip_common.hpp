@@ -66,20 +66,29 @@ struct Planes {
     }
 };
 
-// n / d for finite values away from the ends of the range, correctly rounded:
-// a Newton step for the reciprocal, which several quotients of one divisor
-// share, then two for the quotient.
+// n / d, correctly rounded but for quotients and dividends within some 2^24 of
+// the smallest normal number (an ulp there): a Newton step for the reciprocal,
+// which several quotients of one divisor share, then two for the quotient.
+// Divisors away from 1 are brought there by a power of two, and the fix-up
+// gives what division gives for zeros, infinities and NaN.
 struct Divisor {
-    float d, r;
-    __device__ __forceinline__ explicit Divisor(float div) : d(div), r(__builtin_amdgcn_rcpf(div))
+    float d, r, scale;
+    __device__ __forceinline__ explicit Divisor(float div)
+        : Divisor(div, fabsf(div) < 0x1p-64f ? 0x1p64f : fabsf(div) > 0x1p64f ? 0x1p-64f : 1.0f)
     {
+    }
+    // a divisor between 2^-64 and 2^64: scale 1
+    __device__ __forceinline__ Divisor(float div, float sc) : d(div * sc), scale(sc)
+    {
+        r = __builtin_amdgcn_rcpf(d);
         r = fmaf(fmaf(-d, r, 1.0f), r, r);
     }
     __device__ __forceinline__ float of(float n) const
     {
+        n *= scale;
         float q = n * r;
         q = fmaf(fmaf(-d, q, n), r, q);
-        return fmaf(fmaf(-d, q, n), r, q);
+        return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
     }
 };
 

@@ -218,3 +218,61 @@ def test_step_without_data_terms_keeps_the_norm_mask(dsf, inner):
         b.close()
         assert np.array_equal(other.get_buffer("NORM_MASK"), before)
         assert np.array_equal(other.get_solution(), ctx.get_solution())
+
+
+def _step_from_buffers(ctx, s, U0, alpha, beta, inner):
+    """One step of the oracle from the context's own warps, weights and duals and the solution U0."""
+    V, w, h, W, H = s["V"], s["w"], s["h"], s["W"], s["H"]
+    tx, ty, om = [ctx.get_buffer(k).reshape(V, h, w) for k in ("TAU_X", "TAU_Y", "OMEGA")]
+    st = oracle.SrState(W, H, U0)
+    st.PX[:], st.PY[:] = [ctx.get_buffer(k).reshape(3, H, W) for k in ("PX", "PY")]
+    with np.errstate(all="ignore"):
+        oracle.fista_step(W, H, s["dsf"], tx, ty, s["views"], om, 1 / 255.0, alpha, beta, 1.0, 0, 0.05, inner,
+                          ctx.get_buffer("REG_G").reshape(H, W), st)
+    return st
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf])
+@pytest.mark.parametrize("dsf,inner", [(2, 1), (2, 3), (3, 0), (4, 1)])
+def test_step_with_an_infinite_view_pixel(dsf, inner, value):
+    """An infinite view pixel makes its target pixels' gradient infinite: the clamp takes it to +-1, not to NaN."""
+    s = _scene(dsf=dsf)
+    s["views"] = s["views"].copy()
+    s["views"][0, :, 20, 17] = value  # (a corner camera: its footprints have no weight of 0, whose product is NaN)
+    print(f"infinite view pixel {value} dsf={dsf} inner={inner}", flush=True)
+    with lfrv.Context(pipelines.color_sr_params(s, inner_iterations=inner)) as ctx:
+        pipelines.load_scene(ctx, s)
+        pipelines.color_sr_setup(ctx)
+        U0 = np.random.default_rng(dsf).uniform(0.2, 0.8, (3, s["H"], s["W"])).astype(np.float32)
+        ctx.set_solution(U0)
+        ctx.sr_init_regularizer_weight()
+        st = _step_from_buffers(ctx, s, U0, 1.0, 0.0, inner)
+        ctx.sr_iteration_fista()
+        key = "G" if inner == 0 else "U"
+        got, want = ctx.get_buffer(key).reshape(U0.shape), st.G if inner == 0 else st.U
+        assert np.all(np.isfinite(want)) and np.max(np.abs(got - want)) < 1e-4
+
+
+@pytest.mark.parametrize("dsf,inner", [(1, 1), (1, 4), (2, 1), (2, 2), (4, 1)])
+@pytest.mark.parametrize("at", ["right", "bottom", "corner", "left", "top"])
+def test_duals_beside_an_infinite_pixel(dsf, inner, at):
+    """Forward differences end at the image's edge: an infinite pixel there is not multiplied by a weight of 0, and
+    what is not a number is so in the same places as in the oracle."""
+    s = _scene(dsf=dsf, kind=2 if dsf == 1 else 1)
+    H, W = s["H"], s["W"]
+    y, x = {"right": (9, W - 1), "bottom": (H - 1, 9), "corner": (H - 1, W - 1), "left": (9, 0), "top": (0, 9)}[at]
+    print(f"infinite solution pixel {y},{x} dsf={dsf} inner={inner}", flush=True)
+    with lfrv.Context(pipelines.color_sr_params(s, inner_iterations=inner, dt_alpha=0.0)) as ctx:
+        pipelines.load_scene(ctx, s)
+        pipelines.color_sr_setup(ctx)
+        U0 = np.random.default_rng(dsf).uniform(0.2, 0.8, (3, H, W)).astype(np.float32)
+        U0[1, y, x] = np.inf
+        ctx.set_solution(U0)
+        ctx.sr_init_regularizer_weight()
+        st = _step_from_buffers(ctx, s, U0, 0.0, 0.0, inner)
+        ctx.sr_iteration_fista()
+        for key, want in (("U", st.U), ("PX", st.PX), ("PY", st.PY)):
+            got = ctx.get_buffer(key).reshape(want.shape)
+            assert np.array_equal(np.isfinite(got), np.isfinite(want)), key
+            ok = np.isfinite(want)
+            assert np.max(np.abs(got[ok] - want[ok])) < 1e-4, key
