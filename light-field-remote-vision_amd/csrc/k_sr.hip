@@ -299,7 +299,8 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
     const float n_inner = xin ? nx + 2.0f : 1.0f, n_edge = xin ? nx + (H > 1 ? 1.0f : 0.0f) : 1.0f;
     const float ci = dt_intensity_weight(da), cgd = dt_gradient_weight(da) * da.dsf2;
     const Divisor vden(pa.tau + pa.lam);
-    const bool has_right = xin && x < W - 1;
+    const float vtau = pa.tau * vden.scale, vlam = pa.lam * vden.scale;
+    const int has_right = lane_mask(xin && x < W - 1);
     const float gnone = sb.g ? 0.0f : 1.0f;  // the TV weight where there is no map
     const Planes<WIDE> bU(sb.U, 3, N, W), bC(sb.ops, 5, NA, Wc), bB(sb.ops + 5 * NA, 3, NA, Wc),
         bE(da.gw_type ? sb.ops : sb.ops + 8 * NA, GRAD ? 5 : 0, NA, Wc), bPx(sb.px, 3, N, W), bPy(sb.py, 3, N, W),
@@ -437,13 +438,13 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
         if constexpr (PD && ph >= 2) {
             // the duals (vtv_rof.cu:118-147, 280-321)
-            const bool has_below = yo >= 0 && yo < H - 1;
+            const int has_below = row_mask(yo >= 0 && yo < H - 1);
             float nn = 0.0f;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 const float gx = from_right(up[c]) - up[c], gy = u[(ko + 1) % RING][c] - up[c];
-                a[c] = fmaf(pa.sigma, has_right ? gx : 0.0f, l.p[c]);
-                b[c] = fmaf(pa.sigma, has_below ? gy : 0.0f, l.p[3 + c]);
+                a[c] = fmaf(pa.sigma, where(has_right, gx), l.p[c]);
+                b[c] = fmaf(pa.sigma, where(has_below, gy), l.p[3 + c]);
                 nn += fmaf(a[c], a[c], b[c] * b[c]);
             }
             nn = sqrtf(nn);
@@ -469,7 +470,7 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
                     // (left of the image U and the duals read 0)
                     const float step = a[c] + b[c] - from_left(a[c]) - py1[c];
                     const float un = fmaf(pa.tau, step, up[c]);
-                    const float v = vden.of(fmaf(pa.tau, F, pa.lam * un));
+                    const float v = vden.of_scaled(fmaf(vtau, F, vlam * un));
                     rel = fmaf(pa.theta, v - up[c], up[c]);
                     bPxo.store(a[c], c, yo, vo);
                     bPyo.store(b[c], c, yo, vo);
@@ -600,7 +601,8 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
     const bool xin = x >= 0 && x < W;
     const int vx = xin ? 4 * x : kOutside, vs = lane >= K && lane < 64 - K ? vx : kOutside;
     const Divisor vden(pa.tau + pa.lam);
-    const bool has_right = xin && x < W - 1;
+    const float vtau = pa.tau * vden.scale, vlam = pa.lam * vden.scale;
+    const int has_right = lane_mask(xin && x < W - 1);
     const float gnone = pb.g ? 0.0f : 1.0f;
     const Planes<WIDE> bU(pb.uin, 3, N, W), bPx(pb.px, 3, N, W), bPy(pb.py, 3, N, W), bF(pb.F, 3, N, W), bG(pb.g, 1, N, W),
         bUo(pb.uout, 3, N, W), bPxo(pb.pxout, 3, N, W), bPyo(pb.pyout, 3, N, W), bUf(pb.u_final, 3, N, W);
@@ -648,7 +650,7 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
         for (int j = 0; j < K; j++) {
             const int y = yn - 1 - j;  // the row this iteration completes
             const bool yin = y >= 0 && y < H;
-            const bool has_below = y >= 0 && y < H - 1;
+            const int has_below = row_mask(y >= 0 && y < H - 1);
             if (j > 0) {
                 // what came from iteration j - 1 is for the next turn
                 const float tg = g[j];
@@ -671,8 +673,8 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 const float gx = from_right(u[j][c]) - u[j][c], gy = un[c] - u[j][c];
-                cp[c] = fmaf(pa.sigma, has_right ? gx : 0.0f, cp[c]);
-                cp[3 + c] = fmaf(pa.sigma, has_below ? gy : 0.0f, cp[3 + c]);
+                cp[c] = fmaf(pa.sigma, where(has_right, gx), cp[c]);
+                cp[3 + c] = fmaf(pa.sigma, where(has_below, gy), cp[3 + c]);
                 nn += fmaf(cp[c], cp[c], cp[3 + c] * cp[3 + c]);
             }
             nn = sqrtf(nn);
@@ -682,7 +684,7 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
                 cp[c] *= sc;
                 cp[3 + c] *= sc;
                 const float step = cp[c] + cp[3 + c] - from_left(cp[c]) - py[j][c];
-                const float v = vden.of(fmaf(pa.tau, cF[c], pa.lam * fmaf(pa.tau, step, u[j][c])));
+                const float v = vden.of_scaled(fmaf(vtau, cF[c], vlam * fmaf(pa.tau, step, u[j][c])));
                 py[j][c] = cp[3 + c];
                 u[j][c] = un[c];
                 un[c] = xin && yin ? +v : 0.0f;

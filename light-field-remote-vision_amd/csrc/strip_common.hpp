@@ -32,6 +32,22 @@ __device__ __forceinline__ float from_right(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));  // wave_shl:1
 }
 
+// v where the mask is -1, and 0, whatever v, where it is 0.  A mask is one register where a condition is a pair of
+// the scalar ones, of which the strips have none to spare; the compiler is kept from seeing the condition in it.
+__device__ __forceinline__ float where(int mask, float v) { return __int_as_float(__float_as_int(v) & mask); }
+__device__ __forceinline__ int lane_mask(bool in)
+{
+    int m = in ? -1 : 0;
+    asm("" : "+v"(m));
+    return m;
+}
+__device__ __forceinline__ int row_mask(bool in)  // (of a condition that all lanes share)
+{
+    int m = __builtin_amdgcn_readfirstlane(in ? -1 : 0);
+    asm("" : "+s"(m));
+    return m;
+}
+
 constexpr int kOutside = (int)0x80000000;
 constexpr size_t kNarrowBytes = (size_t)1 << 31;  // kOutside lies past any buffer up to this size
 
@@ -83,9 +99,10 @@ struct Divisor {
         r = __builtin_amdgcn_rcpf(d);
         r = fmaf(fmaf(-d, r, 1.0f), r, r);
     }
-    __device__ __forceinline__ float of(float n) const
+    __device__ __forceinline__ float of(float n) const { return of_scaled(n * scale); }
+    // n times the scale comes from the caller
+    __device__ __forceinline__ float of_scaled(float n) const
     {
-        n *= scale;
         float q = n * r;
         q = fmaf(fmaf(-d, q, n), r, q);
         return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
