@@ -451,8 +451,8 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
             const float gr = l.g + gnone, ratio = gr / nn, sc = nn > gr ? ratio : 1.0f;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                a[c] *= sc;
-                b[c] *= sc;
+                a[c] = product(a[c], sc);
+                b[c] = product(b[c], sc);
             }
         }
         if constexpr (ph == 3) {
@@ -681,8 +681,8 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
             const float ratio = cg / nn, sc = nn > cg ? ratio : 1.0f;  // (outside the image the duals read and stay 0)
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                cp[c] *= sc;
-                cp[3 + c] *= sc;
+                cp[c] = product(cp[c], sc);
+                cp[3 + c] = product(cp[3 + c], sc);
                 const float step = cp[c] + cp[3 + c] - from_left(cp[c]) - py[j][c];
                 const float v = vden.of_scaled(fmaf(vtau, cF[c], vlam * fmaf(pa.tau, step, u[j][c])));
                 py[j][c] = cp[3 + c];

@@ -48,6 +48,14 @@ __device__ __forceinline__ int row_mask(bool in)  // (of a condition that all la
     return m;
 }
 
+// a b, rounded: not to be contracted with a sum that it goes into (where the product is also stored, the sum is of
+// what is stored).
+__device__ __forceinline__ float product(float a, float b)
+{
+#pragma clang fp contract(off)
+    return a * b;
+}
+
 constexpr int kOutside = (int)0x80000000;
 constexpr size_t kNarrowBytes = (size_t)1 << 31;  // kOutside lies past any buffer up to this size
 

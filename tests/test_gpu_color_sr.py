@@ -276,3 +276,43 @@ def test_duals_beside_an_infinite_pixel(dsf, inner, at):
             assert np.array_equal(np.isfinite(got), np.isfinite(want)), key
             ok = np.isfinite(want)
             assert np.max(np.abs(got[ok] - want[ok])) < 1e-4, key
+
+
+def _fma(a, b, c):
+    """a b + c of FP32 values, rounded once."""
+    return np.float32(np.longdouble(a) * np.longdouble(b) + np.longdouble(c))
+
+
+@pytest.mark.parametrize("dsf,inner", [(1, 1), (1, 4), (2, 1), (2, 3), (4, 1)])
+def test_primal_is_formed_from_the_stored_duals(dsf, inner):
+    """Where the projection scales the duals, the divergence is that of the rounded duals, as they are two passes in
+    the reference: the last iteration's primal restated operation by operation, bit for bit."""
+    s = _scene(dsf=dsf, kind=2 if dsf == 1 else 1)
+    H, W = s["H"], s["W"]
+    print(f"primal from the stored duals dsf={dsf} inner={inner}", flush=True)
+    rng = np.random.default_rng(dsf)
+    U0 = rng.uniform(0.2, 0.8, (3, H, W)).astype(np.float32)
+    P0 = rng.uniform(-0.5, 0.5, (2, 3, H, W)).astype(np.float32)
+
+    def step(iterations):  # (without data terms F is the solution itself)
+        with lfrv.Context(pipelines.color_sr_params(s, inner_iterations=iterations, dt_alpha=0.0)) as ctx:
+            pipelines.load_scene(ctx, s)
+            pipelines.color_sr_setup(ctx)
+            ctx.sr_init_regularizer_weight()
+            ctx.set_buffer("REG_G", np.full((H, W), 0.3, np.float32))
+            ctx.set_buffer("PX", P0[0])
+            ctx.set_buffer("PY", P0[1])
+            ctx.set_solution(U0)
+            ctx.sr_iteration_fista()
+            return [ctx.get_buffer(b).reshape(3, H, W) for b in ("U", "PX", "PY")]
+
+    U, px, py = step(inner)
+    before = step(inner - 1)[0] if inner > 1 else U0
+    length = np.sqrt((px.astype(np.float64) ** 2 + py.astype(np.float64) ** 2).sum(0))
+    assert length.max() < 0.3 * (1 + 1e-6) and (length > 0.299).mean() > 0.1
+    left, up = np.zeros_like(px), np.zeros_like(py)
+    left[..., 1:], up[..., 1:, :] = px[..., :-1], py[..., :-1, :]
+    tau, lam = np.float32(0.3 / np.sqrt(8.0)), np.float32(0.05)
+    lam = np.float32(1 / np.float64(np.float32(1 / np.float64(lam))))
+    un = _fma(tau, px + py - left - up, before)
+    assert np.array_equal(U, _fma(tau, U0, lam * un) / (tau + lam))
