@@ -297,6 +297,7 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
     // inside the image, on inner and on edge rows
     const float nx = (x > 0 ? 1.0f : 0.0f) + (x < W - 1 ? 1.0f : 0.0f);
     const float n_inner = xin ? nx + 2.0f : 1.0f, n_edge = xin ? nx + (H > 1 ? 1.0f : 0.0f) : 1.0f;
+    const float r_inner = 1.0f / n_inner, r_edge = 1.0f / n_edge;
     const float ci = dt_intensity_weight(da), cgd = dt_gradient_weight(da) * da.dsf2;
     const Divisor vden(pa.tau + pa.lam);
     const float vtau = pa.tau * vden.scale, vlam = pa.lam * vden.scale;
@@ -382,14 +383,15 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         // row sums of U and lap U at row yb, BU and BL of the anchor row yb
         float bp[1 + G][3][3];
         // (+: of the values; a choice between the captured variables would keep them all in memory)
-        const Divisor nn4(GRAD ? (yb > 0 && yb < H - 1 ? +n_inner : +n_edge) : 1.0f, 1.0f);
+        const bool inner = yb > 0 && yb < H - 1;
+        const float n4 = inner ? +n_inner : +n_edge, r4 = inner ? +r_inner : +r_edge;
         const bool bin = xin && yb >= 0 && yb < H;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const float uc = GRAD ? u[k1][c] : u[ku][c];
             if constexpr (GRAD) {
                 const float sum = ((from_left(uc) + u[k2][c]) + from_right(uc)) + u[ku][c];
-                float t = nn4.of(sum) - uc;
+                float t = small_quotient(sum, n4, r4) - uc;
                 t = bin ? t : 0.0f;
                 float rs = t;
 #pragma unroll
@@ -438,7 +440,7 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
         if constexpr (PD && ph >= 2) {
             // the duals (vtv_rof.cu:118-147, 280-321)
-            const int has_below = row_mask(yo >= 0 && yo < H - 1);
+            const int has_below = mask_below(yo, H - 1);
             float nn = 0.0f;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
@@ -458,10 +460,20 @@ __device__ __forceinline__ void sr_strip(int x0, int y0, int y1, int W, int H, i
         if constexpr (ph == 3) {
             // the step of vtv_sr_ista_step_unstructured, and the primal (cuda_kernels.cu:504-532)
             const int vo = yo < y1 ? vs : kOutside;
-            const Divisor cov(l.cov != 0.0f ? l.cov : 1.0f);
+            // (a lane with a coverage that a division would have to scale is rare: the wave divides then)
+            const float cov = l.cov != 0.0f ? l.cov : 1.0f;
+            float quot[3];
+            if (__all(Divisor::plain(cov))) {
+                const Divisor by(cov, 1.0f);
+#pragma unroll
+                for (int c = 0; c < 3; c++) quot[c] = by.of_scaled(acc[c]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 3; c++) quot[c] = acc[c] / cov;
+            }
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                float Gv = cov.of(acc[c]);
+                float Gv = quot[c];
                 if constexpr (!GRAD) Gv = da.alpha > 0.0f ? da.alpha * (Gv * da.sigma2) : 0.0f;
                 Gv = fminf(1.0f, fmaxf(-1.0f, Gv));
                 const float F = fminf(1.0f, fmaxf(0.0f, fmaf(Gv, da.prox_factor, up[c])));
@@ -650,7 +662,7 @@ __device__ __forceinline__ void pd_strip(int x0, int y0, int y1, int W, int H, c
         for (int j = 0; j < K; j++) {
             const int y = yn - 1 - j;  // the row this iteration completes
             const bool yin = y >= 0 && y < H;
-            const int has_below = row_mask(y >= 0 && y < H - 1);
+            const int has_below = mask_below(y, H - 1);
             if (j > 0) {
                 // what came from iteration j - 1 is for the next turn
                 const float tg = g[j];

@@ -41,12 +41,7 @@ __device__ __forceinline__ int lane_mask(bool in)
     asm("" : "+v"(m));
     return m;
 }
-__device__ __forceinline__ int row_mask(bool in)  // (of a condition that all lanes share)
-{
-    int m = __builtin_amdgcn_readfirstlane(in ? -1 : 0);
-    asm("" : "+s"(m));
-    return m;
-}
+__device__ __forceinline__ int mask_below(int y, int end) { return (~y & (y - end)) >> 31; }  // of 0 <= y < end
 
 // a b, rounded: not to be contracted with a sum that it goes into (where the product is also stored, the sum is of
 // what is stored).
@@ -101,14 +96,17 @@ struct Divisor {
         : Divisor(div, fabsf(div) < 0x1p-64f ? 0x1p64f : fabsf(div) > 0x1p64f ? 0x1p-64f : 1.0f)
     {
     }
-    // a divisor between 2^-64 and 2^64: scale 1
     __device__ __forceinline__ Divisor(float div, float sc) : d(div * sc), scale(sc)
     {
         r = __builtin_amdgcn_rcpf(d);
         r = fmaf(fmaf(-d, r, 1.0f), r, r);
     }
-    __device__ __forceinline__ float of(float n) const { return of_scaled(n * scale); }
-    // n times the scale comes from the caller
+    // whether a divisor can go without a scale: between 2^-126 and 2^125
+    __device__ __forceinline__ static bool plain(float div)
+    {
+        return (unsigned)(__float_as_int(div) - 0x00800000) < 0x7d800000u;
+    }
+    // the quotient of n / scale (which the caller knows to be 1, or has multiplied into n)
     __device__ __forceinline__ float of_scaled(float n) const
     {
         float q = n * r;
@@ -116,5 +114,13 @@ struct Divisor {
         return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
     }
 };
+
+// n / d for d = 1, 2, 3 or 4 and r = 1 / d: with a rounded reciprocal one correction rounds the quotient (checked for
+// every mantissa of n, for n above 2^-102).
+__device__ __forceinline__ float small_quotient(float n, float d, float r)
+{
+    const float q = n * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
+}
 
 }  // namespace lfrv

@@ -316,3 +316,38 @@ def test_primal_is_formed_from_the_stored_duals(dsf, inner):
     lam = np.float32(1 / np.float64(np.float32(1 / np.float64(lam))))
     un = _fma(tau, px + py - left - up, before)
     assert np.array_equal(U, _fma(tau, U0, lam * un) / (tau + lam))
+
+
+@pytest.mark.parametrize("dsf,beta", [(2, 0.0), (3, 0.3), (4, 0.3)])
+def test_step_with_coverages_that_need_a_division(dsf, beta):
+    """A few coverages beyond the range of the shared reciprocal: their waves divide, with the same bits for the
+    ordinary pixels, and theirs are what division gives."""
+    s = _scene(dsf=dsf)
+    H, W = s["H"], s["W"]
+    print(f"extreme coverages dsf={dsf} beta={beta}", flush=True)
+    at = {(3, 5): 1e-40, (20, 30): -0.5, (21, 31): 3e38, (40, 7): np.inf, (H - 1, W - 1): 2e-39, (H - 9, 0): 0.0}
+    U0 = np.random.default_rng(dsf).uniform(0.2, 0.8, (3, H, W)).astype(np.float32)
+    F = []
+    for special in (False, True):
+        with lfrv.Context(pipelines.color_sr_params(s, inner_iterations=0, dt_beta=beta, gradient_step=1.0)) as ctx:
+            pipelines.load_scene(ctx, s)
+            pipelines.color_sr_setup(ctx)
+            cov = ctx.get_buffer("COVERAGE").reshape(H, W).copy()
+            for p, v in at.items():
+                cov[p] = v if special else 1.0
+            ctx.set_buffer("COVERAGE", cov)
+            ctx.set_solution(U0)
+            ctx.sr_iteration_fista()
+            F.append(ctx.get_buffer("G").reshape(3, H, W))
+    rest = np.ones((H, W), bool)
+    for (y, x), v in at.items():
+        rest[y, x] = False
+        step = F[0][:, y, x] - U0[:, y, x]  # minus the clamped gradient at a coverage of 1
+        assert np.all(step != 0)
+        want = {1e-40: np.where(step > 0, 1, 0), 2e-39: np.where(step > 0, 1, 0), 3e38: U0[:, y, x], np.inf: U0[:, y, x],
+                0.0: F[0][:, y, x]}.get(v)
+        if want is not None:
+            assert np.array_equal(F[1][:, y, x], want.astype(np.float32)), v
+        else:
+            assert np.all(np.sign(F[1][:, y, x] - U0[:, y, x]) == -np.sign(step))
+    assert np.array_equal(F[0][:, rest], F[1][:, rest])
