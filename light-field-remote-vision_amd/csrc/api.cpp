@@ -669,6 +669,9 @@ extern "C" lfrv_status lfrv_set_buffer(lfrv_ctx *ctx, int which, const float *in
     return LFRV_OK;
 }
 
+// For tests alone (not in the header): from how many bytes on the marching strips address planes row by row.
+extern "C" void lfrv_test_narrow_bytes(lfrv_ctx *ctx, size_t bytes) { ctx->narrow_bytes = bytes; }
+
 extern "C" lfrv_status lfrv_set_timing(lfrv_ctx *ctx, int enable)
 {
     if (!ctx) return LFRV_E_ARG;

@@ -1576,7 +1576,7 @@ lfrv_status run_cg(lfrv_ctx *ctx, double alpha, double c0, double beta, bool use
         float *wbuf[2] = {ctx->cg_q, ctx->cg_extra + 6 * N};
         const StripSize size{ctx->W, ctx->H};
         const StripGeom sg = strips(ctx->ks - 1, size, strip_rows(ctx->ks - 1, &size, 1));
-        const bool wide = 20 * NA >= kNarrowBytes;
+        const bool wide = strip_wide(5, Wc, Hc, ctx->narrow_bytes);
         if ((size_t)sg.nblocks * 9 > ctx->partials_cap) return fail(ctx, LFRV_E_STATE, "partials buffer too small");
         auto box_poll = [&]() -> lfrv_status {
             {

@@ -1031,7 +1031,10 @@ lfrv_status ensure_sr_ops(lfrv_ctx *ctx)
 }
 
 // Whether the step's planes outgrow one buffer descriptor (the five planes of a coupling set are the largest).
-bool sr_wide(int Wc, int Hc) { return 20 * (size_t)Wc * Hc >= kNarrowBytes; }
+bool sr_wide(const lfrv_ctx *ctx)
+{
+    return strip_wide(5, ctx->W + ctx->ks - 1, ctx->H + ctx->ks - 1, ctx->narrow_bytes);
+}
 
 }  // namespace
 
@@ -1077,7 +1080,7 @@ lfrv_status run_pd_steps(lfrv_ctx *ctx, int iters, const float *F, bool overrela
     const StripSize size{ctx->W, ctx->H};
     PdArgs pa = pd_args(ctx);
     pa.theta = theta;
-    const bool wide = 12 * (size_t)ctx->W * ctx->H >= kNarrowBytes;
+    const bool wide = strip_wide(3, ctx->W, ctx->H, ctx->narrow_bytes);
     int left = iters;
     for (int passes = (iters + 3) / 4; passes > 0; passes--) {
         const int k = (left + passes - 1) / passes;
@@ -1148,7 +1151,7 @@ lfrv_status enqueue_fista(lfrv_ctx *ctx, const int *halt, bool last = true)
         const StripGeom sg = strips(sr_lag(ctx->ks, grad), size, strip_rows(sr_lag(ctx->ks, grad), &size, 1));
         const KernelEvents ev = kernel_events(ctx, 3);  // stamped by the dispatch itself
 #define STEP2(K, GR, PD, EX, WI) hipExtLaunchKernelGGL(k_sr_step_st<K, GR, PD, EX, WI>, dim3(sg.nblocks), dim3(256), 0, ctx->stream, ev.a, ev.b, 0, ctx->W, ctx->H, Wc, Hc, sg, da, pa, NA, sb, halt)
-#define STEP1(K, GR, PD, EX) do { if (sr_wide(Wc, Hc)) STEP2(K, GR, PD, EX, true); else STEP2(K, GR, PD, EX, false); } while (0)
+#define STEP1(K, GR, PD, EX) do { if (sr_wide(ctx)) STEP2(K, GR, PD, EX, true); else STEP2(K, GR, PD, EX, false); } while (0)
 #define STEP(PD, EX)                                                              \
     do {                                                                          \
         if (ctx->ks == 3) { if (grad) STEP1(3, true, PD, EX); else STEP1(3, false, PD, EX); }      \
@@ -1245,7 +1248,7 @@ lfrv_status run_fista(lfrv_ctx *ctx, bool last)
 bool sr_batchable(const lfrv_ctx *ctx)
 {
     return ctx->p.mode == LFRV_MODE_COLOR_SR && ctx->ks >= 3 && ctx->ks <= 5 && ctx->p.inner_iterations == 1 &&
-           !sr_wide(ctx->W + ctx->ks - 1, ctx->H + ctx->ks - 1);
+           !sr_wide(ctx);
 }
 
 lfrv_status sr_batch_begin(lfrv_ctx *ctx, int steps, SrBatchItem *it, float *theta_host)

@@ -344,6 +344,8 @@ struct lfrv_ctx {
     hipStream_t side = nullptr;
     hipEvent_t side_fork = nullptr, side_join = nullptr;
     std::string err;
+    // planes of this many bytes and more are addressed row by row by the marching strips (strip_wide; tests lower it)
+    size_t narrow_bytes = (size_t)1 << 31;
 
     // views (contiguous over views)
     float *views = nullptr;    // V*3n

@@ -52,10 +52,24 @@ __device__ __forceinline__ float product(float a, float b)
 }
 
 constexpr int kOutside = (int)0x80000000;
-constexpr size_t kNarrowBytes = (size_t)1 << 31;  // kOutside lies past any buffer up to this size
+constexpr size_t kNarrowBytes = (size_t)1 << 31;  // kOutside lies past any buffer below this size
+constexpr int kStripOverrun = 16;  // a strip names fewer rows than this past its planes (with kOutside)
+
+// Whether the strips need a descriptor per row: where the scalar offset of a
+// row past the last of `planes` planes of h rows of w values would reach
+// `limit` (kNarrowBytes; int arithmetic, and added to kOutside it would wrap).
+constexpr bool strip_wide(int planes, int w, int h, size_t limit)
+{
+    return 4 * (size_t)w * ((size_t)planes * h + kStripOverrun) >= limit;
+}
+static_assert(strip_wide(5, 10361, 10363, kNarrowBytes),
+              "planes that fit one descriptor, the rows past whose end overflow the offset");
+static_assert(!strip_wide(5, 10360, 10363 - kStripOverrun, kNarrowBytes) &&
+                  4ll * (4 * 10360ll * (10363 - kStripOverrun) + 10360ll * 10363) < (1ll << 31),
+              "the largest narrow planes");
 
 // Planes of `w`-wide rows, `stride` values apart.  Narrow: one descriptor for
-// all of them (at most kNarrowBytes), the row and plane in the scalar offset.
+// all of them (unless strip_wide), the row and plane in the scalar offset.
 // WIDE: a descriptor per row.
 template <bool WIDE>
 struct Planes {

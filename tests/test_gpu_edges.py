@@ -2,6 +2,8 @@
 are no multiple of any tile, a single view, tiny images, and a view whose depth
 is invalid everywhere (import.cpp:292-296 sends all its pixels out of the
 target), for both models."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -140,3 +142,49 @@ def test_box_iterations_at_strip_edges(w, h, dsf):
     r = oracle.gibr_pipeline(s["views"], s["depths"], s["P_views"], s["P_target"], dsf, 1 / 255.0, 1.0, 1.0, 0.5, 1e-6, 3000)
     # two solves to a relative residual of 1e-6 of a system whose condition number is below 1e3
     assert rel_err(U, r["U"]) < 1e-3
+
+
+def _address_row_by_row(ctx):
+    """What planes of 2 GiB and more take: a buffer descriptor per row in the marching strips."""
+    f = lfrv.lib().lfrv_test_narrow_bytes
+    f.restype, f.argtypes = None, [ctypes.c_void_p, ctypes.c_size_t]
+    f(ctx._h, 0)
+
+
+@pytest.mark.parametrize("w,h,dsf,inner,beta", [(62, 5, 1, 1, 0.3), (57, 7, 1, 9, 0.0), (29, 7, 2, 1, 0.3), (61, 8, 2, 1, 0.0),
+                                               (31, 3, 2, 0, 0.3), (31, 3, 2, 0, 0.0), (19, 16, 3, 1, 0.3), (40, 9, 3, 4, 0.0),
+                                               (33, 6, 3, 0, 0.3), (14, 5, 4, 1, 0.3), (30, 4, 4, 2, 0.0), (20, 7, 4, 0, 0.3)])
+def test_color_steps_addressed_row_by_row(w, h, dsf, inner, beta):
+    """The forms of the marching step and of the primal-dual passes for planes beyond one descriptor: the same bits."""
+    s = _planes(w, h, dsf, 3, seed=7)
+    print(f"IBR_color row by row {w}x{h} dsf={dsf} inner={inner} beta={beta}", flush=True)
+    out = []
+    for wide in (False, True):
+        with lfrv.Context(pipelines.color_sr_params(s, inner_iterations=inner, dt_beta=beta, gradient_step=1.0)) as ctx:
+            if wide:
+                _address_row_by_row(ctx)
+            pipelines.load_scene(ctx, s)
+            ctx.clear_solution()
+            pipelines.color_sr_setup(ctx)
+            ctx.sr_init_regularizer_weight()
+            ctx.sr_iteration_fista()
+            ctx.sr_iterate(4)
+            out.append([ctx.get_buffer(k) for k in ("U", "UQ", "PX", "PY", "NORM_MASK") + (("G",) if inner != 1 else ())])
+    for a, b in zip(*out):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("w,h,dsf", [(30, 7, 2), (31, 5, 2), (29, 4, 3), (14, 9, 4), (15, 3, 4)])
+def test_box_iterations_addressed_row_by_row(w, h, dsf):
+    """The marching PCG iteration for planes beyond one descriptor: the same bits."""
+    s = _planes(w, h, dsf, 3, 5)
+    print(f"PCG row by row {w}x{h} dsf {dsf}", flush=True)
+    out = []
+    for wide in (False, True):
+        with lfrv.Context(pipelines.gradient_ibr_params(s)) as ctx:
+            if wide:
+                _address_row_by_row(ctx)
+            pipelines.load_scene(ctx, s)
+            st = pipelines.gradient_ibr_solve(ctx, 1e-6, 3000)
+            out.append((ctx.get_solution(), st["iterations"]))
+    assert out[0][1] == out[1][1] and np.array_equal(out[0][0], out[1][0])
