@@ -21,15 +21,19 @@ __global__ void k_hole_list(size_t N, const float *__restrict__ vis, int *__rest
     list[k] = (int)o;
 }
 
-// The diffusion runs up to kHoleSweeps Jacobi sweeps per launch: a block owns a
-// tile of kHoleTile^2 pixels that holds holes, takes it into LDS with a halo as
-// wide as the sweeps, and the halo's validity shrinks by a pixel per sweep.
+// The diffusion runs up to kHoleSweeps Jacobi sweeps per launch: a block takes a
+// tile of kHoleTile^2 pixels that holds holes into LDS with a halo as wide as
+// the sweeps, and the halo's validity shrinks by a pixel per sweep.
 // The stopping rule is still the one after every sweep: a launch leaves the
 // energy of each of its sweeps, the next one evaluates the rule on them, and if
 // it fired before the last of them runs that many sweeps again from the same
 // start.  100 x 75 holes of a 403 x 301 view, 500 sweeps: 0.79 ms; one sweep per
 // launch, 2.05 ms (4.1 us each, the launch of a dependent tiny kernel).
-constexpr int kHoleTile = 16, kHoleSweeps = 8, kHoleRegion = kHoleTile + 2 * kHoleSweeps;
+// Every block adds up the energies of all of them, so there are at most
+// kHoleBlocks, two per CU, which run through the tiles: 1000 tiles of a 700 x
+// 700 view, 500 sweeps: 2.3 ms (1024 blocks 2.8, a block per tile 2.5); 8200
+// tiles of a 1535 x 1531 view: 10.6 ms (11.3 and 29; one sweep per launch 22.5).
+constexpr int kHoleTile = 16, kHoleSweeps = 8, kHoleRegion = kHoleTile + 2 * kHoleSweeps, kHoleBlocks = 512;
 
 // eh[j] holds the energy of sweep j (eh[0] = 0, the energy the first sweep is
 // compared with); *stopped the number of sweeps run once the rule has fired.
@@ -101,7 +105,7 @@ __global__ void __launch_bounds__(512) k_hole_sweeps(int W, int H, int ntx, cons
     __shared__ double es[kHoleSweeps + 1], ws[NT / 64][kHoleSweeps];
     __shared__ int stop;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int n = *hl.count;
+    const int ntiles = *hl.count, n = min(ntiles, (int)gridDim.x);  // n: the blocks with tiles
     if ((int)blockIdx.x >= n) return;
     // (a stop within the launch before is set by this launch, maybe already)
     if (tid == 0) {
@@ -135,61 +139,65 @@ __global__ void __launch_bounds__(512) k_hole_sweeps(int W, int H, int ntx, cons
     const int sweeps = redo ? stop : K;
     if (sweeps == 0) return;
 
-    const int tile = hl.tiles[blockIdx.x], ty = tile / ntx, tx = tile - ty * ntx;
-    const int rx = tx * kHoleTile - kHoleSweeps, ry = ty * kHoleTile - kHoleSweeps;
     const size_t N = (size_t)W * H;
-    bool hole[PT], own[PT];
-#pragma unroll
-    for (int p = 0; p < PT; p++) {
-        const int i = tid + p * NT, lx = i % R, ly = i / R, x = rx + lx, y = ry + ly;
-        const bool in = x >= 0 && x < W && y >= 0 && y < H;
-        const size_t o = in ? (size_t)y * W + x : 0;
-        hole[p] = in && vis[o] == 0.0f;
-        own[p] = hole[p] && lx >= kHoleSweeps && lx < R - kHoleSweeps && ly >= kHoleSweeps && ly < R - kHoleSweeps;
-        // (the region's rim keeps its values: it has no neighbours beyond)
-        hole[p] = hole[p] && lx > 0 && lx < R - 1 && ly > 0 && ly < R - 1;
-#pragma unroll
-        for (int c = 0; c < 3; c++) us[0][c][i] = us[1][c][i] = in ? src[c * N + o] : 0.0f;
-    }
-    __syncthreads();
     double e[kHoleSweeps];
 #pragma unroll
-    for (int s = 0; s < kHoleSweeps; s++) {
-        e[s] = 0.0;
-        if (s >= sweeps) continue;
+    for (int s = 0; s < kHoleSweeps; s++) e[s] = 0.0;
+    for (int k = blockIdx.x; k < ntiles; k += n) {
+        const int tile = hl.tiles[k], ty = tile / ntx, tx = tile - ty * ntx;
+        const int rx = tx * kHoleTile - kHoleSweeps, ry = ty * kHoleTile - kHoleSweeps;
+        bool hole[PT], own[PT];
 #pragma unroll
         for (int p = 0; p < PT; p++) {
-            if (!hole[p]) continue;
-            const int i = tid + p * NT, x = rx + i % R, y = ry + i / R;
+            const int i = tid + p * NT, lx = i % R, ly = i / R, x = rx + lx, y = ry + ly;
+            const bool in = x >= 0 && x < W && y >= 0 && y < H;
+            const size_t o = in ? (size_t)y * W + x : 0;
+            hole[p] = in && vis[o] == 0.0f;
+            own[p] = hole[p] && lx >= kHoleSweeps && lx < R - kHoleSweeps && ly >= kHoleSweeps && ly < R - kHoleSweeps;
+            // (the region's rim keeps its values: it has no neighbours beyond)
+            hole[p] = hole[p] && lx > 0 && lx < R - 1 && ly > 0 && ly < R - 1;
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const float *u = us[s & 1][c];
-                float mean;
-                if (x > 0 && y > 0 && x < W - 1 && y < H - 1) {  // (a quarter: exact, and no division)
-                    mean = 0.25f * (((u[i - 1] + u[i - R]) + u[i + 1]) + u[i + R]);
-                } else {
-                    float sm = 0.0f, wsum = 0.0f;
-                    if (x > 0) { sm += u[i - 1]; wsum += 1.0f; }
-                    if (y > 0) { sm += u[i - R]; wsum += 1.0f; }
-                    if (x < W - 1) { sm += u[i + 1]; wsum += 1.0f; }
-                    if (y < H - 1) { sm += u[i + R]; wsum += 1.0f; }
-                    mean = sm / wsum;
-                }
-                const float lap = mean - u[i];
-                const float un = u[i] + lap;
-                us[(s & 1) ^ 1][c][i] = un;
-                if (c == 2 && own[p]) e[s] += (double)lap * (double)un;
-            }
+            for (int c = 0; c < 3; c++) us[0][c][i] = us[1][c][i] = in ? src[c * N + o] : 0.0f;
         }
         __syncthreads();
-    }
 #pragma unroll
-    for (int p = 0; p < PT; p++) {
-        if (!own[p]) continue;
-        const int i = tid + p * NT;
-        const size_t o = (size_t)(ry + i / R) * W + rx + i % R;
+        for (int s = 0; s < kHoleSweeps; s++) {
+            if (s >= sweeps) continue;
 #pragma unroll
-        for (int c = 0; c < 3; c++) dst[c * N + o] = us[sweeps & 1][c][i];
+            for (int p = 0; p < PT; p++) {
+                if (!hole[p]) continue;
+                const int i = tid + p * NT, x = rx + i % R, y = ry + i / R;
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const float *u = us[s & 1][c];
+                    float mean;
+                    if (x > 0 && y > 0 && x < W - 1 && y < H - 1) {  // (a quarter: exact, and no division)
+                        mean = 0.25f * (((u[i - 1] + u[i - R]) + u[i + 1]) + u[i + R]);
+                    } else {
+                        float sm = 0.0f, wsum = 0.0f;
+                        if (x > 0) { sm += u[i - 1]; wsum += 1.0f; }
+                        if (y > 0) { sm += u[i - R]; wsum += 1.0f; }
+                        if (x < W - 1) { sm += u[i + 1]; wsum += 1.0f; }
+                        if (y < H - 1) { sm += u[i + R]; wsum += 1.0f; }
+                        mean = sm / wsum;
+                    }
+                    const float lap = mean - u[i];
+                    const float un = u[i] + lap;
+                    us[(s & 1) ^ 1][c][i] = un;
+                    if (c == 2 && own[p]) e[s] += (double)lap * (double)un;
+                }
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int p = 0; p < PT; p++) {
+            if (!own[p]) continue;
+            const int i = tid + p * NT;
+            const size_t o = (size_t)(ry + i / R) * W + rx + i % R;
+#pragma unroll
+            for (int c = 0; c < 3; c++) dst[c * N + o] = us[sweeps & 1][c][i];
+        }
+        // (a pixel of us[] that a thread still reads here is its own: it may take the next tile's at once)
     }
     if (redo) return;
 #pragma unroll
@@ -420,7 +428,8 @@ lfrv_status run_hole_filling(lfrv_ctx *ctx, int iters, double eps, int *ran)
     k_hole_init<<<blocks_for(ntiles), kBlock, 0, ctx->stream>>>(hl, ntiles, flags);
     k_hole_flag<<<blocks_for(nh), kBlock, 0, ctx->stream>>>(ctx->W, ntx, (int)nh, ctx->hole_list, flags);
     k_hole_tiles<<<1, 1024, 0, ctx->stream>>>(ntiles, flags, tiles, count);
-    const unsigned int nb = std::min((unsigned int)ntiles, nh);  // at least as many as have holes
+    // (up to the bound at least as many as there are tiles with holes)
+    const unsigned int nb = std::min({(unsigned int)ntiles, nh, (unsigned int)kHoleBlocks});
     int launched = 0, chunks = 0, prev = 0, host = 0;
     // the rule is read back after 2 launches, then after every 8 (those enqueued behind a stop return at once)
     while (launched < iters && !host) {

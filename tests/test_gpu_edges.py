@@ -112,7 +112,7 @@ def test_color_sr_ragged_inputs(w, h, dsf, inner):
                                       (48, 40, (8, 40, 8, 24)),    # whole tiles of holes
                                       (65, 20, (60, 65, 3, 20))])  # one column in the last tile
 def test_hole_sweeps_at_tile_edges(w, h, dead):
-    """The Poisson diffusion in tiles of 16 x 16 and eight sweeps per launch, against sweep after sweep in FP64."""
+    """A solve from an image whose holes end at the edges of tiles (the diffusion itself: the next test)."""
     print(f"hole filling {w}x{h} holes {dead}", flush=True)
     d = lfrv.synth_desc(2, 11)
     d.grid, d.w, d.h, d.focal = 2, w, h, 1000.0 * w / 1024.0
@@ -126,6 +126,41 @@ def test_hole_sweeps_at_tile_edges(w, h, dead):
     r = oracle.gibr_pipeline(s["views"], s["depths"], s["P_views"], s["P_target"], 1, 1 / 255.0, 1.0, 1.0, 0.5, 1e-5, 3000)
     # two solves to a relative residual of 1e-5
     assert rel_err(U, r["U"]) < 1e-3
+
+
+# (holes to three image edges, one tile past the second; whole tiles of holes; one column in the last tile; a hole
+# across all inner tiles; a tile's middle row; more tiles than blocks).  The scale of the views sets when the rule
+# fires: at sweeps that end a launch of eight, within one, at the first, and at the 500 of the cap, of which the last
+# launch has four.
+@pytest.mark.parametrize("w,h,holes,scale,sweeps", [
+    (17, 33, (0, 17, 0, 16), 0.4, 5), (17, 33, (0, 17, 0, 16), 1.0, 7), (17, 33, (0, 17, 0, 16), 6.0, 56),
+    (48, 40, (8, 40, 8, 24), 0.7, 14), (65, 20, (60, 65, 3, 20), 0.3, 1), (65, 20, (60, 65, 3, 20), 6.0, 11),
+    (64, 48, (3, 60, 2, 47), 6.0, 500), (40, 41, (8, 24, 17, 33), 1.0, 16), (40, 41, (8, 24, 17, 33), 2.0, 26),
+    (560, 530, (0, 560, 3, 530), 0.1, 60), (560, 530, (0, 560, 3, 530), 1.0, 500)])
+def test_hole_sweeps_match_the_oracle(w, h, holes, scale, sweeps):
+    """The Poisson diffusion in tiles of 16 x 16 and eight sweeps per launch: the filled image and the sweep at which
+    the rule fires, against sweep after sweep in FP64."""
+    print(f"hole filling {w}x{h} holes {holes} scale {scale}", flush=True)
+    s = _planes(w, h, 1, 2, seed=11)
+    s["views"] = (np.float32(scale) * s["views"]).astype(np.float32)
+    vis = np.ones((h, w), np.uint8)
+    vis[holes[2]:holes[3], holes[0]:holes[1]] = 0
+    with lfrv.Context(pipelines.gradient_ibr_params(s)) as ctx:
+        pipelines.load_scene(ctx, s)
+        ctx.warps_from_depth()
+        ctx.prepare()
+        ctx.setup_visibility()
+        ctx.compute_weights()
+        ctx.set_buffer("VISIBILITY", vis.astype(np.float32))
+        ctx.compute_initial_image()
+        U, stats = ctx.get_solution(), ctx.hole_stats()
+        tx, ty, om = [ctx.get_buffer(k).reshape(s["V"], h, w) for k in ("TAU_X", "TAU_Y", "OMEGA")]
+    want, _ = oracle.initial_image(w, h, 1, tx, ty, s["views"], om)
+    want, k = oracle.hole_filling(want, vis)
+    # (the energies of FP32 images: their rounding is a percent at most of how far the rule was from firing)
+    assert k == sweeps and stats == (int((vis == 0).sum()), sweeps)
+    # a sweep rounds a mean and a sum of values of the image's scale: half an ulp each, averaged over the sweeps
+    assert np.max(np.abs(U - want)) < scale * 6e-8 * (4 + sweeps)
 
 
 @pytest.mark.parametrize("w,h,dsf", [(30, 7, 2), (31, 5, 2),    # one strip of 60 columns exactly, and two columns more
