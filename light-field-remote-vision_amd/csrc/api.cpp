@@ -228,7 +228,7 @@ extern "C" lfrv_status lfrv_create(const lfrv_params *p, lfrv_ctx **out)
         A(&ctx->box_ops, 5 * (size_t)(ctx->W + ctx->ks - 1) * (ctx->H + ctx->ks - 1));
         A(&ctx->cg_extra, 12 * N);
     }
-    ctx->pp_cap = 3 * (N + N / 2) + 3 * N + N / 4 + 64;
+    ctx->pp_cap = N + N / 8 + 64;  // the levels below the target's: N / 3 pixels of three floats and a byte
     A(&ctx->pp_scratch, ctx->pp_cap);
     A(&ctx->cg_state, 1);
     A(&ctx->sr_loop, 1);

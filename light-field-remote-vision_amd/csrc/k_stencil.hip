@@ -424,7 +424,7 @@ lfrv_status run_hole_filling(lfrv_ctx *ctx, int iters, double eps, int *ran)
     int *flags = reinterpret_cast<int *>(ctx->cg_d), *tiles = flags + ntiles;
     int *stopped = reinterpret_cast<int *>(ctx->counters + 12), *count = reinterpret_cast<int *>(ctx->counters + 13);
     const HoleLoop hl{iters, eps, ctx->partials, stopped, tiles, count};
-    if ((size_t)iters + 1 > ctx->partials_cap - 2048) return fail(ctx, LFRV_E_ARG, "hole filling: too many sweeps");
+    if ((size_t)iters + 1 > ctx->partials_cap) return fail(ctx, LFRV_E_ARG, "hole filling: too many sweeps");
     k_hole_init<<<blocks_for(ntiles), kBlock, 0, ctx->stream>>>(hl, ntiles, flags);
     k_hole_flag<<<blocks_for(nh), kBlock, 0, ctx->stream>>>(ctx->W, ntx, (int)nh, ctx->hole_list, flags);
     k_hole_tiles<<<1, 1024, 0, ctx->stream>>>(ntiles, flags, tiles, count);
@@ -480,15 +480,13 @@ lfrv_status run_push_pull(lfrv_ctx *ctx, int levels)
 {
     const int W = ctx->W, H = ctx->H;
     const size_t N = ctx->N;
-    // level offsets inside the pyramid scratch: level 0 is a copy of U
+    // level offsets inside the pyramid scratch, from level 1 on: level 0 is U itself and the target's map
     std::vector<size_t> off(levels + 1, 0);
     std::vector<int> ws(levels + 1, 0), hs(levels + 1, 0);
     size_t tot = 0;
     int top = 0;
     ws[0] = W;
     hs[0] = H;
-    off[0] = 0;
-    tot = N;
     for (int s = 1; s <= levels; s++) {
         const int wsn = W >> s, hsn = H >> s;
         if (wsn <= 0 || hsn <= 0) break;
@@ -498,7 +496,7 @@ lfrv_status run_push_pull(lfrv_ctx *ctx, int levels)
         tot += (size_t)wsn * hsn;
         top = s;
     }
-    // scratch: pyramid images (3 * tot floats) + vis pyramid (tot bytes); level 0 stays in U and the target's map
+    // scratch: pyramid images (3 * tot floats) + vis pyramid (tot bytes)
     const size_t need = 3 * tot + (tot + 3) / 4 + 1;
     if (need > ctx->pp_cap) return fail(ctx, LFRV_E_ARG, "push-pull scratch too small");
     float *img = ctx->pp_scratch;
