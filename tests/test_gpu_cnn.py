@@ -365,3 +365,36 @@ def test_conv3x3_sums_in_a_fixed_order(Cin, Cout):
     lfrv.device_sync()
     inner = dY.get(np.float32, (B, H, W, Cout))[:, 1:-1, 1:-1]  # (where every term lies in the image)
     assert np.array_equal(inner, np.broadcast_to(want, inner.shape))
+
+
+def test_gradient_at_the_training_size():
+    """8 scenes of 256 x 256: along each layer's gradient the loss changes by the gradient's square, to the rounding
+    of the stepped weights to bf16."""
+    rng, B, H, W, C = np.random.default_rng(1), 8, 256, 256, 100
+    net = Cnn(C, levels=4, base=32, max_batch=B, max_h=H, max_w=W, seed=3)
+    w = _random_params(4, 32, net.cpad, C).astype(np.float64)
+    net.set_params(w)
+    start = rng.uniform(0, 1, (B, 3, H, W)).astype(np.float32)
+    target = (start + 0.1 * rng.standard_normal(start.shape)).astype(np.float32)
+    net.set_batch_host(rng.random((B, H, W, C), dtype=np.float32), start, target)
+    loss = net.loss_grad()
+    g = net.get_grads().astype(np.float64)
+    # the biases stay in FP32; a weight stepped by less than its bf16 spacing moves by all of it, or not at all, with
+    # the probability that gives the step on average
+    spacing = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(w), 1e-30))) - 7)
+
+    def at(step):
+        net.set_params(w + step)
+        return net.loss_grad()
+
+    for name, ws, bs, ci, co in layer_slices(4, 32, net.cpad):
+        d = np.zeros_like(g)
+        d[ws], d[bs] = g[ws], g[bs]
+        square = d @ d
+        h = 0.1 * loss / square / 2  # a tenth of the loss between the two ends
+        ratio = (at(h * d) - at(-h * d)) / (2 * h * square)
+        noise = np.sqrt(2 * h * np.sum(np.abs(d[ws]) ** 3 * spacing[ws])) / (2 * h * square)
+        print(f"{name}: {ratio:.3f}, rounding {noise:.3f}", flush=True)
+        assert abs(ratio - 1) < 5 * noise + 0.05, name
+        assert noise < 0.15, name
+    net.close()
