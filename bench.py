@@ -956,10 +956,12 @@ def main():
         op_kernel = "k_cgcg_st2 (fused single-reduction PCG iteration, assembled 9-point stencil)"
         op_bytes = 144 * N
     else:
-        # entry-walk operator: r, Minv, d_prev, d, q planes (52 B per target pixel)
-        # + tau_x, tau_y, omega of every splatted source pixel (12 B)
-        op_kernel = "k_cg_op (fused PCG operator, entry walk)"
-        op_bytes = 52 * N + 12 * e_unique
+        # one PCG iteration on the box operator, per target pixel: r, w, s, p, x
+        # (60 B) and Minv (4 B) read, r, w, s, p, x (60 B) written; the 5 coupling
+        # planes of the anchor grid (20 B per anchor)
+        D = scene["dsf"]
+        op_kernel = f"k_box_iter<{D}> (fused single-reduction PCG iteration, box operator)"
+        op_bytes = 124 * N + 20 * (scene["W"] + D) * (scene["H"] + D)
     op_avg_s = op_ms / max(op_n, 1) / 1e3
     traffic = measured_traffic() if (scene["dsf"] == 1 and scene["V"] == 9 and N == 1024 * 1024) else None
     achieved = op_bytes / op_avg_s / 1e9

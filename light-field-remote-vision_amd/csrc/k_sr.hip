@@ -251,11 +251,15 @@ __global__ void __launch_bounds__(kPullMaxThreads) k_sr_assemble(TileGeom g, Til
 // Laplacian), and LAG columns at each end of the wave are halo: 54 - 60 of the
 // 64 lanes have an output.
 // Bounds: at large targets the bytes of the step (25 views, 2048^2, dsf 4: 555
-// MB in 141 us, 3.9 TB/s; 188 us before), at small ones the latency of the rows
-// of one wave (256^2, dsf 2: 6.6 us per step; 7.1 before).  The tile form this
-// replaced (32 x 16 pixels, nine LDS phases, 2.1 x halo loads) was bound by its
-// LDS and address instructions.  Results are its own bit for bit: sums in its
-// order, the contractions written out.
+// MB in 140 us, 4.0 TB/s; 188 us before), at small ones the latency of the rows
+// of one wave (256^2, dsf 2: 6.4 us per step; 7.1 before), in a batch at dsf 2
+// with the gradient term the instructions.  The tile form this replaced (32 x
+// 16 pixels, nine LDS phases, 2.1 x halo loads) was bound by its LDS and address
+// instructions.  Sums run in its order, contractions are written out and the
+// projected duals are rounded before they are summed (product), so that the
+// results are its own bit for bit: compared at dsf 1 to 4 over 50 to 500 steps of
+// four scenes each, where the steps with the gradient term would show a single
+// rounding.
 // Loads and stores go through buffer descriptors, and a lane or row outside
 // its plane takes the offset kOutside, past every buffer: it reads 0 and writes
 // nothing, without a compare per value.  Every row issues the same loads and
@@ -277,7 +281,7 @@ struct StepBufs {
 };
 
 // Rows y0 .. y1 - 1 of the strip whose first output column is x0.  With PD the
-// data term and the first primal-dual iteration (k_pd_step's update, with
+// data term and the first primal-dual iteration (k_pd_steps' update, with
 // Uq = U as the step sets it, optimization.cu:1765-1767): the new primal goes
 // to unew, with uq_relax the over-relaxed one (vtv_rof.cu:28-45) there, with
 // gout F.  Without PD F goes to gout and U to uq_relax.  EXTRA: one of
@@ -1044,7 +1048,10 @@ int sr_lag(int ks, bool grad) { return ks - 1 + (grad ? 1 : 0); }
 // the 2 LAG before the first output, and 2 waves per SIMD, 2048 in all, run at
 // once: the height (whole groups of rows) with the least rows per slot.  2048^2,
 // dsf 4 (38 strips across): 42 rows, 1862 waves, 141 us per step; 36 rows, 2166
-// waves, 173 us; 256^2, dsf 2: 3 rows 6.6 us, 12 rows 12.6 us.
+// waves, 173 us; 256^2, dsf 2: 3 rows 6.6 us, 12 rows 12.6 us.  Two waves are
+// what the steps with the gradient term and the PCG iteration have registers
+// for; the steps without it and the primal-dual passes would fit three to seven,
+// and take the same rule without a measurement of theirs at other heights.
 int strip_rows(int lag, const StripSize *sizes, int n)
 {
     int best = kStripGroup;
