@@ -257,9 +257,8 @@ __global__ void __launch_bounds__(kPullMaxThreads) k_sr_assemble(TileGeom g, Til
 // 16 pixels, nine LDS phases, 2.1 x halo loads) was bound by its LDS and address
 // instructions.  Sums run in its order, contractions are written out and the
 // projected duals are rounded before they are summed (product), so that the
-// results are its own bit for bit: compared at dsf 1 to 4 over 50 to 500 steps of
-// four scenes each, where the steps with the gradient term would show a single
-// rounding.
+// results are its own bit for bit: compared at dsf 1 to 4, with and without the
+// gradient term, over 50 to 500 steps of several scenes.
 // Loads and stores go through buffer descriptors, and a lane or row outside
 // its plane takes the offset kOutside, past every buffer: it reads 0 and writes
 // nothing, without a compare per value.  Every row issues the same loads and

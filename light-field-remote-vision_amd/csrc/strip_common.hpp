@@ -103,7 +103,7 @@ struct Planes {
 // the smallest normal number (an ulp there): a Newton step for the reciprocal,
 // which several quotients of one divisor share, then two for the quotient.
 // Divisors away from 1 are brought there by a power of two, and the fix-up
-// gives what division gives for zeros, infinities and NaN.
+// gives what division gives for zeros, infinities and NaN, and where it overflows.
 struct Divisor {
     float d, r, scale;
     __device__ __forceinline__ explicit Divisor(float div)

@@ -351,3 +351,25 @@ def test_step_with_coverages_that_need_a_division(dsf, beta):
         else:
             assert np.all(np.sign(F[1][:, y, x] - U0[:, y, x]) == -np.sign(step))
     assert np.array_equal(F[0][:, rest], F[1][:, rest])
+
+
+@pytest.mark.parametrize("dsf,beta", [(2, 0.0), (4, 0.3)])
+def test_step_whose_quotients_overflow(dsf, beta):
+    """Views of 1e33: over a coverage of 1e-3 the gradient overflows to an infinity, which the clamp takes to the same
+    +-1 as the finite one over 1, not to NaN."""
+    s = _scene(dsf=dsf)
+    H, W = s["H"], s["W"]
+    s["views"] = ((s["views"] - 0.5) * np.float32(1e33)).astype(np.float32)
+    print(f"overflowing quotients dsf={dsf} beta={beta}", flush=True)
+    U0 = np.random.default_rng(dsf).uniform(0.2, 0.8, (3, H, W)).astype(np.float32)
+    F = []
+    for cov in (1.0, 1e-3):
+        with lfrv.Context(pipelines.color_sr_params(s, inner_iterations=0, dt_beta=beta, gradient_step=1.0)) as ctx:
+            pipelines.load_scene(ctx, s)
+            pipelines.color_sr_setup(ctx)
+            ctx.set_buffer("COVERAGE", np.full((H, W), cov, np.float32))
+            ctx.set_solution(U0)
+            ctx.sr_iteration_fista()
+            F.append(ctx.get_buffer("G").reshape(3, H, W))
+    assert np.isin(F[0], (0, 1)).mean() > 0.9 and 0.2 < (F[0] == 1).mean() < 0.8
+    assert np.array_equal(F[0][np.isin(F[0], (0, 1))], F[1][np.isin(F[0], (0, 1))])
